@@ -37,7 +37,7 @@ DEVICE_FLAGS = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",
           f"-I{os.path.join(ROOT, 'include')}"]
 
-LIB_SOURCES = ["knn_kernels.hip", "xtc_kernels.hip", "api.cpp", "serve.cpp", "xtc.cpp",
+LIB_SOURCES = ["knn_kernels.hip", "filter_kernels.hip", "xtc_kernels.hip", "api.cpp", "serve.cpp", "xtc.cpp",
                "xtc_device.cpp", "topology.cpp", "spectral.cpp"]
 # executables: (name, main source)
 TOOLS = [("knn_rms", "knn_rms_main.cpp"), ("make_sysparse", "make_sysparse_main.cpp"),

@@ -740,7 +740,22 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
                   Carve::round((size_t)n * sizeof(unsigned)) + 512
             : 0;
   const size_t mir_bytes = (size_t)n * c->mirror_cap * sizeof(uint2);
-  const size_t sym_bytes = Carve::round(mir_bytes) + perm_bytes;
+  // The tile filter (filter_kernels.hip) over the canonical copy's order.
+  const FilterShape fsh = filter_shape(c->ref.natoms);
+  const int fit_blocks = c->ref.n_tiles / kFilterFitTiles;
+  const size_t tiles_n = (size_t)fit_blocks * ref_pairs;
+  const size_t sort_temp = sort_order_scratch(n);
+  const size_t filter_bytes =
+      Carve::round(filter_operand_bytes(fsh, c->ref.n_tiles)) + 2 * Carve::round(rows * sizeof(float4)) +
+      Carve::round(rows * 12 * sizeof(double)) + Carve::round(rows * 36 * sizeof(ushort)) +
+      Carve::round(fsh.natoms * 3 * sizeof(double)) + Carve::round(fsh.slots() * sizeof(int)) +
+      Carve::round(12 * kFilterSamples * sizeof(double)) + Carve::round(sizeof(FilterMean)) +
+      Carve::round(tiles_n) + Carve::round(tiles_n * sizeof(int)) +
+      Carve::round(fit_blocks * sizeof(int)) + Carve::round(2 * sizeof(int)) +
+      3 * Carve::round((size_t)n * sizeof(int)) + Carve::round(sort_temp) +
+      2 * Carve::round((size_t)nlab * sizeof(int));
+  bool filter = canon && n >= kFilterMinFrames;
+  size_t sym_bytes = Carve::round(mir_bytes) + perm_bytes + (filter ? filter_bytes : 0);
   const size_t small = (size_t)n * nl * (sizeof(int) + sizeof(float)) +
                        (size_t)n * 7 * sizeof(int) + (size_t)nlab * sizeof(int) + 1024;
   // Room: the free device memory plus what the buffers already hold, less a
@@ -748,13 +763,18 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   size_t free_b = 0, total_b = 0;
   HIP_TRY(c, hipMemGetInfo(&free_b, &total_b));
   const size_t have = s.ws_sym_bytes + s.ws_lists_bytes + s.ws_small_bytes;
-  const size_t need = ent_bytes + sym_bytes + small;
   const size_t reserve = size_t(2) << 30;
-  if (need + reserve > free_b + have) return 1;
-  {
+  auto fits = [&]() {
+    const size_t need = ent_bytes + sym_bytes + small;
+    if (need + reserve > free_b + have) return false;
     std::lock_guard<std::mutex> g(c->mem_mu);
-    if (c->budget && c->held - std::min(c->held, have) + need > c->budget) return 1;
+    return !(c->budget && c->held - std::min(c->held, have) + need > c->budget);
+  };
+  if (filter && !fits()) {  // every tile is contracted instead
+    filter = false;
+    sym_bytes = Carve::round(mir_bytes) + perm_bytes;
   }
+  if (!fits()) return 1;
   int rc = ensure(c, &s.ws_sym, &s.ws_sym_bytes, sym_bytes, "mirrored lists");
   if (!rc) rc = ensure(c, &s.ws_lists, &s.ws_lists_bytes, ent_bytes, "candidate lists");
   if (!rc) rc = ensure(c, &s.ws_small, &s.ws_small_bytes, small, "list headers");
@@ -797,12 +817,35 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   HIP_TRY(c, launch_init_lists(LL, n, s.st));
   HIP_TRY(c, launch_contract(R, fit, LL, eps2, q.k1, lstride, q.nofit, nullptr, grid, s.st,
                              nullptr, 1));
-  HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, eps2, lstride, L.thr, label, s.st));
+  Carve fc;
+  fc.base = (char*)s.ws_sym + Carve::round(mir_bytes) + perm_bytes;
+  fc.size = filter ? filter_bytes : 0;
+  if (filter) {
+    // rows in cells of about 6 (k+1) frames around every cell-th landmark,
+    // by distance within a cell
+    unsigned* keys = (unsigned*)fc.take((size_t)n * sizeof(int));
+    unsigned* keys_out = (unsigned*)fc.take((size_t)n * sizeof(int));
+    int* row_ids = (int*)fc.take((size_t)n * sizeof(int));
+    void* temp = fc.take(sort_temp);
+    int* leaders = (int*)fc.take((size_t)nlab * sizeof(int));
+    int* rank = (int*)fc.take((size_t)nlab * sizeof(int));
+    if (!keys || !keys_out || !row_ids || !temp || !leaders || !rank)
+      return fail(c, MDSCTK_ERR_ARG, "symmetric self query: sort workspace carve");
+    const int cell = (int)std::max<int64_t>(
+        1, std::max<int64_t>((int64_t)nlab * 6 * q.k1 / n, nlab / kFilterMaxCells + 1));
+    const int ncells = (nlab + cell - 1) / cell;
+    HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, eps2, lstride, L.thr, label, s.st, cell, keys,
+                                   row_ids, leaders, 1 + std::min(q.k1 / 2, nlab / 256)));
+    HIP_TRY(c, launch_sort_order(leaders, rank, ncells, keys, keys_out, row_ids, order, n, temp,
+                                 sort_temp, s.st));
+  } else {
+    HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, eps2, lstride, L.thr, label, s.st));
+  }
   // rows grouped by nearest landmark: the merge takes them in this order (it
   // pays where candidate frames no longer fit the caches), and the canonical
   // form contracts the frames in it
   const bool ordered = n >= 512;
-  if (ordered) HIP_TRY(c, launch_row_order(label, n, nlab, counts, order, s.st));
+  if (ordered && !filter) HIP_TRY(c, launch_row_order(label, n, nlab, counts, order, s.st));
   // the main pass's frames, windows and thresholds
   DevFrames mref = R, mfit = fit;
   Lists LM = L;
@@ -838,11 +881,49 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     // from the rotated one: both within their windows of the exact scores)
     HIP_TRY(c, launch_permute_thresholds(L.thr, order, meps2, n, LM.thr, s.st));
   }
+  TileList tiles;
+  FilterSet fset;
+  FilterMean* fmean = nullptr;
+  if (filter) {
+    fset.op = (uint4*)fc.take(filter_operand_bytes(fsh, c->ref.n_tiles));
+    fset.full = (float4*)fc.take(rows * sizeof(float4));
+    fset.pre = (float4*)fc.take(rows * sizeof(float4));
+    fset.place = (double*)fc.take(rows * 12 * sizeof(double));
+    fset.extra = (ushort*)fc.take(rows * 36 * sizeof(ushort));
+    double* mean = (double*)fc.take(fsh.natoms * 3 * sizeof(double));
+    int* slots = (int*)fc.take(fsh.slots() * sizeof(int));
+    double* align = (double*)fc.take(12 * kFilterSamples * sizeof(double));
+    fmean = (FilterMean*)fc.take(sizeof(FilterMean));
+    tiles.flags = (unsigned char*)fc.take(tiles_n);
+    tiles.list = (int*)fc.take(tiles_n * sizeof(int));
+    tiles.count = (int*)fc.take(fit_blocks * sizeof(int));
+    tiles.ctrl = (int*)fc.take(2 * sizeof(int));
+    if (!fset.op || !fset.full || !fset.pre || !fset.place || !fset.extra || !mean || !slots ||
+        !align || !fmean || !tiles.flags || !tiles.list || !tiles.count || !tiles.ctrl)
+      return fail(c, MDSCTK_ERR_ARG, "symmetric self query: filter workspace carve");
+    DevFrames src = c->ref;
+    HIP_TRY(c, launch_filter_mean(src, c->w, fsh, align, mean, fmean, slots, s.st));
+    HIP_TRY(c, launch_filter_prep(src, c->w, fsh, mean, fmean, slots, order, fset, s.st));
+    // A band pass over the neighbours in that order tightens the thresholds
+    // that the filter tests against: each block against the reference pairs
+    // around it, into the first 4 lists.
+    Lists LB = LM;
+    LB.nl = 4;
+    HIP_TRY(c, launch_init_lists(LB, n, s.st, false));
+    HIP_TRY(c, launch_band_list(c->ref.n_tiles, c->ref.n_tiles, kFilterFitTiles,
+                                std::min(ref_pairs, std::max(4, q.k1 / 8 + 2)), tiles, s.st));
+    HIP_TRY(c, launch_contract(mref, mfit, LB, meps2, q.k1, 1, q.nofit, nullptr, grid, s.st,
+                               nullptr, 0, &tiles));
+    HIP_TRY(c, launch_landmark_cap(LB, n, q.k1, meps2, 1, LM.thr, nullptr, s.st));
+  }
   HIP_TRY(c, launch_init_lists(LM, n, s.st, false));
   HIP_TRY(c, launch_mirror_init(M, n, s.st));
   HIP_TRY(c, hipEventRecord(s.ev[6], s.st));
+  if (filter)
+    HIP_TRY(c, launch_filter(fset, fset, n, n, c->ref.n_tiles, c->ref.n_tiles, fsh, fmean, LM.thr,
+                             meps2, true, phases, std::max(8, c->n_cu & ~7), tiles, s.st));
   HIP_TRY(c, launch_contract(mref, mfit, LM, meps2, q.k1, phases, q.nofit, nullptr, grid, s.st,
-                             &M));
+                             &M, 0, filter ? &tiles : nullptr));
   HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
   HIP_TRY(c, launch_mirror_sum(M, n, msum, s.st));
   HIP_TRY(c, launch_merge(c->ref, fit, c->w, LM, meps2, q.k1, q.k_out, q.rank_off, q.nofit, d_dist,

@@ -128,7 +128,88 @@ struct Mirror {
   int cap = 0;
 };
 
+// ---- the tile filter (filter_kernels.hip): a proven test of which (fit
+// block, reference pair) tiles of a fitted query can hold a pair below the
+// thresholds, from one BF16 product of the frames' deviations from a mean
+// structure.
+
+// Extra operand slots at the end of each segment (the rank-one terms), and
+// frames averaged into the mean structure.
+constexpr int kFilterExtra = 12;
+constexpr int kFilterSamples = 64;
+// Fit tiles per filter block, and the smallest self query that takes it.
+constexpr int kFilterFitTiles = 4;
+constexpr int64_t kFilterMinFrames = 4096;
+// Cells the rows are sorted into (13 bits of the sort key, above 19 bits of
+// the distance).
+constexpr int kFilterMaxCells = 8000;
+constexpr int kFilterDistBits = 19;
+
+// How a frame's atoms are laid out: one or two segments, each a whole number
+// of units of four stages of gps K-groups (16 slots each).
+struct FilterShape {
+  int natoms = 0;
+  int gps = 1;
+  int u0 = 0, u1 = 0;  // units of the first and second segment (u1 0: one segment)
+  int n0 = 0;          // atoms of the first
+  __host__ __device__ int groups0() const { return 4 * gps * u0; }
+  __host__ __device__ int groups() const { return 4 * gps * (u0 + u1); }
+  __host__ __device__ int slots() const { return 16 * groups(); }
+  __host__ __device__ int segment_slots(int s) const { return 64 * gps * (s ? u1 : u0); }
+};
+FilterShape filter_shape(int natoms);
+size_t filter_operand_bytes(const FilterShape& s, int n_tiles);
+
+// C = sum m m^T of each segment (row-major), the norm of the mean structure
+// over the first segment and over both.
+struct FilterMean {
+  float C[2][9];
+  double norm0, norm;
+};
+
+// A frame set's filter operand and its rows' terms of the bound.
+struct FilterSet {
+  uint4* op = nullptr;
+  float4* full = nullptr;   // [n_tiles * 32]
+  float4* pre = nullptr;    // [n_tiles * 32]
+  double* place = nullptr;  // [n_tiles * 32][12] rotation onto the mean, centroid
+  ushort* extra = nullptr;  // [n_tiles * 32][segments][18]
+};
+
+// Reference pairs per fit block: flags [fit blocks][pairs], the flagged ones
+// in ascending order (same shape) and their count; ctrl: two counters.
+struct TileList {
+  unsigned char* flags = nullptr;
+  int* list = nullptr;
+  int* count = nullptr;
+  int* ctrl = nullptr;
+};
+
 // Launchers (all asynchronous on `st`).
+// The mean structure of the set (sqrt(w) scaled, [natoms][3]), its FilterMean
+// and the slot map (shape.slots() ints); scratch: 12 kFilterSamples doubles.
+hipError_t launch_filter_mean(const DevFrames& f, const DevWeights& w, const FilterShape& sh,
+                              double* scratch, double* mean, FilterMean* mc, int* slots,
+                              hipStream_t st);
+// The set's filter operand and terms, row r from frame perm[r] (or r).
+hipError_t launch_filter_prep(const DevFrames& f, const DevWeights& w, const FilterShape& sh,
+                              const double* mean, const FilterMean* mc, const int* slots,
+                              const int* perm, const FilterSet& out, hipStream_t st);
+// The tiles with a pair that may lie within thr[fit] + eps2[fit] / 2 (sym: or
+// the reference frame's), into tl.
+hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_ref, int64_t n_fit,
+                         int ref_tiles, int fit_tiles, const FilterShape& sh, const FilterMean* mc,
+                         const unsigned* thr, const float* eps2, bool sym, int phases, int grid,
+                         const TileList& tl, hipStream_t st);
+// Each fit block of ft tiles against the `width` reference pairs around it.
+hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, const TileList& tl,
+                            hipStream_t st);
+// order = rows sorted by key (stable), the cells of the keys first put in the
+// order of their leaders (rank: ncells ints of scratch).
+size_t sort_order_scratch(int64_t n);
+hipError_t launch_sort_order(const int* leaders, int* rank, int ncells, unsigned* keys, unsigned* keys_out, const int* rows, int* order,
+                             int64_t n, void* temp, size_t temp_bytes, hipStream_t st);
+
 // The prep pass: the FP64 centroids, G and G~ (one wave per frame), then,
 // if f.op is set, the operand (one workgroup per tile and 4 K-groups).
 // side 0: plain operand; +1 / -1: the dithered split's reference / query
@@ -156,11 +237,13 @@ hipError_t launch_eps(const DevFrames& fit, const DevFrames& ref, double kappa, 
 // only, the reference frame's mirrored list when it lies below that
 // frame's shared threshold L.thr.  ph_run < ref_phases walks phases
 // 0..ph_run-1 only (every ref_phases-th reference tile pair: the landmark
-// pass); 0 = all.
+// pass); 0 = all.  tiles: only the listed reference pairs of each block of
+// kFilterFitTiles fit tiles, dealt out over the phases.
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st,
-                           const Mirror* mirror = nullptr, int ph_run = 0);
+                           const Mirror* mirror = nullptr, int ph_run = 0,
+                           const TileList* tiles = nullptr);
 // The window of a symmetric self query (fit: the reference set's query
 // view): eps2[r] = 2 kappa max(G~q[r] + max G~ref, G~ref[r] + max G~q);
 // *gmax_q receives max G~q.
@@ -169,8 +252,15 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
 // After the landmark pass (lists L of n rows, reference phases `phases`):
 // thr[q] = the certified bound of row q's k1-th smallest key in the full
 // query, label[q] = its nearest landmark (dense, < 64 ceil(pairs / phases)).
+// keys (if given): keys[q] orders rows by their nearest landmark among every
+// cell-th one, then by the distance to it, and rows[q] = q; leaders[cell] =
+// the first cell whose landmark is among the leader_rank + 1 nearest of this
+// cell's landmark.  label null: the lists are of a band pass, and thr[q] is
+// only lowered.
 hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* eps2,
-                               int phases, unsigned* thr, int* label, hipStream_t st);
+                               int phases, unsigned* thr, int* label, hipStream_t st,
+                               int cell = 1, unsigned* keys = nullptr, int* rows = nullptr,
+                               int* leaders = nullptr, int leader_rank = 0);
 // order[0..n) = rows grouped by label (counting sort; counts holds nlab ints).
 hipError_t launch_row_order(const int* label, int64_t n, int nlab, int* counts, int* order,
                             hipStream_t st);

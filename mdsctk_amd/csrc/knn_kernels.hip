@@ -43,6 +43,7 @@
 #include <cmath>
 #include <mutex>
 
+#include "frame_math.h"
 #include "knn_device.h"
 
 namespace mdsctk {
@@ -60,14 +61,6 @@ constexpr int kMergeSmallK1 = 256;
 // ---------------------------------------------------------------------------
 // small helpers
 
-__device__ __forceinline__ unsigned short bf16_rne(float v) {
-  unsigned u = __float_as_uint(v);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
-}
-__device__ __forceinline__ double bf16_val(unsigned short h) {
-  return (double)__uint_as_float(((unsigned)h) << 16);
-}
 __device__ __forceinline__ unsigned short f16_rne(float v) {
   _Float16 h = (_Float16)v;
   return __builtin_bit_cast(unsigned short, h);
@@ -77,11 +70,6 @@ __device__ __forceinline__ double f16_val(unsigned short h) {
 }
 
 __device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-__device__ __forceinline__ double wave_sum_d(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
   return v;
@@ -248,11 +236,6 @@ __device__ __forceinline__ float lambda_upper(const float* m) {
 // ---------------------------------------------------------------------------
 // prep: one 192-thread workgroup per 32-frame tile.  Thread t -> plane
 // c = t/64, lane l = t%64 of that plane's operand block.
-
-// One atom's coordinates: a single 12-byte load per lane.
-struct F3 {
-  float x, y, z;
-};
 
 // Per-atom scale of the dithered split (a golden-ratio sequence in [1, 2)).
 // Reference operands carry sqrt(w) x * s_a and query operands sqrt(w) x / s_a,
@@ -613,6 +596,10 @@ struct ContractParams {
   int* mcnt;
   float* movf;
   int mcap;
+  // The reference pairs to walk, [blocks of kFilterFitTiles fit tiles][ref_pairs]
+  // in ascending order, and how many per block (null: all).
+  const int* tlist;
+  const int* tcount;
 };
 
 // What the contraction's epilogue produces.
@@ -1027,15 +1014,33 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     if (item >= n_items) break;
     const int fb = item / P.ph_run;
     const int ph = item - fb * P.ph_run;
-    const int n_tiles = (P.ref_pairs - ph + P.phases - 1) / P.phases;  // ref pairs ph, ph+R, ...
+    // Tile t of the item is reference pair ph + t R, or that entry of the
+    // block's tile list.
+    const int lb = fb * FT / kFilterFitTiles;
+    const int* const tlist = P.tlist ? P.tlist + (int64_t)lb * P.ref_pairs + ph : nullptr;
+    const int n_pairs = P.tlist ? P.tcount[lb] : P.ref_pairs;
+    const int n_tiles = (n_pairs - ph + P.phases - 1) / P.phases;
+    auto pair_of = [&](int t) -> int {
+      const int u = t * P.phases;
+      return tlist ? __builtin_amdgcn_readfirstlane(tlist[u]) : ph + u;
+    };
     // First tile of the item: 0, or for kOutSym the first reference pair at
     // or after the fit block (pair p holds frames 64p.., the block 32*FT*fb..).
+    // A listed block may span two fit blocks (FP32): the second one's first
+    // entry may lie before it.
     int t0 = 0;
     if constexpr (MODE == kOutSym) {
       const int p_min = fb * FT / kRefTilesPerWG;
-      if (p_min > ph) t0 = (p_min - ph + P.phases - 1) / P.phases;
+      if (tlist) {
+        if (n_tiles > 0 && pair_of(0) < p_min) t0 = 1;
+      } else if (p_min > ph) {
+        t0 = (p_min - ph + P.phases - 1) / P.phases;
+      }
     }
-    if (t0 >= n_tiles) continue;
+    if (t0 >= n_tiles) {
+      // the merge reads the headers, cleared before the launch
+      continue;
+    }
     const int64_t fit_idx = (int64_t)(FT * fb + fi) * kTile + (lane & 31);
     const bool fvalid = fit_idx < P.n_fit;
     const int list_id = (ph * 2 + ri) * 2 + (lane >> 5);
@@ -1052,16 +1057,18 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     // (never used).
     const uint4* const fit_base =
         P.fop + (int64_t)(FT * fb + (copier ? wave : 2) - kRefTilesPerWG) * ng * TILE_VEC;
-    auto src_of = [&](int t, int g) -> const uint4* {
-      if (t >= n_tiles) t = n_tiles - 1;
+    // p_cur, p_next: the current and the next tile's reference pair (its own
+    // again past the last tile, where the copies are never used).
+    int p_cur = pair_of(t0);
+    int p_next = t0 + 1 < n_tiles ? pair_of(t0 + 1) : p_cur;
+    auto src_of = [&](int p, int g) -> const uint4* {
       if (wave >= kRefTilesPerWG) return fit_base + (int64_t)g * TILE_VEC;
-      const int p = ph + t * P.phases;
       return P.rop + ((int64_t)(kRefTilesPerWG * p + wave) * ng + g) * TILE_VEC;
     };
-    auto dma_stage = [&](int t, int g, uint4* dst) {
+    auto dma_stage = [&](int g, uint4* dst) {
       if (!copier) return;
-      if (g >= ngs) { g -= ngs; ++t; }
-      const uint4* src = src_of(t, g) + lane;
+      const bool over = g >= ngs;
+      const uint4* src = src_of(over ? p_next : p_cur, over ? g - ngs : g) + lane;
 #pragma unroll
       for (int j = 0; j < BPG; ++j)
         __builtin_amdgcn_global_load_lds((const void*)(src + j * 64),
@@ -1070,13 +1077,13 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
 
     __syncthreads();  // previous item's readers of sbuf*/sGr/sThr are done
     if (tid < 2 * kTile) {
-      const int64_t f0 = (int64_t)(ph + t0 * P.phases) * 2 * kTile + tid;
+      const int64_t f0 = (int64_t)p_cur * 2 * kTile + tid;
       sGr[t0 & 1][tid] = P.rGt[f0];
       if constexpr (MODE == kOutSym) sThr[t0 & 1][tid] = ref_thr(f0);
     }
-    dma_stage(t0, 0, d0);
-    dma_stage(t0, 1, d1);
-    if constexpr (PIPE) dma_stage(t0, 2, d2);
+    dma_stage(0, d0);
+    dma_stage(1, d1);
+    if constexpr (PIPE) dma_stage(2, d2);
     stage_barrier<BPG>();  // stage 0 (and with PIPE stage 1) landed
     // PIPE: the fragments of the stage about to be computed (B double-buffered)
     uint4 bh0[3], bl0[3], bh1[3], bl1[3], ah, al;
@@ -1091,14 +1098,14 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     }
 
     for (int t = t0; t < n_tiles; ++t) {
-      const int p = ph + t * P.phases;
+      const int p = p_cur;
       // Loads consumed only at the end of the tile: the next tile's G~ (and
       // for kOutSym its frames' thresholds) and the shared per-query
       // threshold.
       double g_next = 0.0;
       float thr_next = INFINITY;
       if (tid < 2 * kTile && t + 1 < n_tiles) {
-        const int64_t f1 = (int64_t)(p + P.phases) * 2 * kTile + tid;
+        const int64_t f1 = (int64_t)p_next * 2 * kTile + tid;
         g_next = P.rGt[f1];
         if constexpr (MODE == kOutSym) thr_next = ref_thr(f1);
       }
@@ -1120,16 +1127,16 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
         // never used).
         for (int g = 0; g < ng; g += 4) {
           pipe_stage<PREC, true, true>(acc, a0, a1, b1, bh0, bl0, bh1, bl1, ah, al, lane);
-          dma_stage(t, g + 3, d3);
+          dma_stage(g + 3, d3);
           stage_barrier_vm<BPG>();
           pipe_stage<PREC, true, true>(acc, a1, a2, b2, bh1, bl1, bh0, bl0, ah, al, lane);
-          dma_stage(t, g + 4, d0);
+          dma_stage(g + 4, d0);
           stage_barrier_vm<BPG>();
           pipe_stage<PREC, true, true>(acc, a2, a3, b3, bh0, bl0, bh1, bl1, ah, al, lane);
-          dma_stage(t, g + 5, d1);
+          dma_stage(g + 5, d1);
           stage_barrier_vm<BPG>();
           pipe_stage<PREC, true, true>(acc, a3, a0, b0, bh1, bl1, bh0, bl0, ah, al, lane);
-          dma_stage(t, g + 6, d2);
+          dma_stage(g + 6, d2);
           stage_barrier_vm<BPG>();
         }
       } else {
@@ -1141,13 +1148,13 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
         // Measured 6 % faster than issuing the copy first.
         for (int g = 0; g < ngs; g += 3) {
           mma_group<PREC, TRACE>(acc, a0, b0, lane);
-          dma_stage(t, g + 2, d2);
+          dma_stage(g + 2, d2);
           stage_barrier<BPG>();
           if (g + 1 < ng) mma_group<PREC, TRACE>(acc, a1, b1, lane);
-          dma_stage(t, g + 3, d0);
+          dma_stage(g + 3, d0);
           stage_barrier<BPG>();
           if (g + 2 < ng) mma_group<PREC, TRACE>(acc, a2, b2, lane);
-          dma_stage(t, g + 4, d1);
+          dma_stage(g + 4, d1);
           stage_barrier<BPG>();
         }
       }
@@ -1232,11 +1239,14 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
                           (unsigned)fit_idx, lane);
         }
       }
-      if constexpr (MODE == kOutDebug) continue;
+      if constexpr (MODE != kOutDebug) {
       const float thr_before = thr;
       compact_lists<PER>(P.ent, my_base, cnt, thr, ovf, e2, P.k1, P.cap, fvalid);
       thr = fminf(thr, __shfl_xor(thr, 32));
       if (fvalid && P.thr && thr < thr_before) atomicMin(&P.thr[fit_idx], __float_as_uint(thr));
+      }
+      p_cur = p_next;
+      if (t + 2 < n_tiles) p_next = pair_of(t + 2);
     }
     if (fvalid && MODE != kOutDebug) {
       P.cnt[hdr] = cnt;
@@ -1654,14 +1664,21 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
                                                            int cap, int k1,
                                                            const float* __restrict__ eps2,
                                                            int phases, unsigned* __restrict__ thr,
-                                                           int* __restrict__ label) {
+                                                           int* __restrict__ label, int cell,
+                                                           unsigned* __restrict__ keys,
+                                                           int* __restrict__ rows,
+                                                           int* __restrict__ leaders,
+                                                           int leader_rank) {
   const int64_t q = blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   __shared__ unsigned hist[256];
   __shared__ unsigned s_prefix;
   __shared__ int s_kk, s_total;
-  __shared__ unsigned long long s_best;
+  __shared__ unsigned long long s_best, s_cell;
+  __shared__ int s_leader;
   const int* c = cnt + q * nl;
+  const unsigned span = 2u * kTile * (unsigned)phases;
+  auto dense = [&](unsigned r) { return (r / span) * (2u * kTile) + r % (2u * kTile); };
   const uint2* e = ent + q * (int64_t)nl * cap;
   auto visit = [&](auto&& f) {
     for (int l = wave; l < nl; l += 4) {
@@ -1671,62 +1688,91 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
   };
   if (tid == 0) {
     s_total = 0;
-    s_best = ~0ull;
+    s_best = s_cell = ~0ull;
   }
   __syncthreads();
   {
     int part = 0;
-    unsigned long long best = ~0ull;
+    unsigned long long best = ~0ull, near = ~0ull;
     for (int l = tid; l < nl; l += 256) part += c[l];
     atomicAdd(&s_total, part);
-    visit([&](const uint2 x) {
-      const unsigned long long kx = ((unsigned long long)x.x << 32) | x.y;
-      best = kx < best ? kx : best;
-    });
-    atomicMin(&s_best, best);
+    if (label) {
+      visit([&](const uint2 x) {
+        const unsigned long long kx = ((unsigned long long)x.x << 32) | x.y;
+        best = kx < best ? kx : best;
+        if (keys && dense(x.y) % (unsigned)cell == 0) near = kx < near ? kx : near;
+      });
+      atomicMin(&s_best, best);
+      if (keys) atomicMin(&s_cell, near);
+    }
   }
   __syncthreads();
-  if (tid == 0) {
-    int lab = 0;
-    if (s_best != ~0ull) {
-      const unsigned r = (unsigned)(s_best & 0xffffffffu);
-      const unsigned span = 2u * kTile * (unsigned)phases;
-      lab = (int)((r / span) * (2u * kTile) + r % (2u * kTile));
+  if (tid == 0 && label) {
+    label[q] = s_best != ~0ull ? (int)dense((unsigned)(s_best & 0xffffffffu)) : 0;
+    if (keys) {
+      // cell number, then the distance's leading 19 bits (its exponent and
+      // 11 of the fraction): enough to lay like distances side by side
+      const unsigned long long b = s_cell != ~0ull ? s_cell : s_best;
+      const unsigned lab = b != ~0ull ? dense((unsigned)(b & 0xffffffffu)) / (unsigned)cell : 0u;
+      keys[q] = (lab << 19) | ((unsigned)(b >> 32) >> 12 & 0x7ffffu);
+      rows[q] = (int)q;
     }
-    label[q] = lab;
+  }
+  // the rank-th smallest key (0-based)
+  auto select = [&](int rank) -> unsigned {
+    unsigned prefix = 0;
+    int kk = rank;
+    for (int shift = 24; shift >= 0; shift -= 8) {
+      hist[tid] = 0;
+      __syncthreads();
+      const unsigned mhi = (shift == 24) ? 0u : (0xFFFFFFFFu << (shift + 8));
+      visit([&](const uint2 x) {
+        if ((x.x & mhi) == (prefix & mhi)) atomicAdd(&hist[(x.x >> shift) & 255u], 1u);
+      });
+      __syncthreads();
+      if (tid == 0) {
+        unsigned cum = 0;
+        int b = 0;
+        for (; b < 255; ++b) {
+          if (cum + hist[b] > (unsigned)kk) break;
+          cum += hist[b];
+        }
+        s_prefix = prefix | ((unsigned)b << shift);
+        s_kk = kk - (int)cum;
+      }
+      __syncthreads();
+      prefix = s_prefix;
+      kk = s_kk;
+    }
+    return prefix;
+  };
+  // A cell's landmark: the first cell landmark among its nearest ones leads
+  // it, so that cells of one neighbourhood follow one another in the order.
+  if (leaders && (q / (2 * kTile)) % phases == 0 && dense((unsigned)q) % (unsigned)cell == 0) {
+    if (tid == 0) s_leader = (int)(dense((unsigned)q) / (unsigned)cell);
+    __syncthreads();
+    if (s_total > leader_rank) {
+      const unsigned near = select(leader_rank);
+      int lead = INT_MAX;
+      visit([&](const uint2 x) {
+        const unsigned l = dense(x.y);
+        if (x.x <= near && l % (unsigned)cell == 0) lead = min(lead, (int)(l / (unsigned)cell));
+      });
+      atomicMin(&s_leader, lead);
+      __syncthreads();
+    }
+    if (tid == 0) leaders[dense((unsigned)q) / (unsigned)cell] = s_leader;
   }
   if (s_total < k1) {
-    if (tid == 0) thr[q] = kInfBits;
+    if (tid == 0 && label) thr[q] = kInfBits;
     return;
   }
-  unsigned prefix = 0;
-  int kk = k1 - 1;
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    hist[tid] = 0;
-    __syncthreads();
-    const unsigned mhi = (shift == 24) ? 0u : (0xFFFFFFFFu << (shift + 8));
-    visit([&](const uint2 x) {
-      if ((x.x & mhi) == (prefix & mhi)) atomicAdd(&hist[(x.x >> shift) & 255u], 1u);
-    });
-    __syncthreads();
-    if (tid == 0) {
-      unsigned cum = 0;
-      int b = 0;
-      for (; b < 255; ++b) {
-        if (cum + hist[b] > (unsigned)kk) break;
-        cum += hist[b];
-      }
-      s_prefix = prefix | ((unsigned)b << shift);
-      s_kk = kk - (int)cum;
-    }
-    __syncthreads();
-    prefix = s_prefix;
-    kk = s_kk;
-  }
+  const unsigned prefix = select(k1 - 1);
   if (tid == 0) {
     const double tau = (double)__uint_as_float(prefix), e2 = (double)eps2[q];
     const float bound = (float)((tau + e2) * (1.0 + 1e-6) + e2);
-    thr[q] = bound < INFINITY ? __float_as_uint(bound) + 1u : kInfBits;
+    const unsigned bits = bound < INFINITY ? __float_as_uint(bound) + 1u : kInfBits;
+    thr[q] = label ? bits : min(bits, thr[q]);
   }
 }
 
@@ -1769,6 +1815,11 @@ __global__ void order_scatter_kernel(const int* __restrict__ label, int64_t n,
                                      int* __restrict__ offsets, int* __restrict__ order) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q < n) order[atomicAdd(&offsets[label[q]], 1)] = (int)q;
+}
+
+__global__ void iota_kernel(int* __restrict__ p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = i;
 }
 
 __global__ void fill_int_kernel(int* __restrict__ p, int64_t n, int v) {
@@ -2270,7 +2321,7 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st, const Mirror* mirror,
-                           int ph_run) {
+                           int ph_run, const TileList* tiles) {
   ContractParams P;
   P.rop = ref.op;
   P.fop = fit.op;
@@ -2297,6 +2348,10 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
   P.mcnt = mirror ? mirror->cnt : nullptr;
   P.movf = mirror ? mirror->ovf : nullptr;
   P.mcap = mirror ? mirror->cap : 0;
+  P.tlist = tiles ? tiles->list : nullptr;
+  P.tcount = tiles ? tiles->count : nullptr;
+  if (tiles && (!tiles->list || !tiles->count || ph_run || fit.n_tiles % kFilterFitTiles))
+    return hipErrorInvalidValue;
   if (P.ph_run > ref_phases || ref_phases < 1) return hipErrorInvalidValue;
   // the split forms' pipelined K-loop walks K-groups four at a time
   if (ref.prec != kFP32 && (ref.n_groups % kSplitGroupAlign)) return hipErrorInvalidValue;
@@ -2425,11 +2480,18 @@ hipError_t launch_permute_thresholds(const unsigned* src, const int* perm, const
 }
 
 hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* eps2,
-                               int phases, unsigned* thr, int* label, hipStream_t st) {
+                               int phases, unsigned* thr, int* label, hipStream_t st, int cell,
+                               unsigned* keys, int* rows, int* leaders, int leader_rank) {
   if (n <= 0) return hipSuccess;
-  if (k1 < 1 || phases < 1 || !thr || !label) return hipErrorInvalidValue;
+  if (k1 < 1 || phases < 1 || !thr || cell < 1 || (keys && (!label || !rows)))
+    return hipErrorInvalidValue;
+  if (leaders) {  // a cell whose landmark is padding leads itself
+    const int ncells = (int)((2 * kTile * ((n + 2 * kTile * phases - 1) / (2 * kTile * phases)) + cell - 1) / cell);
+    hipLaunchKernelGGL(iota_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, st, leaders,
+                       ncells);
+  }
   hipLaunchKernelGGL(landmark_cap_kernel, dim3((unsigned)n), dim3(256), 0, st, L.ent, L.cnt, L.nl,
-                     L.cap, k1, eps2, phases, thr, label);
+                     L.cap, k1, eps2, phases, thr, label, cell, keys, rows, leaders, leader_rank);
   return hipGetLastError();
 }
 
