@@ -261,6 +261,11 @@ void free_plain(mdsctk_knn_ctx* c) {
   p = DevFrames();
 }
 
+void free_ordered(mdsctk_knn_ctx* c) {
+  dfree(c, c->ordered.mem);
+  c->ordered = OrderedRef();
+}
+
 }  // namespace
 
 // The --nofit operands of the resident set (frames as given), built on first
@@ -339,6 +344,7 @@ int set_reference_impl(mdsctk_knn_ctx* c, const float* xyz, bool on_device, int6
   HIP_TRY(c, hipSetDevice(c->device));
   free_frames(c, c->ref);
   free_plain(c);
+  free_ordered(c);
   c->ref_axes = false;
   release_mirror_lists(c);
   dfree(c, c->data_shift);
@@ -405,6 +411,7 @@ int set_data_reference_impl(mdsctk_knn_ctx* c, const double* x, int64_t n_ref, i
   HIP_TRY(c, hipSetDevice(c->device));
   free_frames(c, c->ref);
   free_plain(c);
+  free_ordered(c);
   c->ref_axes = false;
   release_mirror_lists(c);
   dfree(c, c->data_shift);
@@ -473,6 +480,7 @@ void slot_release(mdsctk_knn_ctx* c, Slot& s) {
   dfree(c, s.ws_sym);
   dfree(c, s.ws_relist);
   dfree(c, s.ws_sort);
+  dfree(c, s.ws_cross);
   for (auto& e : s.ev)
     if (e) (void)hipEventDestroy(e);
   if (s.st) (void)hipStreamDestroy(s.st);
@@ -589,6 +597,63 @@ size_t fused_list_entries(const mdsctk_knn_ctx* c, int64_t n_fit, int k1) {
   return (size_t)n_fit * phases * 4 * list_capacity_for(k1);
 }
 
+namespace {
+
+// Landmark pairs of a cross query: every stride-th reference pair, 1/32 of
+// them but at least 8 (k+1) frames.  The (k+1)-th smallest key of L landmarks
+// bounds a row's threshold at rank (k+1) n / L.
+int cross_stride(const mdsctk_knn_ctx* c, int k1) {
+  const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
+  const int want = std::max(8 * k1 / (2 * kTile) + 1, ref_pairs / 32);
+  return std::max(1, std::max(ref_pairs / want, ref_pairs * 2 * kTile / kFilterMaxCells + 1));
+}
+
+// The ordered form's workspace, carved from `cv` (or only its size).
+size_t carve_cross(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit, Carve& cv, CrossPlan* x) {
+  const OrderedRef& o = c->ordered;
+  const int n_tiles = std::max(kTileAlign, padded_tiles(n_fit));
+  const size_t rows = (size_t)n_tiles * kTile, n = (size_t)n_fit;
+  const int fit_blocks = n_tiles / kFilterFitTiles;
+  const size_t tiles = (size_t)fit_blocks * (c->ref.n_tiles / kRefTilesPerWG);
+  DevFrames f;
+  f.n = n_fit;
+  f.natoms = c->ref.natoms;
+  f.n_tiles = f.cap_tiles = n_tiles;
+  f.n_groups = c->ref.n_groups;
+  f.prec = c->ref.prec;
+  f.owns_xyz = false;
+  f.cen = (double*)cv.take(rows * 3 * sizeof(double));
+  f.G = (double*)cv.take(rows * sizeof(double));
+  f.Gt = (double*)cv.take(rows * sizeof(double));
+  f.op = (uint4*)cv.take(operand_bytes(f.prec, n_tiles, f.n_groups));
+  f.rot = (double*)cv.take(rows * 9 * sizeof(double));
+  x->fit = f;
+  x->order = (int*)cv.take(n * sizeof(int));
+  x->rows = (int*)cv.take(n * sizeof(int));
+  x->keys = (unsigned*)cv.take(n * sizeof(unsigned));
+  x->label = (int*)cv.take(n * sizeof(int));
+  x->thr0 = (unsigned*)cv.take(n * sizeof(unsigned));
+  x->eps0 = (float*)cv.take(n * sizeof(float));
+  x->sort_bytes = n_fit > kRankSortMax ? sort_order_scratch(n_fit) : 0;
+  if (x->sort_bytes) {
+    x->keys_out = (unsigned*)cv.take(n * sizeof(unsigned));
+    x->sort_temp = cv.take(x->sort_bytes);
+  }
+  x->set.op = (uint4*)cv.take(filter_operand_bytes(o.sh, n_tiles));
+  x->set.full = (float4*)cv.take(rows * sizeof(float4));
+  x->set.pre = (float4*)cv.take(rows * sizeof(float4));
+  x->set.place = (double*)cv.take(rows * 12 * sizeof(double));
+  x->set.extra = (ushort*)cv.take(rows * 36 * sizeof(ushort));
+  x->tiles.flags = (unsigned char*)cv.take(tiles);
+  x->tiles.list = (int*)cv.take(tiles * sizeof(int));
+  x->tiles.count = (int*)cv.take(fit_blocks * sizeof(int));
+  x->tiles.ctrl = (int*)cv.take(2 * sizeof(int));
+  x->lstride = cross_stride(c, q.k1);
+  return cv.used;
+}
+
+}  // namespace
+
 int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Carve* cv) {
   const DevFrames& fit = s.fit;
   const int64_t n_fit = fit.n;
@@ -658,12 +723,201 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   p->kappa = (c->w.metric == kMetricRMSD ? kappa_for(c->prec, c->ref.natoms)
                                          : kappa_data(c->prec, c->ref.natoms)) *
              c->eps_scale;
+  p->x.on = false;
+  const size_t xb = (cv || fit.xyz == c->ref.xyz) ? 0 : cross_bytes(c, q, n_fit);
+  if (xb) {
+    int rc = ensure(c, &s.ws_cross, &s.ws_cross_bytes, xb, "ordered query frames");
+    if (rc == MDSCTK_ERR_NOMEM) {
+      tl_ctx_err.erase(c);  // every tile instead
+      return 0;
+    }
+    if (rc) return rc;
+    Carve xc;
+    xc.base = (char*)s.ws_cross;
+    xc.size = s.ws_cross_bytes;
+    carve_cross(c, q, n_fit, xc, &p->x);
+    p->x.filter_grid = std::max(8, c->n_cu & ~7);
+    p->x.on = true;
+  }
+  return 0;
+}
+
+namespace {
+
+// A cross query against the ordered set: a landmark pass (every lstride-th
+// reference pair) bounds each row's threshold and names its nearest landmark,
+// the queries are put in that order, the filter lists the tiles that can hold
+// a candidate, and the contraction walks those.  The merge re-scores from the
+// frames as given, so outputs equal the unordered form's.
+int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPlan& p,
+                  double* d_dist, int* d_idx, bool timing) {
+  const DevFrames& fit = s.fit;
+  const int64_t n = fit.n;
+  const CrossPlan& x = p.x;
+  const OrderedRef& o = c->ordered;
+  DevFrames R = o.f;
+  R.gmax = c->ref.gmax;
+  if (timing) HIP_TRY(c, hipEventRecord(s.ev[2], s.st));
+  // the landmark pairs as one list, split over enough phases to fill the grid
+  const int lm_pairs = (c->ref.n_tiles / kRefTilesPerWG + x.lstride - 1) / x.lstride;
+  const int blocks = std::max(1, x.fit.n_tiles / contract_fit_tiles(c->prec));
+  const int lm_phases = std::max(1, std::min({p.phases, lm_pairs / 2, 2 * p.grid / blocks}));
+  TileList lm = x.tiles;
+  lm.shared = true;
+  Lists LL = p.L;
+  LL.nl = 4 * lm_phases;
+  LL.thr = x.thr0;
+  HIP_TRY(c, launch_stride_list(c->ref.n_tiles, x.lstride, lm, s.st));
+  HIP_TRY(c, launch_init_lists(LL, n, s.st));
+  HIP_TRY(c, launch_eps(fit, R, p.kappa, x.eps0, s.n_cand, s.st));
+  HIP_TRY(c, launch_contract(R, fit, LL, x.eps0, q.k1, lm_phases, false, nullptr, p.grid, s.st,
+                             nullptr, 0, &lm));
+  HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, x.eps0, x.lstride, x.thr0, x.label, s.st, 1, x.keys,
+                                 x.rows));
+  if (x.sort_temp)
+    HIP_TRY(c, launch_sort_order(nullptr, nullptr, 0, x.keys, x.keys_out, x.rows, x.order, n,
+                                 x.sort_temp, x.sort_bytes, s.st));
+  else
+    HIP_TRY(c, launch_rank_sort(x.keys, x.order, n, s.st));
+  HIP_TRY(c, launch_prep(x.fit, c->w, dithered(c) ? -1 : 0, nullptr, 0, s.st, fit.xyz, x.order,
+                         x.fit.rot));
+  DevFrames src = fit;
+  HIP_TRY(c, launch_filter_prep(src, c->w, o.sh, o.mean, o.mc, o.slots, x.order, x.set, s.st));
+  HIP_TRY(c, launch_eps(x.fit, R, p.kappa, p.eps2, nullptr, s.st));
+  HIP_TRY(c, launch_permute_thresholds(x.thr0, x.order, p.eps2, n, p.L.thr, s.st));
+  HIP_TRY(c, launch_init_lists(p.L, n, s.st, false));
+  HIP_TRY(c, launch_filter(o.set, x.set, c->ref.n, n, c->ref.n_tiles, x.fit.n_tiles, o.sh, o.mc,
+                           p.L.thr, p.eps2, false, x.filter_grid, x.tiles, s.st));
+  HIP_TRY(c, launch_contract(R, x.fit, p.L, p.eps2, q.k1, p.phases, false, nullptr, p.grid, s.st,
+                             nullptr, 0, &x.tiles));
+  if (timing) HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
+  HIP_TRY(c, launch_merge(c->ref, fit, c->w, p.L, p.eps2, q.k1, q.k_out, q.rank_off, false, d_dist,
+                          d_idx, p.d_fallback, s.n_cand, nullptr, s.st, nullptr, x.order, o.order));
+  if (timing) HIP_TRY(c, hipEventRecord(s.ev[4], s.st));
+  return 0;
+}
+
+}  // namespace
+
+size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
+  if (!q.fused || q.nofit || n_fit < kCrossMinFit || c->budget) return 0;
+  {
+    std::lock_guard<std::mutex> g(c->plain_mu);
+    if (!c->ordered.built) return 0;
+  }
+  Carve cv;
+  cv.base = (char*)256;  // sizes only
+  cv.size = SIZE_MAX / 2;
+  CrossPlan x;
+  return carve_cross(c, q, n_fit, cv, &x);
+}
+
+// Ordering costs about a landmark pass of the whole set (L landmarks a
+// frame) and two operand builds, and saves most of a query's pairs: it is
+// done when the frames queried so far reach kCrossMinSeen.  Not under an HBM
+// budget, nor when it would take more than a quarter of the free memory:
+// the other workspaces keep their room.
+int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
+  const int64_t n = c->ref.n;
+  if (!c->ref_axes || n < kCrossMinRef || n * c->ref.natoms < kCrossMinWork || c->budget) return 0;
+  std::lock_guard<std::mutex> g(c->plain_mu);
+  OrderedRef& o = c->ordered;
+  o.seen += n_fit;
+  if (o.built || o.failed || o.seen < kCrossMinSeen) return 0;
+  const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
+  const size_t rows = (size_t)c->ref.n_tiles * kTile;
+  // cells of about 384 frames
+  const int cells = (int)std::min<int64_t>(1024, std::max<int64_t>(128, n / 384));
+  const int lstride = std::max(1, ref_pairs * 2 * kTile / cells);
+  o.sh = filter_shape(c->ref.natoms);
+  const size_t sort_temp = sort_order_scratch(n);
+  const size_t opb = operand_bytes(c->ref.prec, c->ref.n_tiles, c->ref.n_groups);
+  const size_t bytes =
+      Carve::round(rows * 3 * sizeof(double)) + 2 * Carve::round(rows * sizeof(double)) +
+      Carve::round(opb) + Carve::round(rows * 9 * sizeof(double)) +
+      Carve::round((size_t)n * sizeof(int)) + Carve::round(filter_operand_bytes(o.sh, c->ref.n_tiles)) +
+      2 * Carve::round(rows * sizeof(float4)) + Carve::round(rows * 12 * sizeof(double)) +
+      Carve::round(rows * 36 * sizeof(ushort)) + Carve::round(o.sh.natoms * 3 * sizeof(double)) +
+      Carve::round(o.sh.slots() * sizeof(int)) + Carve::round(sizeof(FilterMean));
+  const size_t scratch = Carve::round((size_t)n * sizeof(unsigned long long)) +
+                         3 * Carve::round((size_t)n * sizeof(int)) + Carve::round(sort_temp) +
+                         Carve::round(12 * kFilterSamples * sizeof(double));
+  size_t free_b = 0, total_b = 0;
+  HIP_TRY(c, hipMemGetInfo(&free_b, &total_b));
+  void* tmp = nullptr;
+  o.failed = true;  // until everything below has worked
+  if (bytes + scratch > free_b / 4) return 0;
+  if (dalloc(c, &o.mem, bytes, "ordered reference set") || dalloc(c, &tmp, scratch, "ordering")) {
+    dfree(c, o.mem);
+    o.mem = nullptr;
+    tl_ctx_err.erase(c);
+    return 0;
+  }
+  Carve cv, ct;
+  cv.base = (char*)o.mem;
+  cv.size = bytes;
+  ct.base = (char*)tmp;
+  ct.size = scratch;
+  DevFrames f = c->ref;
+  f.xyz = nullptr;
+  f.owns_xyz = false;
+  f.op_q = nullptr;
+  f.Gt_q = nullptr;
+  f.cen = (double*)cv.take(rows * 3 * sizeof(double));
+  f.G = (double*)cv.take(rows * sizeof(double));
+  f.Gt = (double*)cv.take(rows * sizeof(double));
+  f.op = (uint4*)cv.take(opb);
+  f.rot = (double*)cv.take(rows * 9 * sizeof(double));
+  o.order = (int*)cv.take((size_t)n * sizeof(int));
+  o.set.op = (uint4*)cv.take(filter_operand_bytes(o.sh, c->ref.n_tiles));
+  o.set.full = (float4*)cv.take(rows * sizeof(float4));
+  o.set.pre = (float4*)cv.take(rows * sizeof(float4));
+  o.set.place = (double*)cv.take(rows * 12 * sizeof(double));
+  o.set.extra = (ushort*)cv.take(rows * 36 * sizeof(ushort));
+  o.mean = (double*)cv.take(o.sh.natoms * 3 * sizeof(double));
+  o.slots = (int*)cv.take(o.sh.slots() * sizeof(int));
+  o.mc = (FilterMean*)cv.take(sizeof(FilterMean));
+  auto* near = (unsigned long long*)ct.take((size_t)n * sizeof(unsigned long long));
+  auto* keys = (unsigned*)ct.take((size_t)n * sizeof(int));
+  auto* keys_out = (unsigned*)ct.take((size_t)n * sizeof(int));
+  int* ids = (int*)ct.take((size_t)n * sizeof(int));
+  void* temp = ct.take(sort_temp);
+  double* align = (double*)ct.take(12 * kFilterSamples * sizeof(double));
+  auto run = [&]() -> int {
+    if (!o.mc || !align) return fail(c, MDSCTK_ERR_ARG, "internal: ordered set carve");
+    HIP_TRY(c, launch_fill_near(near, n, s.st));
+    Lists none;
+    none.nl = 4;
+    none.cap = 256;
+    HIP_TRY(c, launch_contract(c->ref, query_view(c->ref), none, nullptr, 1, lstride, false, nullptr,
+                               contract_grid(c), s.st, nullptr, 1, nullptr, near));
+    HIP_TRY(c, launch_near_keys(near, n, lstride, keys, ids, s.st));
+    HIP_TRY(c, launch_sort_order(nullptr, nullptr, 0, keys, keys_out, ids, o.order, n, temp,
+                                 sort_temp, s.st));
+    HIP_TRY(c, launch_prep(f, c->w, dithered(c) ? +1 : 0, nullptr, 0, s.st, c->ref.xyz, o.order,
+                           f.rot));
+    HIP_TRY(c, launch_filter_mean(c->ref, c->w, o.sh, align, o.mean, o.mc, o.slots, s.st));
+    HIP_TRY(c, launch_filter_prep(c->ref, c->w, o.sh, o.mean, o.mc, o.slots, o.order, o.set, s.st));
+    HIP_TRY(c, hipStreamSynchronize(s.st));
+    return 0;
+  };
+  const int rc = run();
+  dfree(c, tmp);
+  if (rc) {
+    dfree(c, o.mem);
+    o.mem = nullptr;
+    return rc;
+  }
+  o.f = f;
+  o.failed = false;
+  o.built = true;
   return 0;
 }
 
 int enqueue_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPlan& p,
                   double* d_dist, int* d_idx, bool timing) {
   const DevFrames& fit = s.fit;
+  if (p.x.on) return enqueue_cross(c, s, q, p, d_dist, d_idx, timing);
   HIP_TRY(c, launch_init_lists(p.L, fit.n, s.st));
   const DevFrames& R = ref_ops(c, q.nofit);
   HIP_TRY(c, launch_eps(fit, R, p.kappa, p.eps2, s.n_cand, s.st));
@@ -835,7 +1089,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
         1, std::max<int64_t>((int64_t)nlab * 6 * q.k1 / n, nlab / kFilterMaxCells + 1));
     const int ncells = (nlab + cell - 1) / cell;
     HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, eps2, lstride, L.thr, label, s.st, cell, keys,
-                                   row_ids, leaders, 1 + std::min(q.k1 / 2, nlab / 256)));
+                                   row_ids, leaders, 1 + std::min(q.k1 / 2, nlab / 100)));
     HIP_TRY(c, launch_sort_order(leaders, rank, ncells, keys, keys_out, row_ids, order, n, temp,
                                  sort_temp, s.st));
   } else {
@@ -911,7 +1165,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     LB.nl = 4;
     HIP_TRY(c, launch_init_lists(LB, n, s.st, false));
     HIP_TRY(c, launch_band_list(c->ref.n_tiles, c->ref.n_tiles, kFilterFitTiles,
-                                std::min(ref_pairs, std::max(4, q.k1 / 8 + 2)), tiles, s.st));
+                                std::min(ref_pairs, std::max(12, q.k1 / 8 + 2)), tiles, s.st));
     HIP_TRY(c, launch_contract(mref, mfit, LB, meps2, q.k1, 1, q.nofit, nullptr, grid, s.st,
                                nullptr, 0, &tiles));
     HIP_TRY(c, launch_landmark_cap(LB, n, q.k1, meps2, 1, LM.thr, nullptr, s.st));
@@ -921,14 +1175,14 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   HIP_TRY(c, hipEventRecord(s.ev[6], s.st));
   if (filter)
     HIP_TRY(c, launch_filter(fset, fset, n, n, c->ref.n_tiles, c->ref.n_tiles, fsh, fmean, LM.thr,
-                             meps2, true, phases, std::max(8, c->n_cu & ~7), tiles, s.st));
+                             meps2, true, std::max(8, c->n_cu & ~7), tiles, s.st));
   HIP_TRY(c, launch_contract(mref, mfit, LM, meps2, q.k1, phases, q.nofit, nullptr, grid, s.st,
                              &M, 0, filter ? &tiles : nullptr));
   HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
   HIP_TRY(c, launch_mirror_sum(M, n, msum, s.st));
   HIP_TRY(c, launch_merge(c->ref, fit, c->w, LM, meps2, q.k1, q.k_out, q.rank_off, q.nofit, d_dist,
                           d_idx, d_fallback, s.n_cand, (ordered && !canon) ? order : nullptr, s.st,
-                          &M, canon ? order : nullptr));
+                          &M, canon ? order : nullptr, canon ? order : nullptr));
   HIP_TRY(c, hipEventRecord(s.ev[4], s.st));
   // pairs of the upper block triangle: fit block fb against frames from
   // its own first frame on
@@ -1166,6 +1420,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
   int fused_rc = 1;  // 1: the fused pipeline did not run
   FusedInfo info;
   if (!q.full && q.fused && !plain_missing) {
+    if (xyz && !cv && !q.nofit && (rc = ensure_ordered(c, s, n_fit))) return rc;
     DevFrames saved = ws.fit;
     if (!xyz) ws.fit = query_view(ref_ops(c, q.nofit));
     if (!xyz && c->self_sym && !cv) fused_rc = launch_fused_sym(c, ws, q, d_dist, d_idx, &info);

@@ -42,6 +42,8 @@ struct Slot {
   size_t ws_relist_bytes = 0;
   void* ws_sort = nullptr;  // exact rows with k+1 beyond the LDS select: compaction + sort
   size_t ws_sort_bytes = 0;
+  void* ws_cross = nullptr;  // a cross query's ordered copy and tile lists (CrossPlan)
+  size_t ws_cross_bytes = 0;
   // ev[0] start, ev[1] query prepared, ev[2] before the contraction, ev[3]
   // after it, ev[4] after the merge, ev[5] end; ev[6] after a symmetric self
   // query's landmark pass (so ev[2]..ev[6] is that pass).
@@ -58,6 +60,43 @@ struct QueryShape {
   bool fused = false;  // contraction + merge (else exact rows)
 };
 
+// The resident set in the order its cross queries walk it: rows sorted into
+// cells around landmarks, their contraction operand and their filter operand
+// (filter_kernels.hip).  Made once, when queries have brought enough frames
+// to pay for it; only read afterwards.
+struct OrderedRef {
+  bool built = false, failed = false;
+  int64_t seen = 0;  // query frames since the set became resident
+  void* mem = nullptr;
+  DevFrames f;  // xyz null: the coordinates are the resident set's
+  int* order = nullptr;
+  FilterShape sh;
+  FilterSet set;
+  double* mean = nullptr;
+  FilterMean* mc = nullptr;
+  int* slots = nullptr;
+};
+
+// A cross query against the ordered set: the query frames in the order of
+// their nearest landmark, and the tiles that can hold a candidate.
+struct CrossPlan {
+  bool on = false;
+  int lstride = 1;  // every lstride-th reference pair is a landmark pair
+  DevFrames fit;    // the queries' operand in order
+  int* order = nullptr;
+  int* rows = nullptr;
+  unsigned* keys = nullptr;
+  unsigned* keys_out = nullptr;
+  void* sort_temp = nullptr;
+  size_t sort_bytes = 0;
+  int* label = nullptr;
+  unsigned* thr0 = nullptr;  // thresholds and windows of the queries as given
+  float* eps0 = nullptr;
+  FilterSet set;
+  TileList tiles;
+  int filter_grid = 8;
+};
+
 // Workspace layout and launch shape of one fused batch, fixed before any
 // work is enqueued (so that the enqueue step allocates nothing and can be
 // captured into a graph).
@@ -68,6 +107,7 @@ struct FusedPlan {
   int phases = 0;
   int grid = 0;
   double kappa = 0;
+  CrossPlan x;
 };
 
 // What the fused pipeline did for a batch.
@@ -134,6 +174,7 @@ struct mdsctk_knn_ctx {
   mdsctk::DevFrames ref_plain;
   bool ref_axes = false;
   std::mutex plain_mu;
+  mdsctk::OrderedRef ordered;  // guarded by plain_mu until built
   double* data_shift = nullptr;  // data vectors, Euclidean: the reference set's mean vector
   bool has_ref = false;
   mdsctk::Slot main;  // workspace of the synchronous entry points
@@ -182,6 +223,13 @@ int slot_frames(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
 int prep_slot(mdsctk_knn_ctx* c, Slot& s, bool nofit);
 // The resident set's --nofit operands, built on first use (synchronous).
 int ensure_plain(mdsctk_knn_ctx* c, hipStream_t st);
+// Counts a fitted query's frames and, once they pay for it, orders the
+// resident set for cross queries (synchronous, on slot s); no error if it
+// cannot.
+int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
+// Bytes of slot workspace the ordered form of a cross query of n_fit frames
+// takes (0: it takes every tile).
+size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);
 // Contraction grid (workgroups) and reference phases for a batch of
 // `fit_tiles` query tiles; candidate-list entries a batch of n_fit frames
 // needs (each entry 8 bytes; the headers take 8 bytes per list).

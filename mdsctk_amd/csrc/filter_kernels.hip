@@ -30,8 +30,13 @@
 //
 // Measured, self query of 200000 x 1000 atoms, k = 64 (50 metastable
 // states): the contraction over every tile took 917 ms; the filter takes
-// 121 ms and leaves 7 % of the tiles, which take 68 ms.  Without the first
-// segment the filter alone took over 220 ms.
+// 100 ms (0.9 PFLOP/s of BF16, what a large matrix product reaches on this
+// card is 1.1) and leaves 2.3 % of the tiles, which take 30 ms.  Without the
+// first segment the filter alone took over 220 ms.  Cross query of 4096
+// against 100000 x 500 atoms, k = 50 (one basin): contraction 10.0 ms before;
+// the filter takes 4.2 ms (1.1 PFLOP/s) and leaves tiles for 2.1 ms.  50000
+// against 50000 x 304 atoms in plain FP32, k = 100: 124 ms before, now 5 for
+// the landmarks, 15 for the filter and 26 for the tiles left.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -601,13 +606,13 @@ constexpr int kSampleEvery = 16;
 
 // The fit blocks of one part of the filter: every kSampleEvery-th block
 // (part 0, the sample that decides whether the rest is worth it), the others
-// (part 1).
-__device__ __forceinline__ int part_blocks(int fit_blocks, int part) {
+// (part 1), or all of them (part 2, few blocks).
+__host__ __device__ __forceinline__ int part_blocks(int fit_blocks, int part) {
   const int s = (fit_blocks + kSampleEvery - 1) / kSampleEvery;
-  return part == 0 ? s : fit_blocks - s;
+  return part == 0 ? s : part == 1 ? fit_blocks - s : fit_blocks;
 }
 __device__ __forceinline__ int part_block(int i, int part) {
-  return part == 0 ? i * kSampleEvery : i + i / (kSampleEvery - 1) + 1;
+  return part == 0 ? i * kSampleEvery : part == 1 ? i + i / (kSampleEvery - 1) + 1 : i;
 }
 
 // Too many tiles of the sample are left: the contraction takes every tile.
@@ -897,21 +902,87 @@ __global__ void clear_kernel(uint4* p, int64_t n, int* ctrl) {
   if (i < 2 && ctrl) ctrl[i] = 0;
 }
 
-// A cell's place when cells are sorted by (leader, cell).
+// The last of a cell's chain of leaders (each leader is the cell itself or an
+// earlier one, so the chain ends).
+__device__ __forceinline__ int chief(const int* __restrict__ leaders, int c) {
+  for (int l = leaders[c]; l >= 0 && l < c; l = leaders[c]) c = l;
+  return c;
+}
+
+// A cell's place when cells are sorted by (chief, cell).
 __global__ __launch_bounds__(256) void cell_rank_kernel(const int* __restrict__ leaders, int ncells,
                                                         int* __restrict__ rank) {
   const int c = blockIdx.x * 256 + threadIdx.x;
-  const int mine = c < ncells ? leaders[c] : 0;
+  const int mine = c < ncells ? chief(leaders, c) : 0;
   __shared__ int other[256];
   int r = 0;
   for (int j0 = 0; j0 < ncells; j0 += 256) {
     __syncthreads();
-    other[threadIdx.x] = j0 + (int)threadIdx.x < ncells ? leaders[j0 + threadIdx.x] : INT_MAX;
+    other[threadIdx.x] =
+        j0 + (int)threadIdx.x < ncells ? chief(leaders, j0 + (int)threadIdx.x) : INT_MAX;
     __syncthreads();
     for (int j = 0; j < 256; ++j)
       r += other[j] < mine || (other[j] == mine && j0 + j < c);
   }
   if (c < ncells) rank[c] = r;
+}
+
+__global__ void fill_near_kernel(unsigned long long* p, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = ~0ull;
+}
+
+// A frame's cell is its nearest landmark (numbered densely, as
+// landmark_cap_kernel does), then its distance's leading bits.
+__global__ void near_keys_kernel(const unsigned long long* __restrict__ near, int64_t n, int phases,
+                                 unsigned* __restrict__ keys, int* __restrict__ rows) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const unsigned long long b = near[q];
+  const unsigned r = (unsigned)b, span = 2u * kTile * (unsigned)phases;
+  const unsigned cell = b == ~0ull ? 0u : (r / span) * (2u * kTile) + r % (2u * kTile);
+  keys[q] = (cell << kFilterDistBits) |
+            ((unsigned)(b >> 32) >> (31 - kFilterDistBits) & ((1u << kFilterDistBits) - 1u));
+  rows[q] = (int)q;
+}
+
+// order[place of row q among the keys] = q: 64 rows a workgroup against all
+// keys, a quarter of them per wave, four per LDS read.
+__global__ __launch_bounds__(256) void rank_sort_kernel(const unsigned* __restrict__ keys, int n,
+                                                        int* __restrict__ order) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int q = blockIdx.x * 64 + lane;
+  const unsigned mine = q < n ? keys[q] : 0u;
+  __shared__ __align__(16) unsigned other[1024];
+  __shared__ int part[4][64];
+  int r = 0;
+  for (int j0 = 0; j0 < n; j0 += 1024) {
+    __syncthreads();
+    for (int j = threadIdx.x; j < 1024; j += 256) other[j] = j0 + j < n ? keys[j0 + j] : 0xffffffffu;
+    __syncthreads();
+    const uint4* const o = reinterpret_cast<const uint4*>(other) + wave * 64;
+    const int base = j0 + wave * 256;
+    // keys past n compare as larger, and none of them equals a key below q
+#pragma unroll 4
+    for (int j = 0; j < 64; ++j) {
+      const uint4 k = o[j];
+      const int at = base + 4 * j;
+      r += k.x < mine || (k.x == mine && at < q);
+      r += k.y < mine || (k.y == mine && at + 1 < q);
+      r += k.z < mine || (k.z == mine && at + 2 < q);
+      r += k.w < mine || (k.w == mine && at + 3 < q);
+    }
+  }
+  part[wave][lane] = r;
+  __syncthreads();
+  if (wave == 0 && q < n) order[part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]] = q;
+}
+
+__global__ void stride_list_kernel(int ref_pairs, int stride, int* __restrict__ list,
+                                   int* __restrict__ count) {
+  const int m = (ref_pairs + stride - 1) / stride;
+  for (int i = threadIdx.x; i < m; i += blockDim.x) list[i] = i * stride;
+  if (threadIdx.x == 0) count[0] = m;
 }
 
 __global__ void rank_keys_kernel(const int* __restrict__ rank, int ncells, int64_t n,
@@ -977,7 +1048,7 @@ hipError_t launch_filter_prep(const DevFrames& f, const DevWeights& w, const Fil
 
 hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_ref, int64_t n_fit,
                          int ref_tiles, int fit_tiles, const FilterShape& sh, const FilterMean* mc,
-                         const unsigned* thr, const float* eps2, bool sym, int phases, int grid,
+                         const unsigned* thr, const float* eps2, bool sym, int grid,
                          const TileList& tl, hipStream_t st) {
   constexpr int FT = 4;
   FilterParams P;
@@ -993,24 +1064,22 @@ hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_r
   P.n_fit = n_fit;
   P.ref_pairs = ref_tiles / kRefTilesPerWG;
   P.fit_blocks = fit_tiles / FT;
-  P.phases = phases;
   P.thr = thr;
   P.eps2 = eps2;
   P.flags = tl.flags;
   P.ctrl = tl.ctrl;
-  if (ref_tiles % kRefTilesPerWG || fit_tiles % FT || phases < 1 || grid < 8 || (grid & 7))
+  if (ref_tiles % kRefTilesPerWG || fit_tiles % FT || grid < 8 || (grid & 7))
     return hipErrorInvalidValue;
   const int64_t vec = ((int64_t)P.fit_blocks * P.ref_pairs + 15) / 16;
   hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((vec + 255) / 256)), dim3(256), 0, st,
                      reinterpret_cast<uint4*>(tl.flags), vec, tl.ctrl);
-  const int sample = (P.fit_blocks + kSampleEvery - 1) / kSampleEvery;
-  for (int part = 0; part < 2; ++part) {
-    const int blocks = part == 0 ? sample : P.fit_blocks - sample;
-    if (blocks <= 0) break;
+  // The sample costs two launches: from 64 blocks on.  Phases so that every
+  // workgroup gets about four items, of eight tiles or more.
+  for (int part = P.fit_blocks >= 64 ? 0 : 2; part < 3; part += part == 1 ? 2 : 1) {
+    const int blocks = part_blocks(P.fit_blocks, part);
     P.part = part;
-    // the sample is a sixteenth of the blocks: split its rows further, so
-    // that its items still fill the grid evenly
-    P.phases = part == 0 ? std::min(P.ref_pairs, phases * 8) : phases;
+    P.phases = 4;
+    while (P.phases * blocks < 4 * grid && P.phases * 16 <= P.ref_pairs) P.phases *= 2;
     if (sh.gps == 1) {
       if (sym)
         hipLaunchKernelGGL((filter_kernel<1, true>), dim3(grid), dim3(512), 0, st, P);
@@ -1037,6 +1106,32 @@ hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, con
   return hipGetLastError();
 }
 
+hipError_t launch_stride_list(int ref_tiles, int stride, const TileList& tl, hipStream_t st) {
+  if (stride < 1 || !tl.shared) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(stride_list_kernel, dim3(1), dim3(256), 0, st, ref_tiles / kRefTilesPerWG,
+                     stride, tl.list, tl.count);
+  return hipGetLastError();
+}
+
+hipError_t launch_fill_near(unsigned long long* near, int64_t n, hipStream_t st) {
+  hipLaunchKernelGGL(fill_near_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, near, n);
+  return hipGetLastError();
+}
+
+hipError_t launch_near_keys(const unsigned long long* near, int64_t n, int phases, unsigned* keys,
+                            int* rows, hipStream_t st) {
+  hipLaunchKernelGGL(near_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, near, n,
+                     phases, keys, rows);
+  return hipGetLastError();
+}
+
+hipError_t launch_rank_sort(const unsigned* keys, int* order, int64_t n, hipStream_t st) {
+  if (n < 1 || n > kRankSortMax) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(rank_sort_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, st, keys,
+                     (int)n, order);
+  return hipGetLastError();
+}
+
 size_t sort_order_scratch(int64_t n) {
   size_t temp = 0;
   (void)hipcub::DeviceRadixSort::SortPairs<unsigned, int>(nullptr, temp, nullptr, nullptr, nullptr,
@@ -1047,11 +1142,13 @@ size_t sort_order_scratch(int64_t n) {
 hipError_t launch_sort_order(const int* leaders, int* rank, int ncells, unsigned* keys,
                              unsigned* keys_out, const int* rows, int* order, int64_t n, void* temp,
                              size_t temp_bytes, hipStream_t st) {
-  if (ncells < 1) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(cell_rank_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, st,
-                     leaders, ncells, rank);
-  hipLaunchKernelGGL(rank_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rank,
-                     ncells, n, keys);
+  if (leaders) {
+    if (ncells < 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(cell_rank_kernel, dim3((unsigned)((ncells + 255) / 256)), dim3(256), 0, st,
+                       leaders, ncells, rank);
+    hipLaunchKernelGGL(rank_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rank,
+                       ncells, n, keys);
+  }
   return hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, keys, keys_out, rows, order, (int)n, 0,
                                             32, st);
 }

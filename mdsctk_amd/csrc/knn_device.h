@@ -140,6 +140,17 @@ constexpr int kFilterSamples = 64;
 // Fit tiles per filter block, and the smallest self query that takes it.
 constexpr int kFilterFitTiles = 4;
 constexpr int64_t kFilterMinFrames = 4096;
+// Cross queries: resident frames (and frames x atoms) from which the set is
+// ordered, query frames in all from which that is worth it, and the smallest
+// query that takes the ordered form.  Measured at 100000 x 500 resident
+// frames: ordering takes 4.6 ms and saves 3.8 ms per 4096 query frames, so it
+// is even after about 5000 frames, whatever the size of the set (both grow
+// with it); a query of one or two fit blocks would spend the saving on the
+// extra launches.
+constexpr int64_t kCrossMinRef = 8192;
+constexpr int64_t kCrossMinWork = 1 << 22;
+constexpr int64_t kCrossMinSeen = 8192;
+constexpr int64_t kCrossMinFit = 256;
 // Cells the rows are sorted into (13 bits of the sort key, above 19 bits of
 // the distance).
 constexpr int kFilterMaxCells = 8000;
@@ -183,6 +194,7 @@ struct TileList {
   int* list = nullptr;
   int* count = nullptr;
   int* ctrl = nullptr;
+  bool shared = false;  // one list for every block
 };
 
 // Launchers (all asynchronous on `st`).
@@ -199,11 +211,22 @@ hipError_t launch_filter_prep(const DevFrames& f, const DevWeights& w, const Fil
 // the reference frame's), into tl.
 hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_ref, int64_t n_fit,
                          int ref_tiles, int fit_tiles, const FilterShape& sh, const FilterMean* mc,
-                         const unsigned* thr, const float* eps2, bool sym, int phases, int grid,
+                         const unsigned* thr, const float* eps2, bool sym, int grid,
                          const TileList& tl, hipStream_t st);
 // Each fit block of ft tiles against the `width` reference pairs around it.
 hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, const TileList& tl,
                             hipStream_t st);
+// Every stride-th reference pair, as a list shared by every block.
+hipError_t launch_stride_list(int ref_tiles, int stride, const TileList& tl, hipStream_t st);
+// The resident set's order for cross queries, from each frame's nearest
+// landmark (near: launch_contract): keys[q] = cell and distance, rows[q] = q.
+hipError_t launch_fill_near(unsigned long long* near, int64_t n, hipStream_t st);
+hipError_t launch_near_keys(const unsigned long long* near, int64_t n, int phases, unsigned* keys,
+                            int* rows, hipStream_t st);
+// order = rows sorted by key (stable); the rank form takes up to
+// kRankSortMax rows and allocates and clears nothing (it may be captured).
+constexpr int64_t kRankSortMax = 16384;
+hipError_t launch_rank_sort(const unsigned* keys, int* order, int64_t n, hipStream_t st);
 // order = rows sorted by key (stable), the cells of the keys first put in the
 // order of their leaders (rank: ncells ints of scratch).
 size_t sort_order_scratch(int64_t n);
@@ -238,12 +261,14 @@ hipError_t launch_eps(const DevFrames& fit, const DevFrames& ref, double kappa, 
 // frame's shared threshold L.thr.  ph_run < ref_phases walks phases
 // 0..ph_run-1 only (every ref_phases-th reference tile pair: the landmark
 // pass); 0 = all.  tiles: only the listed reference pairs of each block of
-// kFilterFitTiles fit tiles, dealt out over the phases.
+// kFilterFitTiles fit tiles, dealt out over the phases.  near: no lists, only
+// each fit frame's smallest (key << 32 | reference) there (atomic minimum).
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st,
                            const Mirror* mirror = nullptr, int ph_run = 0,
-                           const TileList* tiles = nullptr);
+                           const TileList* tiles = nullptr,
+                           unsigned long long* near = nullptr);
 // The window of a symmetric self query (fit: the reference set's query
 // view): eps2[r] = 2 kappa max(G~q[r] + max G~ref, G~ref[r] + max G~q);
 // *gmax_q receives max G~q.
@@ -276,15 +301,16 @@ hipError_t launch_scatter_rows(const double* sd, const int* si, const int* rows,
                                int k_out, double* dd, int* di, hipStream_t st);
 // order: the query rows in the order the merge workgroups take them
 // (nullptr: 0..n_fit-1).  mirror: a symmetric self query's second list per
-// row (nullptr: none).  perm (replaces order): the lists, mirrored lists and
-// eps2 were built over the frames in the order perm (list row i is frame
-// perm[i], entry index j frame perm[j]); ref/fit and the outputs and
-// fallback flags use the original indices.
+// row (nullptr: none).  perm (replaces order) and ref_perm: the lists,
+// mirrored lists and eps2 were built over the frames in those orders (list
+// row i is frame perm[i], entry index j reference ref_perm[j]); ref/fit and
+// the outputs and fallback flags use the original indices.
 hipError_t launch_merge(const DevFrames& ref, const DevFrames& fit, const DevWeights& w,
                         const Lists& L, const float* eps2, int k1, int k_out, int rank_off,
                         bool nofit, double* out_dist, int* out_idx, int* fallback,
                         int* n_cand, const int* order, hipStream_t st,
-                        const Mirror* mirror = nullptr, const int* perm = nullptr);
+                        const Mirror* mirror = nullptr, const int* perm = nullptr,
+                        const int* ref_perm = nullptr);
 // dst[i] = the float bits src[perm[i]] raised by add[i] (and one unit in the
 // last place): the shared thresholds of a landmark pass moved to the
 // permuted order, widened by the permuted frames' window.

@@ -596,10 +596,13 @@ struct ContractParams {
   int* mcnt;
   float* movf;
   int mcap;
-  // The reference pairs to walk, [blocks of kFilterFitTiles fit tiles][ref_pairs]
-  // in ascending order, and how many per block (null: all).
+  // The reference pairs to walk, in ascending order, and how many: per block
+  // of kFilterFitTiles fit tiles (tblock 1, rows of ref_pairs entries) or the
+  // same for every block (tblock 0).  Null: all.
   const int* tlist;
   const int* tcount;
+  int tblock;
+  unsigned long long* near;  // kOutNear: [n_fit] key bits << 32 | reference
 };
 
 // What the contraction's epilogue produces.
@@ -613,6 +616,7 @@ constexpr int kOutDebug = 1;  // every score in FP64 (dbg, n_fit x n_ref)
 // when it lies below that frame's shared threshold.  No score matrix is
 // written.
 constexpr int kOutSym = 2;
+constexpr int kOutNear = 3;  // each fit frame's nearest reference (key, index) only
 
 // One K-group of MFMA work for a wave: acc[c*3+d] += A_c * B_d^T over the
 // group's atoms, reading the wave's fragments from LDS.  For the split forms
@@ -1016,7 +1020,7 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     const int ph = item - fb * P.ph_run;
     // Tile t of the item is reference pair ph + t R, or that entry of the
     // block's tile list.
-    const int lb = fb * FT / kFilterFitTiles;
+    const int lb = P.tblock * (fb * FT / kFilterFitTiles);
     const int* const tlist = P.tlist ? P.tlist + (int64_t)lb * P.ref_pairs + ph : nullptr;
     const int n_pairs = P.tlist ? P.tcount[lb] : P.ref_pairs;
     const int n_tiles = (n_pairs - ph + P.phases - 1) / P.phases;
@@ -1049,6 +1053,7 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     const double gf = P.fGt[fit_idx];
     const float e2 = (fvalid && P.eps2) ? P.eps2[fit_idx] : 0.f;
     int cnt = 0;
+    unsigned near_idx = 0;  // kOutNear: the reference whose key is thr
     float thr = INFINITY, ovf = INFINITY;
 
     // Stage s of this item is K-group g = s % ngs of tile t = t0 + s / ngs.  Wave
@@ -1222,6 +1227,13 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
             mir = mirror && s <= (double)tr;
           }
         }
+        if constexpr (MODE == kOutNear) {
+          if (own && key < thr) {
+            thr = key;
+            near_idx = (unsigned)ref_idx;
+          }
+          continue;
+        }
         if (own) {
           // The compaction keeps cnt <= cap - 16 between tiles, so the guard
           // never drops; if it did, ovf would send the row to the exact path.
@@ -1239,7 +1251,7 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
                           (unsigned)fit_idx, lane);
         }
       }
-      if constexpr (MODE != kOutDebug) {
+      if constexpr (MODE == kOutLists || MODE == kOutSym) {
       const float thr_before = thr;
       compact_lists<PER>(P.ent, my_base, cnt, thr, ovf, e2, P.k1, P.cap, fvalid);
       thr = fminf(thr, __shfl_xor(thr, 32));
@@ -1248,7 +1260,10 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
       p_cur = p_next;
       if (t + 2 < n_tiles) p_next = pair_of(t + 2);
     }
-    if (fvalid && MODE != kOutDebug) {
+    if constexpr (MODE == kOutNear) {
+      if (fvalid && thr < INFINITY)
+        atomicMin(&P.near[fit_idx], ((unsigned long long)__float_as_uint(thr) << 32) | near_idx);
+    } else if (fvalid && MODE != kOutDebug) {
       P.cnt[hdr] = cnt;
       P.ovf[hdr] = ovf;
     }
@@ -1390,10 +1405,11 @@ struct MergeParams {
   PairSource src;
   const int* order;  // query rows in processing order (nullptr: 0..n_fit-1)
   // the lists were built over a permutation of the frames (the symmetric
-  // self query in landmark order): list row i and list entry index j are
-  // frames perm[i] and perm[j]; the frames' data and the outputs use the
-  // original indices.  Replaces order (the lists are in processing order).
+  // self query in landmark order, a cross query in its reference set's
+  // order): list row i and list entry index j are frames perm[i] and
+  // ref_perm[j]; the frames' data and the outputs use the original indices.  Replaces order (the lists are in processing order).
   const int* perm;
+  const int* ref_perm;  // the entries' permutation
   double W, out_scale;
   const uint2* ent;
   const int* cnt;
@@ -1469,7 +1485,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   const float* ovf = P.ovf + qi * P.nl;
   const int mc = P.ment ? min(P.mcnt[qi], P.mcap) : 0;
   const uint2* ment = P.ment ? P.ment + qi * (int64_t)P.mcap : nullptr;
-  auto frame_of = [&](unsigned j) -> int { return P.perm ? P.perm[j] : (int)j; };
+  auto frame_of = [&](unsigned j) -> int { return P.ref_perm ? P.ref_perm[j] : (int)j; };
   // f(entry) for every entry of the row's lists, and the whole workgroup
   // over the mirrored list.  Few lists: waves over the lists, lanes over
   // entries (coalesced).  Many lists (a small query batch spread over many
@@ -2321,7 +2337,7 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st, const Mirror* mirror,
-                           int ph_run, const TileList* tiles) {
+                           int ph_run, const TileList* tiles, unsigned long long* near) {
   ContractParams P;
   P.rop = ref.op;
   P.fop = fit.op;
@@ -2350,7 +2366,11 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
   P.mcap = mirror ? mirror->cap : 0;
   P.tlist = tiles ? tiles->list : nullptr;
   P.tcount = tiles ? tiles->count : nullptr;
-  if (tiles && (!tiles->list || !tiles->count || ph_run || fit.n_tiles % kFilterFitTiles))
+  P.tblock = tiles && tiles->shared ? 0 : 1;
+  P.near = near;
+  if (near && (nofit || mirror || tiles || dbg_scores)) return hipErrorInvalidValue;
+  if (tiles && (!tiles->list || !tiles->count || ph_run || fit.n_tiles % kFilterFitTiles ||
+                (mirror && tiles->shared)))
     return hipErrorInvalidValue;
   if (P.ph_run > ref_phases || ref_phases < 1) return hipErrorInvalidValue;
   // the split forms' pipelined K-loop walks K-groups four at a time
@@ -2376,6 +2396,8 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
   do {                                              \
     if (dbg_scores)                                 \
       MDSCTK_CONTRACT_TR(PR, 4, FT, kOutDebug);     \
+    else if (near)                                  \
+      MDSCTK_CONTRACT(PR, 4, FT, kOutNear, false);  \
     else if (mirror && L.cap == 256)                \
       MDSCTK_CONTRACT_TR(PR, 4, FT, kOutSym);       \
     else if (mirror && L.cap == 512)                \
@@ -2427,7 +2449,8 @@ static PairSource pair_source(const DevFrames& ref, const DevFrames& fit, const 
 hipError_t launch_merge(const DevFrames& ref, const DevFrames& fit, const DevWeights& w,
                         const Lists& L, const float* eps2, int k1, int k_out, int rank_off,
                         bool nofit, double* out_dist, int* out_idx, int* fallback, int* n_cand,
-                        const int* order, hipStream_t st, const Mirror* mirror, const int* perm) {
+                        const int* order, hipStream_t st, const Mirror* mirror, const int* perm,
+                        const int* ref_perm) {
   MergeParams P;
   P.src = pair_source(ref, fit, w);
   P.W = w.W;
@@ -2452,6 +2475,7 @@ hipError_t launch_merge(const DevFrames& ref, const DevFrames& fit, const DevWei
   P.n_cand = n_cand;
   P.order = order;
   P.perm = perm;
+  P.ref_perm = ref_perm;
   // k1 <= 256: windows of up to 1024 candidates (C3: 184 per query), half
   // the candidate LDS of the general instance
   const bool stage = w.metric == kMetricRMSD && ref.natoms <= kMergeStageAtoms;

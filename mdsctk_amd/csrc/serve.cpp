@@ -43,12 +43,14 @@ struct HipSlot {
   bool all_exact = false;  // the batch took the exact rows, not the contraction
   size_t h_elems = 0, h_rows = 0;
   hipEvent_t done = nullptr;
-  hipGraphExec_t exec = nullptr;  // the slot's batch kernels, updated per batch
+  // the slot's batch kernels, updated per batch: [0] every tile, [1] the
+  // ordered form (another sequence of kernels)
+  hipGraphExec_t exec[2] = {nullptr, nullptr};
   // the captured graph exec was last instantiated or updated from; kept
   // until a later capture has replaced it in exec (and that exec has been
   // launched), so nothing the executable may refer to is released while it
   // can still run
-  hipGraph_t graph = nullptr;
+  hipGraph_t graph[2] = {nullptr, nullptr};
   // shape the workspace was last sized for
   int64_t sized_limit = 0;
   int sized_k_out = -1, sized_k1 = -1;
@@ -89,8 +91,10 @@ class HipServeDevice {
   void release() {
     for (auto& sl : slots_) {
       if (sl.s.st) (void)hipStreamSynchronize(sl.s.st);
-      if (sl.exec) (void)hipGraphExecDestroy(sl.exec);
-      if (sl.graph) (void)hipGraphDestroy(sl.graph);
+      for (auto& e : sl.exec)
+        if (e) (void)hipGraphExecDestroy(e);
+      for (auto& g : sl.graph)
+        if (g) (void)hipGraphDestroy(g);
       slot_release(c_, sl.s);
       if (sl.done) (void)hipEventDestroy(sl.done);
       free_host(sl);
@@ -158,10 +162,16 @@ class HipServeDevice {
     }
     sl.all_exact = !fused;
     if (fused) {
+      if (!q.nofit && (rc = ensure_ordered(c_, s, b.n))) return rc;
       FusedPlan plan;
       if ((rc = plan_fused(c_, s, q, &plan))) return rc;
-      if (c_->serve_share_cus && slots_.size() > 1)
+      // beyond the rank sort the ordering takes a library sort, which is not
+      // for a captured graph
+      if (b.n > kRankSortMax) plan.x.on = false;
+      if (c_->serve_share_cus && slots_.size() > 1) {
         plan.grid = std::max(8, (plan.grid / (int)slots_.size()) & ~7);
+        plan.x.filter_grid = std::max(8, (plan.x.filter_grid / (int)slots_.size()) & ~7);
+      }
       if (c_->serve_graphs) {
         if ((rc = replay_graph(sl, q, plan))) return rc;
       } else {
@@ -333,6 +343,8 @@ class HipServeDevice {
   // then never reads released memory).
   int replay_graph(HipSlot& sl, const QueryShape& q, const FusedPlan& plan) {
     Slot& s = sl.s;
+    hipGraphExec_t& exec = sl.exec[plan.x.on];
+    hipGraph_t& graph = sl.graph[plan.x.on];
     hipError_t e = hipStreamBeginCapture(s.st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(c_, e, "serve: graph capture");
     int rc = prep_slot(c_, s, q.nofit);
@@ -343,31 +355,31 @@ class HipServeDevice {
       if (g) (void)hipGraphDestroy(g);
       return rc ? rc : hip_fail(c_, e, "serve: graph capture");
     }
-    if (sl.exec) {
+    if (exec) {
       hipGraphNode_t err_node = nullptr;
       hipGraphExecUpdateResult res;
-      if (hipGraphExecUpdate(sl.exec, g, &err_node, &res) != hipSuccess ||
+      if (hipGraphExecUpdate(exec, g, &err_node, &res) != hipSuccess ||
           res != hipGraphExecUpdateSuccess) {
         (void)hipGetLastError();
-        (void)hipGraphExecDestroy(sl.exec);
-        sl.exec = nullptr;
+        (void)hipGraphExecDestroy(exec);
+        exec = nullptr;
       }
     }
-    if (!sl.exec) {
-      e = hipGraphInstantiate(&sl.exec, g, nullptr, nullptr, 0);
+    if (!exec) {
+      e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
       if (e != hipSuccess) {
-        sl.exec = nullptr;
+        exec = nullptr;
         (void)hipGraphDestroy(g);
         return hip_fail(c_, e, "serve: graph instantiate");
       }
       ++graph_builds_;
     }
-    e = hipGraphLaunch(sl.exec, s.st);
+    e = hipGraphLaunch(exec, s.st);
     // exec now holds g's parameters and has been launched: the graph it
     // replaced can go (the slot's stream orders every earlier launch of
     // this exec before this one)
-    if (sl.graph) (void)hipGraphDestroy(sl.graph);
-    sl.graph = g;
+    if (graph) (void)hipGraphDestroy(graph);
+    graph = g;
     if (e != hipSuccess) return hip_fail(c_, e, "serve: graph launch");
     ++graph_launches_;
     return 0;

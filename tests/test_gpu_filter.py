@@ -1,10 +1,13 @@
-"""The tile filter of a fitted self query (filter_kernels.hip): from 4096
-frames on, a proven bound decides which tiles of the block triangle are
+"""The tile filter of fitted queries (filter_kernels.hip).  Self queries: from
+4096 frames on, a proven bound decides which tiles of the block triangle are
 contracted at all.  Outputs must equal the candidate-list path's bit for bit
 and the FP64 oracle's, at the edges of the filter's layout: one and two
 segments (384 atoms), one and two K-groups per stage (309), slots exactly
 full and one over (52, 53, 116, 117), frames of 1 to 3 atoms, ragged frame
-counts, and sets whose tiles all stay (a single basin with a wide k)."""
+counts, and sets whose tiles all stay (a single basin with a wide k).  Cross
+queries: once a context has seen enough query frames it orders the resident
+set, and later queries (synchronous and served) walk the filtered tiles; they
+must return what the first ones did."""
 import numpy as np
 import pytest
 
@@ -73,3 +76,44 @@ def test_filtered_self_query_scales(scale):
     d2, i2 = _rows(frames * power, w, 8, "bf16", 1)
     np.testing.assert_array_equal(i, i2)
     np.testing.assert_allclose(d2, d * float(power), rtol=1e-9)
+
+
+@pytest.mark.parametrize("prec", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("gen,natoms,n_ref,n_fit,k", [("states", 470, 9001, 2100, 20),
+                                                      ("basin", 513, 8192, 2085, 40),
+                                                      ("loose", 600, 8300, 2300, 5)])
+def test_ordered_cross_query(gen, natoms, n_ref, n_fit, k, prec):
+    n = n_ref + n_fit
+    if gen == "states":
+        x = synth.metastable_trajectory(n, natoms, 3, n_centres=15)
+    elif gen == "basin":
+        x = synth.trajectory(n, natoms, 4)
+    else:
+        rng = np.random.default_rng(6)
+        x = np.stack([synth.random_walk(natoms, rng) for _ in range(n)]).astype(np.float32)
+    ref, fit = x[:n_ref], x[n_ref:]
+    w = synth.masses(natoms, "random", 2)
+    with knn.KnnContext(0, prec) as ctx:
+        ctx.set_reference(ref, w)
+        d0, i0 = ctx.query(fit, k)
+        held = ctx.stats()["device_bytes"]
+        for _ in range(4):
+            d, i = ctx.query(fit, k)
+            np.testing.assert_array_equal(i, i0)
+            np.testing.assert_array_equal(d, d0)
+        # the ordered copy of the resident set now exists
+        assert ctx.stats()["device_bytes"] > held + 12 * n_ref * natoms
+        for m in (255, 256, 257, 1000):  # either side of the smallest ordered query
+            d, i = ctx.query(fit[:m], k)
+            np.testing.assert_array_equal(i, i0[:m])
+            np.testing.assert_array_equal(d, d0[:m])
+        reqs = [ctx.submit(fit[a:b], k) for a, b in ((0, 1), (1, 900), (900, n_fit))]
+        for r, (a, b) in zip(reqs, ((0, 1), (1, 900), (900, n_fit))):
+            ctx.wait(r)
+            np.testing.assert_array_equal(r.idx, i0[a:b])
+            np.testing.assert_array_equal(r.dist, d0[a:b])
+        d, i = ctx.query(fit, k, knn.KNN_KEEP_RANK0)
+        np.testing.assert_array_equal(i[:, 1:], i0[:, :-1])
+    rows = np.arange(0, n_fit, n_fit // 5)
+    d_o, i_o = oracle.knn_exact(ref, fit[rows], w, k)
+    check_knn(ref, fit[rows], w, d0[rows], i0[rows], d_o, i_o)
