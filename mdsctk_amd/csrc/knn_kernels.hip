@@ -1270,6 +1270,37 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
   }
 }
 
+// The bin of a 256-bin histogram that holds the rank-th (0-based) of its
+// counts, and the rank within the bin, for every thread of a 256-thread
+// workgroup: an inclusive scan over lanes and waves.  (One thread walking the
+// bins took about 7 us a pass, most of the merge and of the landmark caps.)
+__device__ __forceinline__ void pick_bin(const unsigned* hist, int rank, int* bin, int* rest) {
+  __shared__ unsigned wave_total[4];
+  __shared__ int s_bin, s_rest;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const unsigned h = hist[tid];
+  unsigned inc = h;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned t = __shfl_up(inc, o);
+    if (lane >= o) inc += t;
+  }
+  if (lane == 63) wave_total[wave] = inc;
+  if (tid == 0) {  // no bin reaches the rank: the last one
+    s_bin = 255;
+    s_rest = 0;
+  }
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) inc += wave_total[w];
+  if (inc - h <= (unsigned)rank && (unsigned)rank < inc) {
+    s_bin = tid;
+    s_rest = rank - (int)(inc - h);
+  }
+  __syncthreads();
+  *bin = s_bin;
+  *rest = s_rest;
+}
+
 // ---------------------------------------------------------------------------
 // exact FP64 score of one pair, by a 16-lane group (lanes over atoms).
 
@@ -1277,9 +1308,23 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
 // centred coordinates w_i (b_i - c_b) in FP64 (3 per atom).
 extern __shared__ double qw_stage[];
 
+// v of the lane `n` places round the 16-lane row (one DPP move per half).
+template <int N>
+__device__ __forceinline__ double row_rotate(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x120 + N, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x120 + N, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// The sum over a 16-lane group, in every lane: the butterfly over lanes 8, 4,
+// 2 and 1 apart (after a step the values repeat with that period, so a
+// rotation by it reads the same value as the exchange).
 __device__ __forceinline__ double group_sum16(double v) {
-#pragma unroll
-  for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  v += row_rotate<8>(v);
+  v += row_rotate<4>(v);
+  v += row_rotate<2>(v);
+  v += row_rotate<1>(v);
   return v;
 }
 
@@ -1289,22 +1334,21 @@ __device__ __forceinline__ double weighted_centred(float x, double c, double w) 
   return w * ((double)x - c);
 }
 
-// Exact FP64 score of the pair (reference frame a, query frame b) by the
+// The cross-covariance of the pair (reference frame a, query frame b) by the
 // 16 lanes of a group, lane j of the group taking atoms j, j + 16, ...:
 //   S = sum_i a_i (w_i (b_i - c_b))^T
 // with the reference frame uncentred (sum_i w_i (b_i - c_b) = 0, so S is
-// the weighted cross-covariance of the centred frames), then lambda_max of
-// the key matrix and s = G_a + G_b - 2 lambda_max.  Every lane of the group
-// returns the same value.  QS: the query's weighted centred coordinates
-// are in qw_stage (the pointer b is then unused).
+// the weighted cross-covariance of the centred frames).  Every lane of the
+// group gets the same S.  QS: the query's weighted centred coordinates are in
+// qw_stage (the pointer b is then unused).  Every kernel that scores pairs
+// exactly adds in this order, so that a pair has the same score in all.
 template <bool QS>
-__device__ __forceinline__ double group_rmsd_score(const float* __restrict__ a, double ga,
-                                                   const float* __restrict__ b,
-                                                   const double* __restrict__ cb, double gb,
-                                                   const float* __restrict__ w, int natoms,
-                                                   bool nofit) {
+__device__ __forceinline__ void group_cross(const float* __restrict__ a,
+                                            const float* __restrict__ b,
+                                            const double* __restrict__ cb,
+                                            const float* __restrict__ w, int natoms,
+                                            double (&S)[9]) {
   const int sub = threadIdx.x & 15;
-  double S[9];
 #pragma unroll
   for (int i = 0; i < 9; ++i) S[i] = 0.0;
   const double cb0 = cb[0], cb1 = cb[1], cb2 = cb[2];
@@ -1332,6 +1376,10 @@ __device__ __forceinline__ double group_rmsd_score(const float* __restrict__ a, 
   }
 #pragma unroll
   for (int i = 0; i < 9; ++i) S[i] = group_sum16(S[i]);
+}
+
+// The exact score of a pair from its cross-covariance and G terms.
+__device__ __forceinline__ double cross_score(const double* S, double ga, double gb, bool nofit) {
   const double lam = nofit ? (S[0] + S[4] + S[8]) : qcp_lambda_exact(S, ga, gb);
   return fmax(ga + gb - 2.0 * lam, 0.0);
 }
@@ -1382,15 +1430,6 @@ struct PairSource {
   const double* f64;
   const double* faux;
 };
-
-// RMSD: the exact score of reference r against query q by a 16-lane group.
-template <bool QS = false>
-__device__ __forceinline__ double group_pair_score(const PairSource& P, int64_t r, int64_t q,
-                                                   bool nofit) {
-  return group_rmsd_score<QS>(P.rxyz + r * (int64_t)P.natoms * 3, P.rG[r],
-                              P.fxyz + q * (int64_t)P.natoms * 3, P.fcen + q * 3, P.fG[q], P.w,
-                              P.natoms, nofit);
-}
 
 // Data vectors: the exact score of reference r against query q by a wave.
 __device__ __forceinline__ double wave_data_pair_score(const PairSource& P, int64_t r, int64_t q) {
@@ -1452,6 +1491,8 @@ __device__ void block_bitonic_sort(double* s, int* idx, int n_pow2) {
 
 // Keys just above a row's cut that the merge re-scores to check the window.
 constexpr int kMergeGuard = 32;
+// Pairs whose cross-covariances the merge holds in LDS at a time.
+constexpr int kMergeChunk = 128;
 
 // STAGE: for frames of up to kMergeStageAtoms atoms the query frame's
 // weighted centred coordinates are formed once, in FP64 in LDS (24 KB at
@@ -1468,8 +1509,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   const int64_t q = P.perm ? P.perm[qi] : qi;  // the frame: data and output row
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   __shared__ unsigned hist[256];
-  __shared__ unsigned s_prefix;
-  __shared__ int s_kk, s_nc, s_flag, s_total;
+  __shared__ int s_nc, s_flag, s_total;
   __shared__ int cand_idx[CAND];
   __shared__ double cand_s[CAND];
   __shared__ float cand_key[CAND];
@@ -1479,6 +1519,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   __shared__ float guard_key[kMergeGuard];
   __shared__ double guard_s[kMergeGuard];
   __shared__ int s_ng;
+  __shared__ double pair_S[kMergeChunk * 9];
 
   const int* cnt = P.cnt + qi * P.nl;
   const uint2* ent = P.ent + qi * P.nl * (int64_t)P.cap;
@@ -1541,19 +1582,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
       if ((k & mhi) == (prefix & mhi)) atomicAdd(&hist[(k >> shift) & 255u], 1u);
     });
     __syncthreads();
-    if (tid == 0) {
-      unsigned cum = 0;
-      int b = 0;
-      for (; b < 255; ++b) {
-        if (cum + hist[b] > (unsigned)kk) break;
-        cum += hist[b];
-      }
-      s_prefix = prefix | ((unsigned)b << shift);
-      s_kk = kk - (int)cum;
-    }
-    __syncthreads();
-    prefix = s_prefix;
-    kk = s_kk;
+    int b;
+    pick_bin(hist, kk, &b, &kk);
+    prefix |= (unsigned)b << shift;
   }
   const float tau = __uint_as_float(prefix);
   const float e2q = P.eps2[qi];
@@ -1612,15 +1643,33 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
       guard_s[c - nc] = s;
   };
   if (P.src.metric == kMetricRMSD) {
-    // four pairs per wave, one per 16-lane group
-    const int grp = lane >> 4;
-    for (int c0 = 4 * wave; c0 < nc + ng; c0 += 16) {
-      const int c = c0 + grp;
-      if (c < nc + ng) {
-        const int r = c < nc ? cand_idx[c] : guard_idx[c - nc];
-        const double s = group_pair_score<STAGE>(P.src, r, q, P.nofit);
-        if ((lane & 15) == 0) put(c, s);
+    // kMergeChunk pairs at a time: first their cross-covariances, a pair per
+    // 16-lane group, into LDS; then their QCPs, a pair per thread.  (With each
+    // group running its own pair's QCP in all 16 lanes, the QCP took most of
+    // the kernel for frames of a few hundred atoms.)
+    const int total = nc + ng;
+    const double gq = P.src.fG[q];
+    for (int c0 = 0; c0 < total; c0 += kMergeChunk) {
+      const int m = min(kMergeChunk, total - c0);
+      for (int j = tid >> 4; j < m; j += 16) {
+        const int c = c0 + j;
+        const int64_t r = c < nc ? cand_idx[c] : guard_idx[c - nc];
+        double S[9];
+        group_cross<STAGE>(P.src.rxyz + r * (int64_t)P.src.natoms * 3,
+                           P.src.fxyz + q * (int64_t)P.src.natoms * 3, P.src.fcen + q * 3, P.src.w,
+                           P.src.natoms, S);
+        if ((lane & 15) == 0) {
+#pragma unroll
+          for (int i = 0; i < 9; ++i) pair_S[j * 9 + i] = S[i];
+        }
       }
+      __syncthreads();
+      for (int j = tid; j < m; j += 256) {
+        const int c = c0 + j;
+        const int64_t r = c < nc ? cand_idx[c] : guard_idx[c - nc];
+        put(c, cross_score(pair_S + j * 9, P.src.rG[r], gq, P.nofit));
+      }
+      __syncthreads();
     }
   } else {
     for (int c = wave; c < nc + ng; c += 4) {
@@ -1688,8 +1737,7 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
   const int64_t q = blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   __shared__ unsigned hist[256];
-  __shared__ unsigned s_prefix;
-  __shared__ int s_kk, s_total;
+  __shared__ int s_total;
   __shared__ unsigned long long s_best, s_cell;
   __shared__ int s_leader;
   const int* c = cnt + q * nl;
@@ -1746,19 +1794,9 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
         if ((x.x & mhi) == (prefix & mhi)) atomicAdd(&hist[(x.x >> shift) & 255u], 1u);
       });
       __syncthreads();
-      if (tid == 0) {
-        unsigned cum = 0;
-        int b = 0;
-        for (; b < 255; ++b) {
-          if (cum + hist[b] > (unsigned)kk) break;
-          cum += hist[b];
-        }
-        s_prefix = prefix | ((unsigned)b << shift);
-        s_kk = kk - (int)cum;
-      }
-      __syncthreads();
-      prefix = s_prefix;
-      kk = s_kk;
+      int b;
+      pick_bin(hist, kk, &b, &kk);
+      prefix |= (unsigned)b << shift;
     }
     return prefix;
   };
@@ -1930,35 +1968,137 @@ struct ExactParams {
   int64_t out_ld;
 };
 
-constexpr int kExactRefsPerWG = 64;
+constexpr int kExactRefsPerWG = 32;  // a workgroup's references
+constexpr int kExactRows = 4;        // and query rows
+constexpr int kExactChunk = 256;     // atoms staged at a time (a multiple of 16)
 
-__global__ __launch_bounds__(256) void exact_rows_kernel(ExactParams P) {
+__device__ __forceinline__ void put_exact(const ExactParams& P, int64_t ri, int64_t q, int64_t r,
+                                          double s) {
+  if (P.out_full)
+    P.out_full[q * P.out_ld + r] = P.out_scale * sqrt(fmax(s, 0.0) / P.W);
+  else
+    P.srow[ri * P.n_ref + r] = s;
+}
+
+// v of the lane `X` apart (X = 4, 2 or 1) in the 16-lane row.
+template <int X>
+__device__ __forceinline__ double row_exchange(double v) {
+  const long long b = __double_as_longlong(v);
+  constexpr int kPattern = (X << 10) | 0x1f;  // lane ^ X
+  const int lo = __builtin_amdgcn_ds_swizzle((int)b, kPattern);
+  const int hi = __builtin_amdgcn_ds_swizzle((int)(b >> 32), kPattern);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Whole rows of exact scores: a workgroup takes 4 query rows against 32
+// references, a 16-lane group 2 references against the 4 rows.  The rows'
+// weighted centred coordinates are staged in LDS in FP64, so that an atom of
+// a reference is loaded and converted once for 4 rows and an atom of a row
+// read once for 2 references: 36 FMAs per 24-byte LDS read and 12-byte load
+// instead of 9 (with one pair per group every pair read both frames again).
+// The 8 cross-covariances are summed over the group by halving: each lane
+// keeps the pairs of its half, so that the sums land in different lanes and
+// every pair's QCP runs in two lanes instead of 16.  Sums are added in
+// group_cross's order.  501 rows against 20011 x 304 atoms: the
+// kernel 5.6 -> 2.4 ms (the FP64 FMAs alone are 0.7 ms).
+__global__ __launch_bounds__(256) void exact_rows_kernel(ExactParams P, int nrows) {
+  __shared__ double qs[kExactRows][3 * kExactChunk];
+  const int tid = threadIdx.x, lane = tid & 63, sub = lane & 15, grp = tid >> 4;
+  const int64_t ri0 = (int64_t)blockIdx.y * kExactRows;
+  const int64_t r0 = (int64_t)blockIdx.x * kExactRefsPerWG + grp;
+  const int natoms = P.src.natoms;
+  auto query = [&](int k) -> int64_t {  // the last row again past the end
+    const int64_t ri = min(ri0 + k, (int64_t)nrows - 1);
+    return P.rows ? P.rows[ri] : P.row0 + ri;
+  };
+  const F3* a3[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    a3[k] = reinterpret_cast<const F3*>(P.src.rxyz) + min(r0 + 16 * k, P.n_ref - 1) * natoms;
+  double S[8][9];
+#pragma unroll
+  for (int p = 0; p < 8; ++p)
+#pragma unroll
+    for (int i = 0; i < 9; ++i) S[p][i] = 0.0;
+  for (int c0 = 0; c0 < natoms; c0 += kExactChunk) {
+    const int m = min(kExactChunk, natoms - c0);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kExactRows; ++k) {
+      const int64_t q = query(k);
+      const F3* const b3 = reinterpret_cast<const F3*>(P.src.fxyz) + q * natoms + c0;
+      const double* const cb = P.src.fcen + q * 3;
+      for (int i = tid; i < m; i += 256) {
+        const F3 b = b3[i];
+        const double wi = (double)P.src.w[c0 + i];
+        qs[k][3 * i] = weighted_centred(b.x, cb[0], wi);
+        qs[k][3 * i + 1] = weighted_centred(b.y, cb[1], wi);
+        qs[k][3 * i + 2] = weighted_centred(b.z, cb[2], wi);
+      }
+    }
+    __syncthreads();
+#pragma unroll 2
+    for (int i = sub; i < m; i += 16) {
+      double a[2][3];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const F3 v = a3[k][c0 + i];
+        a[k][0] = (double)v.x;
+        a[k][1] = (double)v.y;
+        a[k][2] = (double)v.z;
+      }
+#pragma unroll
+      for (int k = 0; k < kExactRows; ++k) {
+        const double bx = qs[k][3 * i], by = qs[k][3 * i + 1], bz = qs[k][3 * i + 2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          double(&s)[9] = S[j * kExactRows + k];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            s[3 * c] = fma(a[j][c], bx, s[3 * c]);
+            s[3 * c + 1] = fma(a[j][c], by, s[3 * c + 1]);
+            s[3 * c + 2] = fma(a[j][c], bz, s[3 * c + 2]);
+          }
+        }
+      }
+    }
+  }
+  const bool b8 = sub & 8, b4 = sub & 4, b2 = sub & 2;
+  double v[9];
+#pragma unroll
+  for (int i = 0; i < 9; ++i) {
+    double h[4], g[2];
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      h[p] = (b8 ? S[p + 4][i] : S[p][i]) + row_rotate<8>(b8 ? S[p][i] : S[p + 4][i]);
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      g[p] = (b4 ? h[p + 2] : h[p]) + row_exchange<4>(b4 ? h[p] : h[p + 2]);
+    v[i] = (b2 ? g[1] : g[0]) + row_exchange<2>(b2 ? g[0] : g[1]);
+    v[i] += row_exchange<1>(v[i]);
+  }
+  // this lane's pair: reference r0 + 16 (b8), row 2 (b4) + (b2)
+  const int k = (b4 ? 2 : 0) + (b2 ? 1 : 0);
+  const int64_t r = r0 + (b8 ? 16 : 0), ri = ri0 + k;
+  if (r >= P.n_ref || ri >= nrows) return;
+  const int64_t q = query(k);
+  const double s = cross_score(v, P.src.rG[r], P.src.fG[q], P.nofit);
+  if (!(sub & 1)) put_exact(P, ri, q, r, s);
+}
+
+constexpr int kExactDataRefsPerWG = 64;
+
+// Data vectors: a pair per wave.
+__global__ __launch_bounds__(256) void exact_data_rows_kernel(ExactParams P) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t ri = blockIdx.y;
   const int64_t q = P.rows ? P.rows[ri] : P.row0 + ri;
-  const int64_t r0 = (int64_t)blockIdx.x * kExactRefsPerWG;
-  auto put = [&](int64_t r, double s) {
-    if (P.out_full)
-      P.out_full[q * P.out_ld + r] = P.out_scale * sqrt(fmax(s, 0.0) / P.W);
-    else
-      P.srow[ri * P.n_ref + r] = s;
-  };
-  if (P.src.metric == kMetricRMSD) {
-    // four pairs per wave, one per 16-lane group
-    const int grp = lane >> 4;
-    for (int j = 4 * wave + grp; j < kExactRefsPerWG; j += 16) {
-      const int64_t r = r0 + j;
-      if (r >= P.n_ref) break;
-      const double s = group_pair_score(P.src, r, q, P.nofit);
-      if ((lane & 15) == 0) put(r, s);
-    }
-  } else {
-    for (int j = wave; j < kExactRefsPerWG; j += 4) {
-      const int64_t r = r0 + j;
-      if (r >= P.n_ref) break;
-      const double s = wave_data_pair_score(P.src, r, q);
-      if (lane == 0) put(r, s);
-    }
+  const int64_t r0 = (int64_t)blockIdx.x * kExactDataRefsPerWG;
+  for (int j = wave; j < kExactDataRefsPerWG; j += 4) {
+    const int64_t r = r0 + j;
+    if (r >= P.n_ref) break;
+    const double s = wave_data_pair_score(P.src, r, q);
+    if (lane == 0) put_exact(P, ri, q, r, s);
   }
 }
 
@@ -1971,9 +2111,6 @@ __device__ void row_threshold(const double* __restrict__ s, int64_t n_ref, int k
                               unsigned long long* prefix_out, unsigned* ip_out) {
   const int tid = threadIdx.x;
   __shared__ unsigned hist[256];
-  __shared__ unsigned long long s_prefix;
-  __shared__ int s_kk;
-  __shared__ unsigned s_iprefix;
   unsigned long long prefix = 0;
   int kk = k1 - 1;
   for (int shift = 56; shift >= 0; shift -= 8) {
@@ -1985,19 +2122,9 @@ __device__ void row_threshold(const double* __restrict__ s, int64_t n_ref, int k
       if ((k & mhi) == (prefix & mhi)) atomicAdd(&hist[(k >> shift) & 255ull], 1u);
     }
     __syncthreads();
-    if (tid == 0) {
-      unsigned cum = 0;
-      int b = 0;
-      for (; b < 255; ++b) {
-        if (cum + hist[b] > (unsigned)kk) break;
-        cum += hist[b];
-      }
-      s_prefix = prefix | ((unsigned long long)b << shift);
-      s_kk = kk - (int)cum;
-    }
-    __syncthreads();
-    prefix = s_prefix;
-    kk = s_kk;
+    int b;
+    pick_bin(hist, kk, &b, &kk);
+    prefix |= (unsigned long long)b << shift;
   }
   // Among keys equal to tau take the kk+1 smallest indices: radix select on
   // the index.
@@ -2013,19 +2140,9 @@ __device__ void row_threshold(const double* __restrict__ s, int64_t n_ref, int k
       if ((k & mhi) == (ip & mhi)) atomicAdd(&hist[(k >> shift) & 255u], 1u);
     }
     __syncthreads();
-    if (tid == 0) {
-      unsigned cum = 0;
-      int b = 0;
-      for (; b < 255; ++b) {
-        if (cum + hist[b] > (unsigned)ik) break;
-        cum += hist[b];
-      }
-      s_iprefix = ip | ((unsigned)b << shift);
-      s_kk = ik - (int)cum;
-    }
-    __syncthreads();
-    ip = s_iprefix;
-    ik = s_kk;
+    int b;
+    pick_bin(hist, ik, &b, &ik);
+    ip |= (unsigned)b << shift;
   }
   *prefix_out = prefix;
   *ip_out = ip;
@@ -2580,8 +2697,14 @@ hipError_t launch_exact_rows(const DevFrames& ref, const DevFrames& fit, const D
     P.row0 = rows ? 0 : r0;
     P.srow = srow ? srow + (int64_t)r0 * ref.n : nullptr;
     P.out_full = out_full;
-    dim3 grid((unsigned)((ref.n + kExactRefsPerWG - 1) / kExactRefsPerWG), (unsigned)nr);
-    hipLaunchKernelGGL(exact_rows_kernel, grid, dim3(256), 0, st, P);
+    if (w.metric == kMetricRMSD) {
+      dim3 grid((unsigned)((ref.n + kExactRefsPerWG - 1) / kExactRefsPerWG),
+                (unsigned)((nr + kExactRows - 1) / kExactRows));
+      hipLaunchKernelGGL(exact_rows_kernel, grid, dim3(256), 0, st, P, nr);
+    } else {
+      dim3 grid((unsigned)((ref.n + kExactDataRefsPerWG - 1) / kExactDataRefsPerWG), (unsigned)nr);
+      hipLaunchKernelGGL(exact_data_rows_kernel, grid, dim3(256), 0, st, P);
+    }
   }
   return hipGetLastError();
 }
