@@ -570,21 +570,22 @@ int stage_input(mdsctk_knn_ctx* c, Slot& s, const void* in, bool on_device, int6
   return prep_slot(c, s, nofit);
 }
 
-int contract_grid(const mdsctk_knn_ctx* c) {
-  // workgroups resident at once: two 4-wave or one 8-wave per CU
-  const int ft = contract_fit_tiles(c->prec == kExact ? kFP32 : c->prec);
-  return std::max(8, (c->n_cu * (ft == 2 ? 2 : 1)) & ~7);
+int contract_grid(const mdsctk_knn_ctx* c, int ft) {
+  // workgroups resident at once: two 2- or 4-wave or one 8-wave per CU
+  return std::max(8, (c->n_cu * (ft <= 2 ? 2 : 1)) & ~7);
 }
 
-int fused_phases(const mdsctk_knn_ctx* c, int fit_tiles) {
-  const int ft = contract_fit_tiles(c->prec == kExact ? kFP32 : c->prec);
-  const int fit_blocks = std::max(1, fit_tiles / ft);
+int fused_phases(const mdsctk_knn_ctx* c, int64_t n_fit) {
+  const int ft = contract_fit_tiles(c->prec == kExact ? kFP32 : c->prec, n_fit);
+  const int fit_blocks = ft == 1 ? 1 : std::max(1, std::max(kTileAlign, padded_tiles(n_fit)) / ft);
   const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
-  const int grid = contract_grid(c);
+  const int grid = contract_grid(c, ft);
   int phases = c->forced_phases;
   if (phases <= 0) {
     // enough (fit block, phase) items to fill the grid, at least 8 phases
-    phases = std::max(8, (grid + fit_blocks - 1) / fit_blocks);
+    // (the small workgroups of a short query: half as many, so that each
+    // walks several reference pairs after filling its pipeline)
+    phases = std::max(8, ((ft == 1 ? grid / 2 : grid) + fit_blocks - 1) / fit_blocks);
     int p2 = 1;
     while (p2 < phases) p2 <<= 1;
     phases = p2;
@@ -593,7 +594,7 @@ int fused_phases(const mdsctk_knn_ctx* c, int fit_tiles) {
 }
 
 size_t fused_list_entries(const mdsctk_knn_ctx* c, int64_t n_fit, int k1) {
-  const int phases = fused_phases(c, std::max(kTileAlign, padded_tiles(n_fit)));
+  const int phases = fused_phases(c, n_fit);
   return (size_t)n_fit * phases * 4 * list_capacity_for(k1);
 }
 
@@ -658,12 +659,25 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   const DevFrames& fit = s.fit;
   const int64_t n_fit = fit.n;
   const int cap = list_capacity_for(q.k1);
-  p->grid = contract_grid(c);
-  p->phases = fused_phases(c, fit.n_tiles);
+  p->ft = contract_fit_tiles(c->prec == kExact ? kFP32 : c->prec, n_fit);
+  p->grid = contract_grid(c, p->ft);
+  p->phases = fused_phases(c, n_fit);
   auto ent_bytes_for = [&](int phases) { return (size_t)n_fit * phases * 4 * cap * sizeof(uint2); };
+  // A sample pass of short queries: 1/16 of the reference pairs, or enough
+  // for 8 (k+1) frames.
+  const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
+  p->sample = 0;
+  p->sample_pairs = 0;
+  if (n_fit < kCrossMinFit && c->ref.n >= kSampleMinRef) {
+    const int want = std::max(ref_pairs / 16, 8 * q.k1 / (2 * kTile) + 1);
+    p->sample = ref_pairs / want;
+    if (p->sample < 4) p->sample = 0;  // too large a part of the query
+    if (p->sample) p->sample_pairs = (ref_pairs + p->sample - 1) / p->sample;
+  }
+  const size_t sample_bytes = p->sample ? (size_t)(p->sample_pairs + 1) * sizeof(int) : 0;
   auto small_bytes_for = [&](int phases) {
     return (size_t)n_fit * phases * 4 * (sizeof(int) + sizeof(float)) +
-           (size_t)n_fit * (sizeof(unsigned) + sizeof(float) + sizeof(int)) + 256;
+           (size_t)n_fit * (sizeof(unsigned) + sizeof(float) + sizeof(int)) + 256 + sample_bytes;
   };
   void* ent = nullptr;
   void* small_p = nullptr;
@@ -717,6 +731,7 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   L.thr = (unsigned*)sp; sp += n_fit * sizeof(unsigned);
   p->eps2 = (float*)sp; sp += n_fit * sizeof(float);
   p->d_fallback = (int*)sp; sp += n_fit * sizeof(int);
+  p->sample_list = (int*)sp; sp += sample_bytes;
   if ((size_t)(sp - (char*)small_p) > small_bytes_for(p->phases))
     return fail(c, MDSCTK_ERR_ARG, "internal: list headers for %d lists per query exceed their %zu bytes",
                 L.nl, small_bytes_for(p->phases));
@@ -890,7 +905,8 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
     none.nl = 4;
     none.cap = 256;
     HIP_TRY(c, launch_contract(c->ref, query_view(c->ref), none, nullptr, 1, lstride, false, nullptr,
-                               contract_grid(c), s.st, nullptr, 1, nullptr, near));
+                               contract_grid(c, contract_fit_tiles(c->prec)), s.st, nullptr, 1,
+                               nullptr, near));
     HIP_TRY(c, launch_near_keys(near, n, lstride, keys, ids, s.st));
     HIP_TRY(c, launch_sort_order(nullptr, nullptr, 0, keys, keys_out, ids, o.order, n, temp,
                                  sort_temp, s.st));
@@ -922,8 +938,23 @@ int enqueue_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   const DevFrames& R = ref_ops(c, q.nofit);
   HIP_TRY(c, launch_eps(fit, R, p.kappa, p.eps2, s.n_cand, s.st));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[2], s.st));
-  HIP_TRY(c, launch_contract(R, fit, p.L, p.eps2, q.k1, p.phases, q.nofit, nullptr, p.grid,
-                             s.st));
+  if (p.sample) {
+    // every p.sample-th reference pair, as one shared list over the phases;
+    // the (k+1)-th smallest key there bounds the row's threshold
+    TileList lm;
+    lm.shared = true;
+    lm.list = p.sample_list;
+    lm.count = p.sample_list + p.sample_pairs;
+    HIP_TRY(c, launch_stride_list(c->ref.n_tiles, p.sample, lm, s.st));
+    Lists LS = p.L;
+    LS.nl = 4 * std::min(p.phases, p.sample_pairs);
+    HIP_TRY(c, launch_contract(R, fit, LS, p.eps2, q.k1, LS.nl / 4, q.nofit, nullptr, p.grid, s.st,
+                               nullptr, 0, &lm, nullptr, p.ft));
+    HIP_TRY(c, launch_landmark_cap(LS, fit.n, q.k1, p.eps2, 1, p.L.thr, nullptr, s.st));
+    HIP_TRY(c, launch_init_lists(p.L, fit.n, s.st, false));
+  }
+  HIP_TRY(c, launch_contract(R, fit, p.L, p.eps2, q.k1, p.phases, q.nofit, nullptr, p.grid, s.st,
+                             nullptr, 0, nullptr, nullptr, p.ft));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
   HIP_TRY(c, launch_merge(c->ref, fit, c->w, p.L, p.eps2, q.k1, q.k_out, q.rank_off, q.nofit,
                           d_dist, d_idx, p.d_fallback, s.n_cand, nullptr, s.st));
@@ -955,7 +986,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
   // Each fit frame sees about half of its pairs, so half the list form's
   // phases (longer lists per phase, tighter list thresholds).
-  int phases = fused_phases(c, fit.n_tiles);
+  int phases = std::max(1, std::min(ref_pairs, fused_phases(c, std::max<int64_t>(n, kTile + 1))));
   if (c->forced_phases <= 0) phases = std::max(1, std::min(ref_pairs, std::max(4, phases / 2)));
   const int nl = phases * 4;
   // Landmark pass: every lstride-th reference tile pair.  The (k+1)-th
@@ -1061,7 +1092,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   const double kappa = (c->w.metric == kMetricRMSD ? kappa_for(c->prec, c->ref.natoms)
                                                    : kappa_data(c->prec, c->ref.natoms)) *
                        c->eps_scale;
-  const int grid = contract_grid(c);
+  const int grid = contract_grid(c, contract_fit_tiles(c->prec));
   const DevFrames& R = ref_ops(c, q.nofit);
   HIP_TRY(c, launch_eps_sym(fit, R, kappa, gmax_q, eps2, s.n_cand, s.st));
   HIP_TRY(c, hipEventRecord(s.ev[2], s.st));

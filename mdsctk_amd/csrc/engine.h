@@ -106,8 +106,14 @@ struct FusedPlan {
   int* d_fallback = nullptr;
   int phases = 0;
   int grid = 0;
+  int ft = 0;  // fit tiles per workgroup
+  // short queries: a sample pass over every sample-th reference pair (0: none)
+  int sample = 0;
+  int sample_pairs = 0;
+  int* sample_list = nullptr;
   double kappa = 0;
   CrossPlan x;
+  int kind() const { return x.on ? 2 : sample ? 1 : 0; }  // sequence of kernels
 };
 
 // What the fused pipeline did for a batch.
@@ -230,11 +236,11 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
 // Bytes of slot workspace the ordered form of a cross query of n_fit frames
 // takes (0: it takes every tile).
 size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);
-// Contraction grid (workgroups) and reference phases for a batch of
-// `fit_tiles` query tiles; candidate-list entries a batch of n_fit frames
+// Contraction grid (workgroups of ft fit tiles) and reference phases for a
+// batch of n_fit frames; candidate-list entries a batch of n_fit frames
 // needs (each entry 8 bytes; the headers take 8 bytes per list).
-int contract_grid(const mdsctk_knn_ctx* c);
-int fused_phases(const mdsctk_knn_ctx* c, int fit_tiles);
+int contract_grid(const mdsctk_knn_ctx* c, int ft);
+int fused_phases(const mdsctk_knn_ctx* c, int64_t n_fit);
 size_t fused_list_entries(const mdsctk_knn_ctx* c, int64_t n_fit, int k1);
 // The fused pipeline (lists, contraction, merge) for the slot's query
 // frames: plan_fused sizes the slot's workspace (it may allocate);

@@ -263,12 +263,13 @@ hipError_t launch_eps(const DevFrames& fit, const DevFrames& ref, double kappa, 
 // pass); 0 = all.  tiles: only the listed reference pairs of each block of
 // kFilterFitTiles fit tiles, dealt out over the phases.  near: no lists, only
 // each fit frame's smallest (key << 32 | reference) there (atomic minimum).
+// ft 1: the one-fit-tile workgroup of short queries (contract_fit_tiles).
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st,
                            const Mirror* mirror = nullptr, int ph_run = 0,
                            const TileList* tiles = nullptr,
-                           unsigned long long* near = nullptr);
+                           unsigned long long* near = nullptr, int ft = 0);
 // The window of a symmetric self query (fit: the reference set's query
 // view): eps2[r] = 2 kappa max(G~q[r] + max G~ref, G~ref[r] + max G~q);
 // *gmax_q receives max G~q.
@@ -354,6 +355,19 @@ hipError_t scratch_region(int device, void** addr);
 
 // Fit tiles per contraction workgroup for a precision (2 or 4).
 int contract_fit_tiles(int prec);
+// The same for a query of n_fit frames: 1 for split forms and up to 32
+// frames, where three of four fit tiles would be padding.  Two 2-wave
+// workgroups per CU then stream the resident operand.  Measured, 1 frame
+// against 100000 x 500 (614 MB of operand) with half the CUs, as a served
+// batch gets: contraction 582 -> 199 us, 3.1 TB/s.
+int contract_fit_tiles(int prec, int64_t n_fit);
+// Queries of fewer frames than kCrossMinFit against this many resident frames
+// or more bound their thresholds by a sample pass first: without a threshold
+// every pair of a row enters its lists (no list fills up), and the merge of
+// a few rows, a workgroup each, then walks n_ref entries a row in every
+// radix pass.  Measured, 1 frame against 100000: merge 230 -> 98 us for a
+// sample pass of 41 us and its cap of 22 us.
+constexpr int64_t kSampleMinRef = 16384;
 // Choose the per-list capacity for k1 (0 when the fused path cannot serve it).
 int list_capacity_for(int k1);
 

@@ -982,6 +982,11 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
   // skip the MFMAs.
   const int ngs = PIPE ? ng : (ng + 2) / 3 * 3;
 
+  // FT 1 (two waves, three tiles): each wave copies its reference tile and
+  // half of the fit tile.
+  constexpr bool HALF = FT == 1;
+  constexpr int LPS = BPG + (HALF ? BPG / 2 : 0);  // copies of a wave per stage
+  static_assert(!HALF || BPG % 2 == 0, "the fit tile splits in two");
   // Waves 0..kSlots-1 each copy one stage slot (slot = wave); the others
   // only compute.
   constexpr int kSlots = kRefTilesPerWG + FT;
@@ -998,7 +1003,8 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
   uint4* const d3 = sbuf3 + (PIPE && copier ? wave : 0) * TILE_VEC;
   const uint4* const a3 = sbuf3 + (PIPE ? ri : 0) * TILE_VEC;
   const uint4* const b3 = sbuf3 + (PIPE ? kRefTilesPerWG + fi : 0) * TILE_VEC;
-  const int fit_blocks = P.fit_tiles / FT;
+  // blocks of padding alone are left out
+  const int fit_blocks = (int)((P.n_fit + (int64_t)FT * kTile - 1) / (FT * kTile));
 
   // Workgroups are dispatched round-robin over the 8 XCDs; renumber them so
   // that consecutive work items (same fit block, neighbouring reference
@@ -1061,7 +1067,7 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     // FT*fb+w-2.  Stages past the item's last tile re-read its last tile
     // (never used).
     const uint4* const fit_base =
-        P.fop + (int64_t)(FT * fb + (copier ? wave : 2) - kRefTilesPerWG) * ng * TILE_VEC;
+        P.fop + (int64_t)(FT * fb + (HALF || !copier ? 0 : wave - kRefTilesPerWG)) * ng * TILE_VEC;
     // p_cur, p_next: the current and the next tile's reference pair (its own
     // again past the last tile, where the copies are never used).
     int p_cur = pair_of(t0);
@@ -1078,6 +1084,16 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
       for (int j = 0; j < BPG; ++j)
         __builtin_amdgcn_global_load_lds((const void*)(src + j * 64),
                                          (lds_void_t*)(dst + j * 64), 16, 0, 0);
+      if constexpr (HALF) {
+        // the fit tile is the third slot of the stage
+        const int h = wave * (BPG / 2) * 64;
+        const uint4* const fsrc = fit_base + (int64_t)(over ? g - ngs : g) * TILE_VEC + h + lane;
+        uint4* const fdst = dst + (kRefTilesPerWG - wave) * TILE_VEC + h;
+#pragma unroll
+        for (int j = 0; j < BPG / 2; ++j)
+          __builtin_amdgcn_global_load_lds((const void*)(fsrc + j * 64),
+                                           (lds_void_t*)(fdst + j * 64), 16, 0, 0);
+      }
     };
 
     __syncthreads();  // previous item's readers of sbuf*/sGr/sThr are done
@@ -1089,7 +1105,7 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     dma_stage(0, d0);
     dma_stage(1, d1);
     if constexpr (PIPE) dma_stage(2, d2);
-    stage_barrier<BPG>();  // stage 0 (and with PIPE stage 1) landed
+    stage_barrier<LPS>();  // stage 0 (and with PIPE stage 1) landed
     // PIPE: the fragments of the stage about to be computed (B double-buffered)
     uint4 bh0[3], bl0[3], bh1[3], bl1[3], ah, al;
     if constexpr (PIPE) {
@@ -1133,16 +1149,16 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
         for (int g = 0; g < ng; g += 4) {
           pipe_stage<PREC, true, true>(acc, a0, a1, b1, bh0, bl0, bh1, bl1, ah, al, lane);
           dma_stage(g + 3, d3);
-          stage_barrier_vm<BPG>();
+          stage_barrier_vm<LPS>();
           pipe_stage<PREC, true, true>(acc, a1, a2, b2, bh1, bl1, bh0, bl0, ah, al, lane);
           dma_stage(g + 4, d0);
-          stage_barrier_vm<BPG>();
+          stage_barrier_vm<LPS>();
           pipe_stage<PREC, true, true>(acc, a2, a3, b3, bh0, bl0, bh1, bl1, ah, al, lane);
           dma_stage(g + 5, d1);
-          stage_barrier_vm<BPG>();
+          stage_barrier_vm<LPS>();
           pipe_stage<PREC, true, true>(acc, a3, a0, b0, bh1, bl1, bh0, bl0, ah, al, lane);
           dma_stage(g + 6, d2);
-          stage_barrier_vm<BPG>();
+          stage_barrier_vm<LPS>();
         }
       } else {
         // Stage g lives in buffer g % 3; while it is consumed, stage g+2 (in
@@ -1154,13 +1170,13 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
         for (int g = 0; g < ngs; g += 3) {
           mma_group<PREC, TRACE>(acc, a0, b0, lane);
           dma_stage(g + 2, d2);
-          stage_barrier<BPG>();
+          stage_barrier<LPS>();
           if (g + 1 < ng) mma_group<PREC, TRACE>(acc, a1, b1, lane);
           dma_stage(g + 3, d0);
-          stage_barrier<BPG>();
+          stage_barrier<LPS>();
           if (g + 2 < ng) mma_group<PREC, TRACE>(acc, a2, b2, lane);
           dma_stage(g + 4, d1);
-          stage_barrier<BPG>();
+          stage_barrier<LPS>();
         }
       }
       // Publish the next tile's G~ and thresholds (read by its epilogue,
@@ -1271,28 +1287,28 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
 }
 
 // The bin of a 256-bin histogram that holds the rank-th (0-based) of its
-// counts, and the rank within the bin, for every thread of a 256-thread
-// workgroup: an inclusive scan over lanes and waves.  (One thread walking the
+// counts, and the rank within the bin, for every thread of a workgroup of 256
+// threads or more: an inclusive scan over lanes and waves.  (One thread walking the
 // bins took about 7 us a pass, most of the merge and of the landmark caps.)
 __device__ __forceinline__ void pick_bin(const unsigned* hist, int rank, int* bin, int* rest) {
   __shared__ unsigned wave_total[4];
   __shared__ int s_bin, s_rest;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const unsigned h = hist[tid];
+  const unsigned h = tid < 256 ? hist[tid] : 0u;
   unsigned inc = h;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
     const unsigned t = __shfl_up(inc, o);
     if (lane >= o) inc += t;
   }
-  if (lane == 63) wave_total[wave] = inc;
+  if (lane == 63 && wave < 4) wave_total[wave] = inc;
   if (tid == 0) {  // no bin reaches the rank: the last one
     s_bin = 255;
     s_rest = 0;
   }
   __syncthreads();
-  for (int w = 0; w < wave; ++w) inc += wave_total[w];
-  if (inc - h <= (unsigned)rank && (unsigned)rank < inc) {
+  for (int w = 0; w < wave && w < 4; ++w) inc += wave_total[w];
+  if (tid < 256 && inc - h <= (unsigned)rank && (unsigned)rank < inc) {
     s_bin = tid;
     s_rest = rank - (int)(inc - h);
   }
@@ -1503,8 +1519,13 @@ constexpr int kMergeStageAtoms = 1024;
 // CAND: the most candidates a row's window may hold (more: exact path).
 // The smaller instance leaves room for more workgroups per CU; the
 // waves-per-EU hint keeps it within 96 VGPRs (5 workgroups per CU).
-template <bool STAGE, int CAND>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void merge_kernel(MergeParams P) {
+// T: threads.  256, or 1024 for queries of few rows, where a row's workgroup
+// has a CU to itself and waits on its lists' and candidates' loads: four
+// times as many are then in flight (one row of 100000 x 500 atoms, 1024
+// lists: 98 -> 48 us).
+template <bool STAGE, int CAND, int T>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T == 256 ? 5 : 4))) void merge_kernel(
+    MergeParams P) {
   const int64_t qi = P.perm ? (int64_t)blockIdx.x : (P.order ? P.order[blockIdx.x] : blockIdx.x);
   const int64_t q = P.perm ? P.perm[qi] : qi;  // the frame: data and output row
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -1536,7 +1557,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   const bool list_per_thread = P.nl >= 256;
   auto visit = [&](auto&& f) {
     if (list_per_thread) {
-      for (int l = tid; l < P.nl; l += 256) {
+      for (int l = tid; l < P.nl; l += T) {
         const int c = cnt[l];
         const uint2* el = ent + (int64_t)l * P.cap;
         int i = 0;
@@ -1550,19 +1571,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
         for (; i < c; ++i) f(el[i]);
       }
     } else {
-      for (int l = wave; l < P.nl; l += 4) {
+      for (int l = wave; l < P.nl; l += T / 64) {
         const int c = cnt[l];
         for (int i = lane; i < c; i += 64) f(ent[(int64_t)l * P.cap + i]);
       }
     }
-    for (int i = tid; i < mc; i += 256) f(ment[i]);
+    for (int i = tid; i < mc; i += T) f(ment[i]);
   };
-
   if (tid == 0) { s_total = mc; s_nc = 0; s_flag = 0; s_bad = 0; s_ng = 0; }
   __syncthreads();
   {
     int part = 0;
-    for (int l = tid; l < P.nl; l += 256) part += cnt[l];
+    for (int l = tid; l < P.nl; l += T) part += cnt[l];
     atomicAdd(&s_total, part);
   }
   __syncthreads();
@@ -1574,7 +1594,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   unsigned prefix = 0;
   int kk = P.k1 - 1;
   for (int shift = 24; shift >= 0; shift -= 8) {
-    hist[tid] = 0;
+    if (tid < 256) hist[tid] = 0;
     __syncthreads();
     const unsigned mhi = (shift == 24) ? 0u : (0xFFFFFFFFu << (shift + 8));
     visit([&](const uint2 e) {
@@ -1593,7 +1613,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   // narrow for its row would drop pairs whose keys lie just above the cut,
   // so up to kMergeGuard of those are re-scored as well.
   const float guard_cut = cut + e2q;
-  for (int l = tid; l < P.nl; l += 256)
+  for (int l = tid; l < P.nl; l += T)
     if (ovf[l] <= cut) s_flag = 1;
   if (tid == 0 && P.ment && P.movf[qi] <= cut) s_flag = 1;
   visit([&](const uint2 e) {
@@ -1627,7 +1647,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   if constexpr (STAGE) {
     const F3* fx = reinterpret_cast<const F3*>(P.src.fxyz) + q * (int64_t)P.src.natoms;
     const double c0 = P.src.fcen[q * 3], c1 = P.src.fcen[q * 3 + 1], c2 = P.src.fcen[q * 3 + 2];
-    for (int i = tid; i < P.src.natoms; i += 256) {
+    for (int i = tid; i < P.src.natoms; i += T) {
       const F3 b = fx[i];
       const double wi = (double)P.src.w[i];
       qw_stage[3 * i] = weighted_centred(b.x, c0, wi);
@@ -1651,7 +1671,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
     const double gq = P.src.fG[q];
     for (int c0 = 0; c0 < total; c0 += kMergeChunk) {
       const int m = min(kMergeChunk, total - c0);
-      for (int j = tid >> 4; j < m; j += 16) {
+      for (int j = tid >> 4; j < m; j += T / 16) {
         const int c = c0 + j;
         const int64_t r = c < nc ? cand_idx[c] : guard_idx[c - nc];
         double S[9];
@@ -1664,7 +1684,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
         }
       }
       __syncthreads();
-      for (int j = tid; j < m; j += 256) {
+      for (int j = tid; j < m; j += T) {
         const int c = c0 + j;
         const int64_t r = c < nc ? cand_idx[c] : guard_idx[c - nc];
         put(c, cross_score(pair_S + j * 9, P.src.rG[r], gq, P.nofit));
@@ -1672,7 +1692,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
       __syncthreads();
     }
   } else {
-    for (int c = wave; c < nc + ng; c += 4) {
+    for (int c = wave; c < nc + ng; c += T / 64) {
       const int r = c < nc ? cand_idx[c] : guard_idx[c - nc];
       const double s = wave_data_pair_score(P.src, r, q);
       if (lane == 0) put(c, s);
@@ -1686,7 +1706,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   // allowance.
   {
     const double eps = 0.5 * (double)e2q;
-    for (int c = tid; c < nc + ng; c += 256) {
+    for (int c = tid; c < nc + ng; c += T) {
       const double s = c < nc ? cand_s[c] : guard_s[c - nc];
       const double kq = (double)(c < nc ? cand_key[c] : guard_key[c - nc]);
       if (fabs(kq - s) > eps + 1.2e-7 * fmax(kq, s)) s_bad = 1;
@@ -1699,12 +1719,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void m
   }
   int np2 = 64;
   while (np2 < nc) np2 <<= 1;
-  for (int i = nc + tid; i < np2; i += 256) {
+  for (int i = nc + tid; i < np2; i += T) {
     cand_s[i] = INFINITY;
     cand_idx[i] = INT_MAX;
   }
   block_bitonic_sort(cand_s, cand_idx, np2);
-  for (int j = tid; j < P.k_out; j += 256) {
+  for (int j = tid; j < P.k_out; j += T) {
     const int src = j + P.rank_off;
     P.out_dist[q * P.k_out + j] = P.out_scale * sqrt(fmax(cand_s[src], 0.0) / P.W);
     P.out_idx[q * P.k_out + j] = cand_idx[src];
@@ -1744,10 +1764,27 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
   const unsigned span = 2u * kTile * (unsigned)phases;
   auto dense = [&](unsigned r) { return (r / span) * (2u * kTile) + r % (2u * kTile); };
   const uint2* e = ent + q * (int64_t)nl * cap;
+  // many lists (a short query's sample pass): a thread per list, as the merge
   auto visit = [&](auto&& f) {
-    for (int l = wave; l < nl; l += 4) {
-      const int cl = c[l];
-      for (int i = lane; i < cl; i += 64) f(e[(int64_t)l * cap + i]);
+    if (nl >= 256) {
+      for (int l = tid; l < nl; l += 256) {
+        const int cl = c[l];
+        const uint2* el = e + (int64_t)l * cap;
+        int i = 0;
+        for (; i + 4 <= cl; i += 4) {
+          const uint2 x0 = el[i], x1 = el[i + 1], x2 = el[i + 2], x3 = el[i + 3];
+          f(x0);
+          f(x1);
+          f(x2);
+          f(x3);
+        }
+        for (; i < cl; ++i) f(el[i]);
+      }
+    } else {
+      for (int l = wave; l < nl; l += 4) {
+        const int cl = c[l];
+        for (int i = lane; i < cl; i += 64) f(e[(int64_t)l * cap + i]);
+      }
     }
   };
   if (tid == 0) {
@@ -2379,6 +2416,10 @@ __global__ __launch_bounds__(256) void data_prep_kernel(const double* __restrict
 
 int contract_fit_tiles(int prec) { return prec == kFP32 ? 2 : 4; }
 
+int contract_fit_tiles(int prec, int64_t n_fit) {
+  return prec != kFP32 && n_fit <= kTile ? 1 : contract_fit_tiles(prec);
+}
+
 int list_capacity_for(int k1) {
   if (k1 <= 128) return 256;
   if (k1 <= 384) return 512;
@@ -2454,7 +2495,7 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st, const Mirror* mirror,
-                           int ph_run, const TileList* tiles, unsigned long long* near) {
+                           int ph_run, const TileList* tiles, unsigned long long* near, int ft) {
   ContractParams P;
   P.rop = ref.op;
   P.fop = fit.op;
@@ -2532,6 +2573,26 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
     else                                            \
       return hipErrorInvalidValue;                  \
   } while (0)
+#define MDSCTK_CONTRACT_SMALL(PR)                   \
+  do {                                              \
+    if (L.cap == 256)                               \
+      MDSCTK_CONTRACT_TR(PR, 4, 1, kOutLists);      \
+    else if (L.cap == 512)                          \
+      MDSCTK_CONTRACT_TR(PR, 8, 1, kOutLists);      \
+    else if (L.cap == 1024)                         \
+      MDSCTK_CONTRACT_TR(PR, 16, 1, kOutLists);     \
+    else                                            \
+      return hipErrorInvalidValue;                  \
+  } while (0)
+  if (ft == 1) {
+    if (dbg_scores || near || mirror || (tiles && !tiles->shared)) return hipErrorInvalidValue;
+    switch (ref.prec) {
+      case kBF16: MDSCTK_CONTRACT_SMALL(kBF16); break;
+      case kFP16: MDSCTK_CONTRACT_SMALL(kFP16); break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   switch (ref.prec) {
     case kFP32: MDSCTK_CONTRACT_CAP(kFP32, 2); break;
     case kBF16: MDSCTK_CONTRACT_CAP(kBF16, 4); break;
@@ -2539,6 +2600,7 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
     default: return hipErrorInvalidValue;
   }
 #undef MDSCTK_CONTRACT_CAP
+#undef MDSCTK_CONTRACT_SMALL
 #undef MDSCTK_CONTRACT_TR
 #undef MDSCTK_CONTRACT
   return hipGetLastError();
@@ -2597,18 +2659,28 @@ hipError_t launch_merge(const DevFrames& ref, const DevFrames& fit, const DevWei
   // the candidate LDS of the general instance
   const bool stage = w.metric == kMetricRMSD && ref.natoms <= kMergeStageAtoms;
   const size_t dyn = stage ? (size_t)ref.natoms * 3 * sizeof(double) : 0;
-  const dim3 grid((unsigned)fit.n), block(256);
+  // few rows: a CU or more to each
+  const bool wide = fit.n <= 256;
+  const dim3 grid((unsigned)fit.n);
+#define MDSCTK_MERGE(ST, CA)                                                                 \
+  do {                                                                                       \
+    if (wide)                                                                                \
+      hipLaunchKernelGGL((merge_kernel<ST, CA, 1024>), grid, dim3(1024), dyn, st, P);        \
+    else                                                                                     \
+      hipLaunchKernelGGL((merge_kernel<ST, CA, 256>), grid, dim3(256), dyn, st, P);          \
+  } while (0)
   if (k1 <= kMergeSmallK1) {
     if (stage)
-      hipLaunchKernelGGL((merge_kernel<true, kCandSmall>), grid, block, dyn, st, P);
+      MDSCTK_MERGE(true, kCandSmall);
     else
-      hipLaunchKernelGGL((merge_kernel<false, kCandSmall>), grid, block, dyn, st, P);
+      MDSCTK_MERGE(false, kCandSmall);
   } else {
     if (stage)
-      hipLaunchKernelGGL((merge_kernel<true, kCandMax>), grid, block, dyn, st, P);
+      MDSCTK_MERGE(true, kCandMax);
     else
-      hipLaunchKernelGGL((merge_kernel<false, kCandMax>), grid, block, dyn, st, P);
+      MDSCTK_MERGE(false, kCandMax);
   }
+#undef MDSCTK_MERGE
   return hipGetLastError();
 }
 

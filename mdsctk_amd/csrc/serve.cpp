@@ -43,14 +43,14 @@ struct HipSlot {
   bool all_exact = false;  // the batch took the exact rows, not the contraction
   size_t h_elems = 0, h_rows = 0;
   hipEvent_t done = nullptr;
-  // the slot's batch kernels, updated per batch: [0] every tile, [1] the
-  // ordered form (another sequence of kernels)
-  hipGraphExec_t exec[2] = {nullptr, nullptr};
+  // the slot's batch kernels, updated per batch: one per
+  // sequence of kernels (FusedPlan::kind)
+  hipGraphExec_t exec[3] = {};
   // the captured graph exec was last instantiated or updated from; kept
   // until a later capture has replaced it in exec (and that exec has been
   // launched), so nothing the executable may refer to is released while it
   // can still run
-  hipGraph_t graph[2] = {nullptr, nullptr};
+  hipGraph_t graph[3] = {};
   // shape the workspace was last sized for
   int64_t sized_limit = 0;
   int sized_k_out = -1, sized_k1 = -1;
@@ -246,11 +246,13 @@ class HipServeDevice {
  private:
   // Largest list workspace (entries, list headers) any batch of up to
   // `limit` frames needs: the phase count grows as batches shrink, so take
-  // the maximum over batch sizes (it changes only at 128-frame steps).
+  // the maximum over batch sizes (it changes only at 128-frame
+  // steps, and above the 32 frames of the shortest form).
   void list_need(int64_t limit, const QueryShape& q, size_t* entries, size_t* headers) const {
     *entries = *headers = 0;
     const size_t cap = (size_t)list_capacity_for(q.k1);
-    for (int64_t n = std::min<int64_t>(limit, 128);; n = std::min<int64_t>(limit, n + 128)) {
+    for (int64_t n = std::min<int64_t>(limit, kTile);;
+         n = std::min<int64_t>(limit, n < 128 ? 128 : n + 128)) {
       const size_t e = fused_list_entries(c_, n, q.k1);
       *entries = std::max(*entries, e);
       *headers = std::max(*headers, e / cap);
@@ -283,7 +285,9 @@ class HipServeDevice {
       size_t ent, hdr;
       list_need(limit, q, &ent, &hdr);
       if ((rc = ensure(c_, &s.ws_lists, &s.ws_lists_bytes, ent * 8, "candidate lists"))) return rc;
-      const size_t small = hdr * 8 + (size_t)limit * 12 + 256;
+      // the headers, per-frame terms and a short query's sample list
+      const size_t small = hdr * 8 + (size_t)limit * 12 + 256 +
+                           (size_t)(c_->ref.n_tiles / kRefTilesPerWG + 2) * sizeof(int);
       if ((rc = ensure(c_, &s.ws_small, &s.ws_small_bytes, small, "list headers"))) return rc;
     }
     const size_t elems = (size_t)limit * q.k_out;
@@ -343,8 +347,8 @@ class HipServeDevice {
   // then never reads released memory).
   int replay_graph(HipSlot& sl, const QueryShape& q, const FusedPlan& plan) {
     Slot& s = sl.s;
-    hipGraphExec_t& exec = sl.exec[plan.x.on];
-    hipGraph_t& graph = sl.graph[plan.x.on];
+    hipGraphExec_t& exec = sl.exec[plan.kind()];
+    hipGraph_t& graph = sl.graph[plan.kind()];
     hipError_t e = hipStreamBeginCapture(s.st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(c_, e, "serve: graph capture");
     int rc = prep_slot(c_, s, q.nofit);
