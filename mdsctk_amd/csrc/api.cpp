@@ -984,10 +984,18 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   const int cap = list_capacity_for(q.k1);
   if (cap == 0) return 1;
   const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
-  // Each fit frame sees about half of its pairs, so half the list form's
-  // phases (longer lists per phase, tighter list thresholds).
-  int phases = std::max(1, std::min(ref_pairs, fused_phases(c, std::max<int64_t>(n, kTile + 1))));
-  if (c->forced_phases <= 0) phases = std::max(1, std::min(ref_pairs, std::max(4, phases / 2)));
+  // Four phases (each fit frame sees about half of its pairs: longer lists
+  // per phase, tighter list thresholds), more for a small set, until its
+  // items, half of them below the diagonal, fill the grid twice: a 2000-frame
+  // set then takes one tile an item (contraction of 2000 x 304 atoms 207 ->
+  // 110 us).
+  const int grid = contract_grid(c, contract_fit_tiles(c->prec));
+  const int blocks = std::max(1, fit.n_tiles / contract_fit_tiles(c->prec));
+  int phases = c->forced_phases;
+  if (phases <= 0)
+    for (phases = 4; phases * blocks < 2 * grid; phases *= 2) {
+    }
+  phases = std::max(1, std::min(ref_pairs, phases));
   const int nl = phases * 4;
   // Landmark pass: every lstride-th reference tile pair.  The (k+1)-th
   // smallest key of L landmarks ranks about (k+1) n / L among a row's n
@@ -1005,15 +1013,18 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
                                      (int)((int64_t)ref_pairs * 2 * kTile / lm_target))));
   const int lm_pairs = (ref_pairs + lstride - 1) / lstride;
   const int nlab = lm_pairs * 2 * kTile;
+  // its pairs as one list, split over enough phases to fill the grid
+  const int lm_phases = std::max(1, std::min({phases, lm_pairs, 2 * grid / blocks}));
   const size_t ent_bytes = (size_t)n * nl * cap * sizeof(uint2);
-  // Canonical form (fitted scores of frames, n >= 512): the main pass runs
-  // over a copy of the set in landmark order, every frame in its principal
-  // axes.  Frames near each other in the order are near each other in
+  // Canonical form (fitted scores of frames, kFilterMinFrames or more): the
+  // main pass runs over a copy of the set in landmark order, every frame in
+  // its principal axes.  (Below that, ordering and copying cost more than the
+  // order saves: 105 us of the 2000-frame query.)  Frames near each other in the order are near each other in
   // space, so most 32 x 32 tiles hold only far pairs, which the
   // contraction's lambda_max bound rejects without the QCP; the axes make
   // that bound nearly exact for similar frames.  The copy: operands (both
   // dither sides), centroids, G, G~, rotations, windows, thresholds.
-  const bool canon = !q.nofit && c->w.metric == kMetricRMSD && n >= 512;
+  const bool canon = !q.nofit && c->w.metric == kMetricRMSD && n >= kFilterMinFrames;
   const bool dith = c->ref.op_q != nullptr;
   const size_t rows = (size_t)c->ref.n_tiles * kTile;
   const size_t opb = operand_bytes(c->ref.prec, c->ref.n_tiles, c->ref.n_groups);
@@ -1042,7 +1053,8 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   bool filter = canon && n >= kFilterMinFrames;
   size_t sym_bytes = Carve::round(mir_bytes) + perm_bytes + (filter ? filter_bytes : 0);
   const size_t small = (size_t)n * nl * (sizeof(int) + sizeof(float)) +
-                       (size_t)n * 7 * sizeof(int) + (size_t)nlab * sizeof(int) + 1024;
+                       (size_t)n * 7 * sizeof(int) + (size_t)nlab * sizeof(int) +
+                       (size_t)(lm_pairs + 1) * sizeof(int) + 1024;
   // Room: the free device memory plus what the buffers already hold, less a
   // reserve for everything else; and the context's budget.
   size_t free_b = 0, total_b = 0;
@@ -1088,20 +1100,24 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   M.ent = (uint2*)s.ws_sym;
   M.cap = c->mirror_cap;
   M.cnt = (int*)sp; sp += n * sizeof(int);
-  M.ovf = (float*)sp;
+  M.ovf = (float*)sp; sp += n * sizeof(float);
+  TileList lm;
+  lm.shared = true;
+  lm.list = (int*)sp; sp += lm_pairs * sizeof(int);
+  lm.count = (int*)sp;
   const double kappa = (c->w.metric == kMetricRMSD ? kappa_for(c->prec, c->ref.natoms)
                                                    : kappa_data(c->prec, c->ref.natoms)) *
                        c->eps_scale;
-  const int grid = contract_grid(c, contract_fit_tiles(c->prec));
   const DevFrames& R = ref_ops(c, q.nofit);
   HIP_TRY(c, launch_eps_sym(fit, R, kappa, gmax_q, eps2, s.n_cand, s.st));
   HIP_TRY(c, hipEventRecord(s.ev[2], s.st));
-  // landmark pass into the first 4 lists' worth of the list workspace
+  // landmark pass into the first lists' worth of the list workspace
   Lists LL = L;
-  LL.nl = 4;
+  LL.nl = 4 * lm_phases;
+  HIP_TRY(c, launch_stride_list(c->ref.n_tiles, lstride, lm, s.st));
   HIP_TRY(c, launch_init_lists(LL, n, s.st));
-  HIP_TRY(c, launch_contract(R, fit, LL, eps2, q.k1, lstride, q.nofit, nullptr, grid, s.st,
-                             nullptr, 1));
+  HIP_TRY(c, launch_contract(R, fit, LL, eps2, q.k1, lm_phases, q.nofit, nullptr, grid, s.st,
+                             nullptr, 0, &lm));
   Carve fc;
   fc.base = (char*)s.ws_sym + Carve::round(mir_bytes) + perm_bytes;
   fc.size = filter ? filter_bytes : 0;
@@ -1129,7 +1145,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   // rows grouped by nearest landmark: the merge takes them in this order (it
   // pays where candidate frames no longer fit the caches), and the canonical
   // form contracts the frames in it
-  const bool ordered = n >= 512;
+  const bool ordered = n >= kFilterMinFrames;
   if (ordered && !filter) HIP_TRY(c, launch_row_order(label, n, nlab, counts, order, s.st));
   // the main pass's frames, windows and thresholds
   DevFrames mref = R, mfit = fit;

@@ -1554,7 +1554,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T == 256 ? 5 
   // reference phases): a thread per list, streaming its entries with four
   // loads in flight -- a wave per list would wait on one list's count and
   // entries at a time, hundreds of times per pass.
-  const bool list_per_thread = P.nl >= 256;
+  const bool list_per_thread = P.nl >= 64;
   auto visit = [&](auto&& f) {
     if (list_per_thread) {
       for (int l = tid; l < P.nl; l += T) {
@@ -1766,7 +1766,7 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
   const uint2* e = ent + q * (int64_t)nl * cap;
   // many lists (a short query's sample pass): a thread per list, as the merge
   auto visit = [&](auto&& f) {
-    if (nl >= 256) {
+    if (nl >= 64) {
       for (int l = tid; l < nl; l += 256) {
         const int cl = c[l];
         const uint2* el = e + (int64_t)l * cap;
