@@ -234,8 +234,8 @@ int prep_frames(mdsctk_knn_ctx* c, DevFrames& f, hipStream_t st, bool resident, 
 // max Gt of a resident set, kept on the device for every later window.
 int resident_gmax(mdsctk_knn_ctx* c, DevFrames& f, hipStream_t st) {
   if (c->prec == kExact) return 0;  // no contraction, no window
-  int rc = dalloc(c, (void**)&f.gmax, sizeof(double), "max G term");
-  if (rc) return rc;
+  int rc = 0;
+  if (!f.gmax && (rc = dalloc(c, (void**)&f.gmax, sizeof(double), "max G term"))) return rc;
   HIP_TRY(c, launch_max_gt(f, f.gmax, st));
   return 0;
 }
@@ -316,12 +316,19 @@ int set_weights(mdsctk_knn_ctx* c, const float* weights, int natoms) {
     W += wi;
   }
   if (!(W > 0)) return fail(c, MDSCTK_ERR_ARG, "weights sum to zero");
-  dfree(c, c->w.w);
-  dfree(c, c->w.sw);
-  c->w = DevWeights();
+  // kept for a set of as many atoms
+  DevWeights keep;
+  if (c->w.natoms == natoms) {
+    keep.w = c->w.w;
+    keep.sw = c->w.sw;
+  } else {
+    dfree(c, c->w.w);
+    dfree(c, c->w.sw);
+  }
+  c->w = keep;
   int rc;
-  if ((rc = dalloc(c, (void**)&c->w.w, natoms * sizeof(float), "weights"))) return rc;
-  if ((rc = dalloc(c, (void**)&c->w.sw, natoms * sizeof(float), "weights"))) return rc;
+  if (!c->w.w && (rc = dalloc(c, (void**)&c->w.w, natoms * sizeof(float), "weights"))) return rc;
+  if (!c->w.sw && (rc = dalloc(c, (void**)&c->w.sw, natoms * sizeof(float), "weights"))) return rc;
   hipStream_t st = c->main.st;
   HIP_TRY(c, hipMemcpyAsync(c->w.w, w.data(), natoms * sizeof(float), hipMemcpyHostToDevice, st));
   HIP_TRY(c, hipMemcpyAsync(c->w.sw, sw.data(), natoms * sizeof(float), hipMemcpyHostToDevice, st));
@@ -342,23 +349,32 @@ int set_reference_impl(mdsctk_knn_ctx* c, const float* xyz, bool on_device, int6
     return fail(c, MDSCTK_ERR_STATE, "set_reference: served requests are still outstanding");
   server_stop(c);
   HIP_TRY(c, hipSetDevice(c->device));
-  free_frames(c, c->ref);
+  // A set of the same shape takes over the last one's buffers (trajectory
+  // after trajectory of one system): nine allocations and their frees, each
+  // of which waits for the device, took a third of a 1000 x 60-frame run.
+  // Not under an HBM budget, which is checked as the buffers are allocated.
+  const bool same = c->has_ref && !c->budget && c->w.metric == kMetricRMSD && c->ref.vdim == 0 &&
+                    c->ref.n == n_ref && c->ref.natoms == natoms;
+  if (!same) free_frames(c, c->ref);
   free_plain(c);
   free_ordered(c);
   c->ref_axes = false;
-  release_mirror_lists(c);
+  if (!same) release_mirror_lists(c);
   dfree(c, c->data_shift);
   c->data_shift = nullptr;
   c->has_ref = false;
   int rc = set_weights(c, weights, natoms);
-  if (rc) return rc;
+  if (rc) {
+    free_frames(c, c->ref);
+    return rc;
+  }
   const size_t xbytes = (size_t)n_ref * natoms * 3 * sizeof(float);
-  if ((rc = dalloc(c, (void**)&c->ref.xyz, xbytes, "reference coordinates"))) return rc;
+  if (!same && (rc = dalloc(c, (void**)&c->ref.xyz, xbytes, "reference coordinates"))) return rc;
   HIP_TRY(c, hipMemcpyAsync(c->ref.xyz, xyz, xbytes,
                             on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice,
                             c->main.st));
   c->ref.owns_xyz = true;
-  if ((rc = alloc_frames(c, c->ref, n_ref, natoms, c->prec))) return rc;
+  if (!same && (rc = alloc_frames(c, c->ref, n_ref, natoms, c->prec))) return rc;
   c->ref_axes = axes_form(c);
   if ((rc = prep_frames(c, c->ref, c->main.st, true, c->ref_axes))) return rc;
   if ((rc = resident_gmax(c, c->ref, c->main.st))) return rc;
@@ -456,7 +472,7 @@ int slot_init(mdsctk_knn_ctx* c, Slot& s) {
   HIP_TRY(c, hipStreamCreateWithFlags(&s.st, hipStreamNonBlocking));
   for (auto& e : s.ev) HIP_TRY(c, hipEventCreate(&e));
   int rc;
-  if ((rc = dalloc(c, (void**)&s.n_cand, 256, "scratch"))) return rc;
+  if ((rc = dalloc(c, (void**)&s.sum, sizeof(QuerySummary), "scratch"))) return rc;
   return 0;
 }
 
@@ -474,7 +490,8 @@ void slot_release(mdsctk_knn_ctx* c, Slot& s) {
   free_frames(c, s.fit);
   dfree(c, s.ws_lists);
   dfree(c, s.ws_small);
-  dfree(c, s.n_cand);
+  dfree(c, s.sum);
+  if (s.h_out) (void)hipHostFree(s.h_out);
   dfree(c, s.ws_out);
   dfree(c, s.ws_rows);
   dfree(c, s.ws_sym);
@@ -784,7 +801,7 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   LL.thr = x.thr0;
   HIP_TRY(c, launch_stride_list(c->ref.n_tiles, x.lstride, lm, s.st));
   HIP_TRY(c, launch_init_lists(LL, n, s.st));
-  HIP_TRY(c, launch_eps(fit, R, p.kappa, x.eps0, s.n_cand, s.st));
+  HIP_TRY(c, launch_eps(fit, R, p.kappa, x.eps0, s.sum, s.st));
   HIP_TRY(c, launch_contract(R, fit, LL, x.eps0, q.k1, lm_phases, false, nullptr, p.grid, s.st,
                              nullptr, 0, &lm));
   HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, x.eps0, x.lstride, x.thr0, x.label, s.st, 1, x.keys,
@@ -807,7 +824,7 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
                              nullptr, 0, &x.tiles));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
   HIP_TRY(c, launch_merge(c->ref, fit, c->w, p.L, p.eps2, q.k1, q.k_out, q.rank_off, false, d_dist,
-                          d_idx, p.d_fallback, s.n_cand, nullptr, s.st, nullptr, x.order, o.order));
+                          d_idx, p.d_fallback, s.sum, nullptr, s.st, nullptr, x.order, o.order));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[4], s.st));
   return 0;
 }
@@ -936,7 +953,7 @@ int enqueue_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   if (p.x.on) return enqueue_cross(c, s, q, p, d_dist, d_idx, timing);
   HIP_TRY(c, launch_init_lists(p.L, fit.n, s.st));
   const DevFrames& R = ref_ops(c, q.nofit);
-  HIP_TRY(c, launch_eps(fit, R, p.kappa, p.eps2, s.n_cand, s.st));
+  HIP_TRY(c, launch_eps(fit, R, p.kappa, p.eps2, s.sum, s.st));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[2], s.st));
   if (p.sample) {
     // every p.sample-th reference pair, as one shared list over the phases;
@@ -957,7 +974,7 @@ int enqueue_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
                              nullptr, 0, nullptr, nullptr, p.ft));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
   HIP_TRY(c, launch_merge(c->ref, fit, c->w, p.L, p.eps2, q.k1, q.k_out, q.rank_off, q.nofit,
-                          d_dist, d_idx, p.d_fallback, s.n_cand, nullptr, s.st));
+                          d_dist, d_idx, p.d_fallback, s.sum, nullptr, s.st));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[4], s.st));
   return 0;
 }
@@ -1057,8 +1074,12 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
                        (size_t)(lm_pairs + 1) * sizeof(int) + 1024;
   // Room: the free device memory plus what the buffers already hold, less a
   // reserve for everything else; and the context's budget.
+  // (Buffers that are large enough already need no look at the device.)
   size_t free_b = 0, total_b = 0;
-  HIP_TRY(c, hipMemGetInfo(&free_b, &total_b));
+  if (s.ws_sym_bytes < sym_bytes || s.ws_lists_bytes < ent_bytes || s.ws_small_bytes < small)
+    HIP_TRY(c, hipMemGetInfo(&free_b, &total_b));
+  else
+    free_b = SIZE_MAX / 2;
   const size_t have = s.ws_sym_bytes + s.ws_lists_bytes + s.ws_small_bytes;
   const size_t reserve = size_t(2) << 30;
   auto fits = [&]() {
@@ -1087,7 +1108,6 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   L.ent = (uint2*)s.ws_lists;
   char* sp = (char*)s.ws_small;
   double* gmax_q = (double*)sp; sp += 256;
-  unsigned long long* msum = (unsigned long long*)sp; sp += 256;
   L.cnt = (int*)sp; sp += (size_t)n * nl * sizeof(int);
   L.ovf = (float*)sp; sp += (size_t)n * nl * sizeof(float);
   L.thr = (unsigned*)sp; sp += n * sizeof(unsigned);
@@ -1109,7 +1129,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
                                                    : kappa_data(c->prec, c->ref.natoms)) *
                        c->eps_scale;
   const DevFrames& R = ref_ops(c, q.nofit);
-  HIP_TRY(c, launch_eps_sym(fit, R, kappa, gmax_q, eps2, s.n_cand, s.st));
+  HIP_TRY(c, launch_eps_sym(fit, R, kappa, gmax_q, eps2, s.sum, s.st));
   HIP_TRY(c, hipEventRecord(s.ev[2], s.st));
   // landmark pass into the first lists' worth of the list workspace
   Lists LL = L;
@@ -1226,9 +1246,9 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   HIP_TRY(c, launch_contract(mref, mfit, LM, meps2, q.k1, phases, q.nofit, nullptr, grid, s.st,
                              &M, 0, filter ? &tiles : nullptr));
   HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
-  HIP_TRY(c, launch_mirror_sum(M, n, msum, s.st));
+  HIP_TRY(c, launch_mirror_sum(M, n, s.sum, s.st));
   HIP_TRY(c, launch_merge(c->ref, fit, c->w, LM, meps2, q.k1, q.k_out, q.rank_off, q.nofit, d_dist,
-                          d_idx, d_fallback, s.n_cand, (ordered && !canon) ? order : nullptr, s.st,
+                          d_idx, d_fallback, s.sum, (ordered && !canon) ? order : nullptr, s.st,
                           &M, canon ? order : nullptr, canon ? order : nullptr));
   HIP_TRY(c, hipEventRecord(s.ev[4], s.st));
   // pairs of the upper block triangle: fit block fb against frames from
@@ -1243,7 +1263,6 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   info->pairs_computed = pairs;
   info->symmetric = true;
   info->pairs_landmark = n * std::min<int64_t>(n, (int64_t)lm_pairs * 2 * kTile);
-  info->d_mirror_sum = msum;
   return 0;
 }
 
@@ -1414,7 +1433,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
   if (cv) {
     cs = s;
     cs.fit = DevFrames();
-    cs.n_cand = (int*)cv->take(sizeof(int));
+    cs.sum = (QuerySummary*)cv->take(sizeof(QuerySummary));
     if (xyz) {
       DevFrames& f = cs.fit;
       f.n = n_fit;
@@ -1432,7 +1451,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
       if (c->prec != kExact) f.op = (uint4*)cv->take(operand_bytes(f.prec, f.n_tiles, f.n_groups));
       const bool axes = c->ref_axes && !q.nofit;
       if (axes) f.rot = (double*)cv->take(rows * 9 * sizeof(double));
-      if (!cs.n_cand || !f.cen || !f.G || !f.Gt || (c->prec != kExact && !f.op) ||
+      if (!cs.sum || !f.cen || !f.G || !f.Gt || (c->prec != kExact && !f.op) ||
           (axes && !f.rot))
         return fail(c, MDSCTK_ERR_ARG,
                     "query (fixed workspace): %lld query frames of %d atoms do not fit the %zu-byte "
@@ -1496,14 +1515,10 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
     ms_fallback = elapsed(s.ev[2], s.ev[3]);
     S.n_fallback_rows = n_fit;
   } else {
-    std::vector<int> fb(n_fit);
-    int ncand = 0;
-    unsigned long long msum[2] = {0, 0};
-    HIP_TRY(c, hipMemcpyAsync(fb.data(), info.d_fallback, n_fit * sizeof(int),
-                              hipMemcpyDeviceToHost, s.st));
-    HIP_TRY(c, hipMemcpyAsync(&ncand, ws.n_cand, sizeof(int), hipMemcpyDeviceToHost, s.st));
-    if (info.d_mirror_sum)
-      HIP_TRY(c, hipMemcpyAsync(msum, info.d_mirror_sum, sizeof msum, hipMemcpyDeviceToHost, s.st));
+    // One small copy; the rows' flags only when one is set.  (Three copies, the
+    // flags among them, took 30 us each.)
+    QuerySummary sum;
+    HIP_TRY(c, hipMemcpyAsync(&sum, ws.sum, sizeof sum, hipMemcpyDeviceToHost, s.st));
     HIP_TRY(c, hipStreamSynchronize(s.st));
     if (info.symmetric) {
       S.ms_landmark = elapsed(s.ev[2], s.ev[6]);
@@ -1512,17 +1527,25 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
       ms_contract = elapsed(s.ev[2], s.ev[3]);
     }
     ms_merge = elapsed(s.ev[3], s.ev[4]);
-    S.n_candidates = ncand;
+    S.n_candidates = sum.n_cand;
     S.ref_splits = info.phases;
     S.list_capacity = info.cap;
     S.eps_rel = info.kappa;
     S.n_pairs_computed = info.pairs_computed;
     S.n_pairs_landmark = info.pairs_landmark;
-    S.n_mirrored = (int64_t)msum[0];
-    S.n_mirrored_max = (int64_t)msum[1];
+    if (info.symmetric) {
+      S.n_mirrored = (int64_t)sum.mirrored;
+      S.n_mirrored_max = (int64_t)sum.mirrored_max;
+    }
     std::vector<int> rows;
-    for (int64_t i = 0; i < n_fit; ++i)
-      if (fb[i]) rows.push_back((int)i);
+    if (sum.n_flagged > 0) {
+      std::vector<int> fb(n_fit);
+      HIP_TRY(c, hipMemcpyAsync(fb.data(), info.d_fallback, n_fit * sizeof(int),
+                                hipMemcpyDeviceToHost, s.st));
+      HIP_TRY(c, hipStreamSynchronize(s.st));
+      for (int64_t i = 0; i < n_fit; ++i)
+        if (fb[i]) rows.push_back((int)i);
+    }
     if (!rows.empty()) {
       HIP_TRY(c, hipEventRecord(s.ev[2], s.st));
       // rows of a symmetric self query whose mirrored list overflowed go
@@ -1542,7 +1565,15 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
       S.n_fallback_rows = (int64_t)rows.size();
     }
   }
-  if (!out_on_device) {
+  // Short outputs come back in one copy (they lie side by side) to a pinned
+  // buffer of the slot's, long ones straight to the caller's memory.
+  const size_t out_bytes = out_elems * (sizeof(double) + sizeof(int));
+  const bool pinned = !out_on_device && out_bytes <= kPinnedOut;
+  if (pinned && !s.h_out)
+    HIP_TRY(c, hipHostMalloc(&s.h_out, kPinnedOut, hipHostMallocDefault));
+  if (pinned) {
+    HIP_TRY(c, hipMemcpyAsync(s.h_out, d_dist, out_bytes, hipMemcpyDeviceToHost, s.st));
+  } else if (!out_on_device) {
     HIP_TRY(c, hipMemcpyAsync(out_dist, d_dist, out_elems * sizeof(double), hipMemcpyDeviceToHost,
                               s.st));
     HIP_TRY(c, hipMemcpyAsync(out_idx, d_idx, out_elems * sizeof(int), hipMemcpyDeviceToHost,
@@ -1550,6 +1581,10 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
   }
   HIP_TRY(c, hipEventRecord(s.ev[5], s.st));
   HIP_TRY(c, hipEventSynchronize(s.ev[5]));
+  if (pinned) {
+    std::memcpy(out_dist, s.h_out, out_elems * sizeof(double));
+    std::memcpy(out_idx, (char*)s.h_out + out_elems * sizeof(double), out_elems * sizeof(int));
+  }
   // While serving runs, a self query does not keep its mirrored lists: the
   // memory goes back to the serving slots' workspace.
   bool serving;

@@ -17,6 +17,9 @@
 
 namespace mdsctk {
 
+// Host outputs up to this size go through a pinned buffer.
+constexpr size_t kPinnedOut = size_t(1) << 20;
+
 // Device workspace of one query batch in flight: its stream, the query
 // frames and their derived arrays, candidate lists and device outputs.
 // Every buffer grows on demand and is reused by later batches.
@@ -31,7 +34,8 @@ struct Slot {
   size_t ws_lists_bytes = 0;
   void* ws_small = nullptr;
   size_t ws_small_bytes = 0;
-  int* n_cand = nullptr;
+  QuerySummary* sum = nullptr;  // device
+  void* h_out = nullptr;        // pinned, kPinnedOut bytes: short host outputs (on first use)
   void* ws_out = nullptr;
   size_t ws_out_bytes = 0;
   void* ws_rows = nullptr;
@@ -126,7 +130,6 @@ struct FusedInfo {
   // symmetric self query only
   bool symmetric = false;
   int64_t pairs_landmark = 0;  // pairs of its landmark pass (0: none)
-  unsigned long long* d_mirror_sum = nullptr;  // [2]: mirrored appends, most per frame
 };
 
 // Pieces of caller-provided device memory handed out in order, 256-byte
@@ -212,7 +215,7 @@ int slot_init(mdsctk_knn_ctx* c, Slot& s);
 void slot_release(mdsctk_knn_ctx* c, Slot& s);
 // Free the symmetric self query's mirrored lists, which the context
 // otherwise keeps for the next self query.  Called by the synchronous entry
-// points only (a new reference set; a query that is not a self query; the
+// points only (a reference set of another shape; a query that is not a self query; the
 // end of a self query while serving runs), so it never races a query that
 // uses them.
 void release_mirror_lists(mdsctk_knn_ctx* c);

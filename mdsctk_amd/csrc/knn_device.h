@@ -118,6 +118,13 @@ struct Lists {
   unsigned* thr = nullptr;    // [n_fit] shared threshold (float bits)
 };
 
+// What a query's kernels count: one small block, read back in one copy.
+struct QuerySummary {
+  int n_cand;     // candidates re-scored
+  int n_flagged;  // rows the merge could not certify
+  unsigned long long mirrored, mirrored_max;  // symmetric self query only
+};
+
 // The symmetric self query's second list per frame: the scores a frame
 // receives as the reference side of a pair contracted only the other way
 // round ([n][cap] entries, counters, smallest key dropped past cap).
@@ -249,9 +256,10 @@ hipError_t launch_prep(const DevFrames& f, const DevWeights& w, int side,
 // reset_thr false keeps the shared thresholds (a landmark pass set them).
 hipError_t launch_init_lists(const Lists& L, int64_t n_fit, hipStream_t st,
                              bool reset_thr = true);
-// eps2[q] = 2 kappa (Gt_fit[q] + *ref.gmax); *n_cand (if given) is set to 0.
+// eps2[q] = 2 kappa (Gt_fit[q] + *ref.gmax); the merge's counters in *sum (if
+// given) are set to 0.
 hipError_t launch_eps(const DevFrames& fit, const DevFrames& ref, double kappa, float* eps2,
-                      int* n_cand, hipStream_t st);
+                      QuerySummary* sum, hipStream_t st);
 // Approximate contraction into candidate lists.  When dbg_scores != nullptr
 // it instead writes the approximate score of every pair to
 // dbg_scores[fit*n_ref+ref] (small sizes).  With `mirror` (a self query: fit
@@ -274,7 +282,7 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
 // view): eps2[r] = 2 kappa max(G~q[r] + max G~ref, G~ref[r] + max G~q);
 // *gmax_q receives max G~q.
 hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kappa,
-                          double* gmax_q, float* eps2, int* n_cand, hipStream_t st);
+                          double* gmax_q, float* eps2, QuerySummary* sum, hipStream_t st);
 // After the landmark pass (lists L of n rows, reference phases `phases`):
 // thr[q] = the certified bound of row q's k1-th smallest key in the full
 // query, label[q] = its nearest landmark (dense, < 64 ceil(pairs / phases)).
@@ -291,9 +299,9 @@ hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* e
 hipError_t launch_row_order(const int* label, int64_t n, int nlab, int* counts, int* order,
                             hipStream_t st);
 hipError_t launch_mirror_init(const Mirror& m, int64_t n, hipStream_t st);
-// out[0] = total mirrored appends (including those dropped past cap), out[1] = max per frame.
-hipError_t launch_mirror_sum(const Mirror& m, int64_t n, unsigned long long* out,
-                             hipStream_t st);
+// out->mirrored = total mirrored appends (including those dropped past cap),
+// out->mirrored_max = most per frame.
+hipError_t launch_mirror_sum(const Mirror& m, int64_t n, QuerySummary* out, hipStream_t st);
 // dst[i] = frame rows[i] of src (natoms x 3 floats each).
 hipError_t launch_gather_frames(const float* src, const int* rows, int nrows, int natoms,
                                 float* dst, hipStream_t st);
@@ -309,7 +317,7 @@ hipError_t launch_scatter_rows(const double* sd, const int* si, const int* rows,
 hipError_t launch_merge(const DevFrames& ref, const DevFrames& fit, const DevWeights& w,
                         const Lists& L, const float* eps2, int k1, int k_out, int rank_off,
                         bool nofit, double* out_dist, int* out_idx, int* fallback,
-                        int* n_cand, const int* order, hipStream_t st,
+                        QuerySummary* sum, const int* order, hipStream_t st,
                         const Mirror* mirror = nullptr, const int* perm = nullptr,
                         const int* ref_perm = nullptr);
 // dst[i] = the float bits src[perm[i]] raised by add[i] (and one unit in the
