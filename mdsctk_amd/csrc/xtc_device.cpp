@@ -114,7 +114,9 @@ int mdsctk_xtc_read_device(const char* path, int32_t natoms, int device, float**
   hipError_t e;
   if ((e = hipSetDevice(device)) != hipSuccess) return hip_err(e, "hipSetDevice");
   if ((e = hipMalloc((void**)&h.d_file, size + 64)) != hipSuccess) return hip_err(e, "hipMalloc");
-  constexpr size_t kChunk = size_t(64) << 20;
+  // Two pinned chunks: pinning costs about as much per byte as reading, and
+  // smaller chunks start the upload earlier.
+  constexpr size_t kChunk = size_t(4) << 20;
   const size_t chunk = std::min(kChunk, (size + 4095) & ~size_t(4095));
   for (auto& p : h.pinned)
     if ((e = hipHostMalloc((void**)&p, chunk, hipHostMallocDefault)) != hipSuccess)
