@@ -626,6 +626,26 @@ int cross_stride(const mdsctk_knn_ctx* c, int k1) {
   return std::max(1, std::max(ref_pairs / want, ref_pairs * 2 * kTile / kFilterMaxCells + 1));
 }
 
+// Whether a query bounds its thresholds by a sample pass first: without a
+// threshold every pair of a row enters its lists until they fill, and each
+// list then bounds its own part of the row alone.
+// Short queries: kSampleMinRef.  Longer ones: the pass (1/16 of the
+// contraction and a cap kernel, 50 us at least) against the epilogue's work
+// on the pairs that it rejects.  Measured, bf16, whole query without -> with:
+//   8000 x 8000 x 100, k 32, fitted 2.38 -> 1.92 ms, --nofit 1.55 -> 1.17
+//   2000 x 8000 x 100, k 32, fitted .78 -> .59,      --nofit .79 -> .46
+//   1500 x 20000 x 100, k 4, fitted 1.17 -> .79,     --nofit .68 -> .67
+//   2000 x 8000 x 600, k 4,  fitted 1.33 -> 1.37,    --nofit 1.23 -> 1.33
+//   1500 x 20000 x 2000, k 32,                       --nofit 3.54 -> 3.31
+//   8000 x 2000 x 100, k 32, fitted 1.18 -> 1.23,    --nofit 1.05 -> 1.11
+//   400 x 4000 x 100, k 32,  fitted .21 -> .25,      --nofit .20 -> .23
+// Without a QCP to save, a short list (k below 11) gains nothing.
+bool sampled_query(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
+  if (n_fit < kCrossMinFit && c->ref.n >= kSampleMinRef) return true;
+  return c->ref.n >= 3000 && n_fit * c->ref.n >= 6000000 && c->ref.natoms <= 64 * q.k1 &&
+         (!q.nofit || q.k1 >= 12);
+}
+
 // The ordered form's workspace, carved from `cv` (or only its size).
 size_t carve_cross(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit, Carve& cv, CrossPlan* x) {
   const OrderedRef& o = c->ordered;
@@ -680,12 +700,12 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   p->grid = contract_grid(c, p->ft);
   p->phases = fused_phases(c, n_fit);
   auto ent_bytes_for = [&](int phases) { return (size_t)n_fit * phases * 4 * cap * sizeof(uint2); };
-  // A sample pass of short queries: 1/16 of the reference pairs, or enough
+  // A sample pass: 1/16 of the reference pairs, or enough
   // for 8 (k+1) frames.
   const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
   p->sample = 0;
   p->sample_pairs = 0;
-  if (n_fit < kCrossMinFit && c->ref.n >= kSampleMinRef) {
+  if (sampled_query(c, q, n_fit)) {
     const int want = std::max(ref_pairs / 16, 8 * q.k1 / (2 * kTile) + 1);
     p->sample = ref_pairs / want;
     if (p->sample < 4) p->sample = 0;  // too large a part of the query
@@ -1033,22 +1053,28 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   // its pairs as one list, split over enough phases to fill the grid
   const int lm_phases = std::max(1, std::min({phases, lm_pairs, 2 * grid / blocks}));
   const size_t ent_bytes = (size_t)n * nl * cap * sizeof(uint2);
-  // Canonical form (fitted scores of frames, kFilterMinFrames or more): the
-  // main pass runs over a copy of the set in landmark order, every frame in
+  // Canonical form (kFilterMinFrames frames or more): the main pass runs over
+  // a copy of the set in landmark order, for fitted scores with every frame in
   // its principal axes.  (Below that, ordering and copying cost more than the
-  // order saves: 105 us of the 2000-frame query.)  Frames near each other in the order are near each other in
-  // space, so most 32 x 32 tiles hold only far pairs, which the
-  // contraction's lambda_max bound rejects without the QCP; the axes make
-  // that bound nearly exact for similar frames.  The copy: operands (both
-  // dither sides), centroids, G, G~, rotations, windows, thresholds.
-  const bool canon = !q.nofit && c->w.metric == kMetricRMSD && n >= kFilterMinFrames;
+  // order saves: 105 us of the 2000-frame query.)  Frames near each other in
+  // the order are near each other in space, so a pass over each block's
+  // neighbours finds thresholds close to the final ones, and most 32 x 32
+  // tiles hold only far pairs: the tile filter drops them unread (fitted
+  // scores), the epilogue rejects theirs without a score.  The axes make the
+  // lambda_max bound nearly exact for similar frames.  The copy: operands
+  // (both dither sides), centroids, G, G~, rotations, windows, thresholds.
+  // 40007 vectors of 90 values, k 100, whose main pass went by the landmark
+  // thresholds before: main pass 6.4 -> 1.9 ms, merge 2.8 -> 1.75, for .3 ms
+  // of band pass and .3 of cap.
+  const bool fitted = !q.nofit && c->w.metric == kMetricRMSD;
+  bool canon = n >= kFilterMinFrames;
   const bool dith = c->ref.op_q != nullptr;
   const size_t rows = (size_t)c->ref.n_tiles * kTile;
   const size_t opb = operand_bytes(c->ref.prec, c->ref.n_tiles, c->ref.n_groups);
   const size_t perm_bytes =
       canon ? Carve::round(rows * 3 * sizeof(double)) + Carve::round(rows * sizeof(double)) * 2 +
                   (dith ? Carve::round(rows * sizeof(double)) + Carve::round(opb) : 0) +
-                  Carve::round(rows * 9 * sizeof(double)) + Carve::round(opb) +
+                  (fitted ? Carve::round(rows * 9 * sizeof(double)) : 0) + Carve::round(opb) +
                   Carve::round((size_t)n * sizeof(float)) +
                   Carve::round((size_t)n * sizeof(unsigned)) + 512
             : 0;
@@ -1058,17 +1084,19 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   const int fit_blocks = c->ref.n_tiles / kFilterFitTiles;
   const size_t tiles_n = (size_t)fit_blocks * ref_pairs;
   const size_t sort_temp = sort_order_scratch(n);
-  const size_t filter_bytes =
+  const size_t filter_set =
       Carve::round(filter_operand_bytes(fsh, c->ref.n_tiles)) + 2 * Carve::round(rows * sizeof(float4)) +
       Carve::round(rows * 12 * sizeof(double)) + Carve::round(rows * 36 * sizeof(ushort)) +
       Carve::round(fsh.natoms * 3 * sizeof(double)) + Carve::round(fsh.slots() * sizeof(int)) +
       Carve::round(12 * kFilterSamples * sizeof(double)) + Carve::round(sizeof(FilterMean)) +
-      Carve::round(tiles_n) + Carve::round(tiles_n * sizeof(int)) +
+      Carve::round(tiles_n);
+  const size_t filter_bytes =
+      (fitted ? filter_set : 0) + Carve::round(tiles_n * sizeof(int)) +
       Carve::round(fit_blocks * sizeof(int)) + Carve::round(2 * sizeof(int)) +
       3 * Carve::round((size_t)n * sizeof(int)) + Carve::round(sort_temp) +
       2 * Carve::round((size_t)nlab * sizeof(int));
-  bool filter = canon && n >= kFilterMinFrames;
-  size_t sym_bytes = Carve::round(mir_bytes) + perm_bytes + (filter ? filter_bytes : 0);
+  bool band = canon;  // order by cells, the band pass, and if fitted the filter
+  size_t sym_bytes = Carve::round(mir_bytes) + perm_bytes + (band ? filter_bytes : 0);
   const size_t small = (size_t)n * nl * (sizeof(int) + sizeof(float)) +
                        (size_t)n * 7 * sizeof(int) + (size_t)nlab * sizeof(int) +
                        (size_t)(lm_pairs + 1) * sizeof(int) + 1024;
@@ -1088,10 +1116,15 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     std::lock_guard<std::mutex> g(c->mem_mu);
     return !(c->budget && c->held - std::min(c->held, have) + need > c->budget);
   };
-  if (filter && !fits()) {  // every tile is contracted instead
-    filter = false;
+  if (band && !fits()) {  // every tile is contracted instead
+    band = false;
     sym_bytes = Carve::round(mir_bytes) + perm_bytes;
   }
+  if (canon && !fitted && !fits()) {  // over the set as it is
+    canon = false;
+    sym_bytes = Carve::round(mir_bytes);
+  }
+  const bool filter = band && fitted;
   if (!fits()) return 1;
   int rc = ensure(c, &s.ws_sym, &s.ws_sym_bytes, sym_bytes, "mirrored lists");
   if (!rc) rc = ensure(c, &s.ws_lists, &s.ws_lists_bytes, ent_bytes, "candidate lists");
@@ -1140,8 +1173,8 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
                              nullptr, 0, &lm));
   Carve fc;
   fc.base = (char*)s.ws_sym + Carve::round(mir_bytes) + perm_bytes;
-  fc.size = filter ? filter_bytes : 0;
-  if (filter) {
+  fc.size = band ? filter_bytes : 0;
+  if (band) {
     // rows in cells of about 6 (k+1) frames around every cell-th landmark,
     // by distance within a cell
     unsigned* keys = (unsigned*)fc.take((size_t)n * sizeof(int));
@@ -1166,7 +1199,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   // pays where candidate frames no longer fit the caches), and the canonical
   // form contracts the frames in it
   const bool ordered = n >= kFilterMinFrames;
-  if (ordered && !filter) HIP_TRY(c, launch_row_order(label, n, nlab, counts, order, s.st));
+  if (ordered && !band) HIP_TRY(c, launch_row_order(label, n, nlab, counts, order, s.st));
   // the main pass's frames, windows and thresholds
   DevFrames mref = R, mfit = fit;
   Lists LM = L;
@@ -1183,12 +1216,12 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     mref.op = (uint4*)cp.take(opb);
     mref.op_q = dith ? (uint4*)cp.take(opb) : nullptr;
     mref.Gt_q = dith ? (double*)cp.take(rows * sizeof(double)) : nullptr;
-    double* rot = (double*)cp.take(rows * 9 * sizeof(double));
+    double* rot = fitted ? (double*)cp.take(rows * 9 * sizeof(double)) : nullptr;
     meps2 = (float*)cp.take((size_t)n * sizeof(float));
     LM.thr = (unsigned*)cp.take((size_t)n * sizeof(unsigned));
     double* gm = (double*)cp.take(2 * sizeof(double));
     mref.gmax = gm;
-    if (!mref.cen || !mref.G || !mref.Gt || !mref.op || !rot || !meps2 || !LM.thr || !gm ||
+    if (!mref.cen || !mref.G || !mref.Gt || !mref.op || (fitted && !rot) || !meps2 || !LM.thr || !gm ||
         (dith && (!mref.op_q || !mref.Gt_q)))
       return fail(c, MDSCTK_ERR_ARG, "symmetric self query: canonical workspace carve");
     const DevFrames mq = query_view(mref);
@@ -1216,18 +1249,22 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     double* align = (double*)fc.take(12 * kFilterSamples * sizeof(double));
     fmean = (FilterMean*)fc.take(sizeof(FilterMean));
     tiles.flags = (unsigned char*)fc.take(tiles_n);
-    tiles.list = (int*)fc.take(tiles_n * sizeof(int));
-    tiles.count = (int*)fc.take(fit_blocks * sizeof(int));
-    tiles.ctrl = (int*)fc.take(2 * sizeof(int));
     if (!fset.op || !fset.full || !fset.pre || !fset.place || !fset.extra || !mean || !slots ||
-        !align || !fmean || !tiles.flags || !tiles.list || !tiles.count || !tiles.ctrl)
+        !align || !fmean || !tiles.flags)
       return fail(c, MDSCTK_ERR_ARG, "symmetric self query: filter workspace carve");
     DevFrames src = c->ref;
     HIP_TRY(c, launch_filter_mean(src, c->w, fsh, align, mean, fmean, slots, s.st));
     HIP_TRY(c, launch_filter_prep(src, c->w, fsh, mean, fmean, slots, order, fset, s.st));
+  }
+  if (band) {
     // A band pass over the neighbours in that order tightens the thresholds
-    // that the filter tests against: each block against the reference pairs
-    // around it, into the first 4 lists.
+    // that the filter and the epilogue test against: each block against the
+    // reference pairs around it, into the first 4 lists.
+    tiles.list = (int*)fc.take(tiles_n * sizeof(int));
+    tiles.count = (int*)fc.take(fit_blocks * sizeof(int));
+    tiles.ctrl = (int*)fc.take(2 * sizeof(int));
+    if (!tiles.list || !tiles.count || !tiles.ctrl)
+      return fail(c, MDSCTK_ERR_ARG, "symmetric self query: band workspace carve");
     Lists LB = LM;
     LB.nl = 4;
     HIP_TRY(c, launch_init_lists(LB, n, s.st, false));

@@ -577,6 +577,7 @@ struct ContractParams {
   const double* fGt;
   int64_t n_ref, n_fit;
   int ref_pairs, fit_tiles, n_groups, phases, k1;
+  int k_groups;  // K-groups that hold atoms (the others are padding)
   const float* eps2;
   uint2* ent;
   int* cnt;
@@ -803,7 +804,8 @@ __device__ __forceinline__ unsigned wave_select(const unsigned (&key)[PER], int 
   return low ? (t | ((1u << low) - 1u)) : t;
 }
 
-// Compact the lists of every lane whose list is nearly full, or holds 2 k1
+// Compact the lists of every lane whose list has no room for another `room`
+// entries (a tile's, at most 64), or holds 2 k1
 // entries while the lane has no threshold yet (a query without a bound from
 // elsewhere: the first compaction sets one early, so the row's other lists
 // stop taking every pair).  The whole wave
@@ -817,9 +819,9 @@ __device__ __forceinline__ unsigned wave_select(const unsigned (&key)[PER], int 
 template <int PER>
 __device__ __attribute__((noinline)) void compact_lists(uint2* __restrict__ ent, int64_t my_base, int& cnt,
                                               float& thr, float& ovf, float eps2, int k1,
-                                              int cap, bool active) {
+                                              int cap, bool active, int room) {
   const int lane = threadIdx.x & 63;
-  uint64_t need = __ballot(active && (cnt > cap - 16 || (cnt >= 2 * k1 && thr == INFINITY)));
+  uint64_t need = __ballot(active && (cnt > cap - room || (cnt >= 2 * k1 && thr == INFINITY)));
   while (need) {
     const int L = __builtin_ctzll(need);
     need &= need - 1;
@@ -868,7 +870,7 @@ __device__ __attribute__((noinline)) void compact_lists(uint2* __restrict__ ent,
       pos += __popcll(__ballot(kp[j]) & lanes_below);
     }
     // At most kcap entries survive (only the d == 0 case has more to drop):
-    // the list then has room for the next tile's 16 appends per lane.
+    // the list then has room for the next tile's appends.
     int wrote = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j)
@@ -904,29 +906,43 @@ __device__ __forceinline__ void stage_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Append this lane's mirrored score (pass: the key is below the reference
-// frame's threshold) to the reference frame's list.  For a fixed accumulator
-// element, the lanes of a half-wave hold the same reference frame (row) and
-// 32 different fit frames, so each half-wave reserves its slots with one
-// atomic add on that row's counter and its passing lanes write in lane
-// order.  b: the wave's ballot of pass.
+// Append a wave's mirrored scores of one 32 x 32 tile (16 elements a lane, row
+// 8 (r/4) + 4 (lane/32) + r%4 of the tile for element r) to the reference
+// frames' lists.  Lane 32 h + r holds in `mask` which lanes of its half of the
+// wave pass in element r, and reserves their slots with one atomic on that
+// row's counter: one round trip a tile.  (An atomic as each element came up
+// waited for up to 16 of them in turn.)
 __device__ __forceinline__ void mirror_append(uint2* __restrict__ ment, int* __restrict__ mcnt,
-                                              float* __restrict__ movf, int mcap, int64_t row,
-                                              bool pass, uint64_t b, float key,
+                                              float* __restrict__ movf, int mcap, int64_t ref_base,
+                                              unsigned mask, const float (&key)[16],
                                               unsigned other, int lane) {
-  const int h = lane >> 5;
-  const unsigned hb = h ? (unsigned)(b >> 32) : (unsigned)b;
-  const int lead = hb ? (int)__builtin_ctz(hb) + 32 * h : lane;
+  if (!__ballot(mask != 0)) return;
   int base = 0;
-  if (hb && lane == lead) base = atomicAdd(&mcnt[row], __builtin_popcount(hb));
-  base = __shfl(base, lead);
-  if (pass) {
-    const int pos = base + __builtin_popcount(hb & ((1u << (lane & 31)) - 1u));
-    if (pos < mcap)
-      ment[row * (int64_t)mcap + pos] = make_uint2(__float_as_uint(key), other);
-    else
-      atomicMin(reinterpret_cast<unsigned*>(&movf[row]), __float_as_uint(key));
+  if (mask)
+    base = atomicAdd(&mcnt[ref_base + 8 * ((lane & 15) >> 2) + 4 * (lane >> 5) + (lane & 3)],
+                     __builtin_popcount(mask));
+  const bool up = lane >= 32;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const unsigned m0 = __builtin_amdgcn_readlane(mask, r);
+    const unsigned m1 = __builtin_amdgcn_readlane(mask, 32 + r);
+    if (!(m0 | m1)) continue;
+    const unsigned m = up ? m1 : m0;
+    const int b = up ? __builtin_amdgcn_readlane(base, 32 + r) : __builtin_amdgcn_readlane(base, r);
+    if (m >> (lane & 31) & 1) {
+      const int pos = b + __builtin_popcount(m & ((1u << (lane & 31)) - 1u));
+      const int64_t row = ref_base + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+      if (pos < mcap)
+        ment[row * mcap + pos] = make_uint2(__float_as_uint(key[r]), other);
+      else
+        atomicMin(reinterpret_cast<unsigned*>(&movf[row]), __float_as_uint(key[r]));
+    }
   }
+}
+
+// Element r's part of that mask: b is the wave's ballot.
+__device__ __forceinline__ unsigned mirror_mask(uint64_t b, int r, int lane) {
+  return lane == r ? (unsigned)b : lane == 32 + r ? (unsigned)(b >> 32) : 0u;
 }
 
 // The pipelined K-loop's stage end: this wave's copies older than the N
@@ -1020,8 +1036,11 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
 
   const int rounds = (n_items + nwg - 1) / nwg;
   for (int round = 0; round < rounds; ++round) {
-    const int item = logical + round * nwg;
-    if (item >= n_items) break;
+    // kOutSym: an item's tiles decrease with its block, so odd rounds deal
+    // them out in reverse
+    const int turn = MODE == kOutSym && (round & 1) ? nwg - 1 - logical : logical;
+    const int item = turn + round * nwg;
+    if (item >= n_items) continue;
     const int fb = item / P.ph_run;
     const int ph = item - fb * P.ph_run;
     // Tile t of the item is reference pair ph + t R, or that entry of the
@@ -1202,6 +1221,8 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
         asm volatile("" : "+v"(mir));
         mirror = __builtin_amdgcn_readfirstlane(mir) != 0;
       }
+      float keys[16];
+      unsigned mir_mask = 0;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int rl = 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
@@ -1261,15 +1282,17 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
           }
         }
         if constexpr (MODE == kOutSym) {
+          keys[r] = key;
           const uint64_t b = __ballot(mir);
-          if (b)
-            mirror_append(P.ment, P.mcnt, P.movf, P.mcap, ref_idx, mir, b, key,
-                          (unsigned)fit_idx, lane);
+          if (b) mir_mask |= mirror_mask(b, r, lane);
         }
       }
+      if constexpr (MODE == kOutSym)
+        mirror_append(P.ment, P.mcnt, P.movf, P.mcap, ref_base, mir_mask, keys,
+                      (unsigned)fit_idx, lane);
       if constexpr (MODE == kOutLists || MODE == kOutSym) {
       const float thr_before = thr;
-      compact_lists<PER>(P.ent, my_base, cnt, thr, ovf, e2, P.k1, P.cap, fvalid);
+      compact_lists<PER>(P.ent, my_base, cnt, thr, ovf, e2, P.k1, P.cap, fvalid, 16);
       thr = fminf(thr, __shfl_xor(thr, 32));
       if (fvalid && P.thr && thr < thr_before) atomicMin(&P.thr[fit_idx], __float_as_uint(thr));
       }
@@ -1284,6 +1307,322 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
       P.ovf[hdr] = ovf;
     }
   }
+}
+
+// One plane of a K-group for a wave's 2 x 2 tiles: acc[2 i + j] += A_i * B_j^T,
+// the three split products in mma_group's order (the same sums, bit for bit).
+template <int PREC>
+__device__ __forceinline__ void trace_plane(f32x16 (&acc)[4], const uint4* __restrict__ As,
+                                            const uint4* __restrict__ Bs, int lane) {
+  uint4 a[2][2], b[2][2];  // [tile][hi, lo]
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      a[i][h] = As[(2 * i + h) * 64 + lane];
+      b[i][h] = Bs[(2 * i + h) * 64 + lane];
+    }
+#pragma unroll
+  for (int prod = 0; prod < 3; ++prod)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint4 av = a[i][prod == 2], bv = b[j][prod == 1];
+        if constexpr (PREC == kBF16)
+          acc[2 * i + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+              __builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, bv), acc[2 * i + j], 0, 0, 0);
+        else
+          acc[2 * i + j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+              __builtin_bit_cast(f16x8, av), __builtin_bit_cast(f16x8, bv), acc[2 * i + j], 0, 0, 0);
+      }
+}
+
+// The split forms' contraction where only the trace of the 3x3 block counts
+// (--nofit and data vectors): a plain product of 3 N values with a list
+// epilogue.  contract_kernel's shape, a 32x32 tile a wave, gives the trace 9
+// MFMAs per 12 KB read from LDS and 36 KB copied a K-group, and is bound by
+// those.  Here a wave holds 2 x 2 tiles (three accumulators each: one for all
+// three planes would triple the FP32 chain), 12 MFMAs per 8 KB; four waves,
+// two workgroups a CU, so that one's epilogue runs under the other's K-loop.
+// A stage is one plane of a K-group (16 KB, three buffers: stage 3 g + c in
+// buffer c), and groups of padding alone are left out.  The epilogue rejects
+// in FP32 with a slack and forms the FP64 score only where some lane passes.
+// Measured: 8191 x 30011 x 151 FP16 --nofit 2.2 -> 1.68 ms, and .95 ms (sample
+// pass included, .7 PFLOP/s) with thresholds from a sample; 40007 vectors of
+// 90 values against themselves 6.8 -> 6.4 ms by loose thresholds (bound by
+// the appends), 1.9 ms by the band pass's.
+template <int PREC, int PER, int MODE>
+__global__ __launch_bounds__(256, 2) void trace_kernel(ContractParams P) {
+  constexpr int SLOT = 2 * 64;       // 16-byte vectors of a tile's plane (hi, lo)
+  constexpr int STAGE = 8 * SLOT;    // reference tiles 0..3, fit tiles 0..3
+  constexpr int GROUP = 6 * 64;      // of a tile's K-group in the operand
+  constexpr int LPS = 4;             // copies of a wave per stage: 2 slots
+  __shared__ uint4 sbuf0[STAGE];
+  __shared__ uint4 sbuf1[STAGE];
+  __shared__ uint4 sbuf2[STAGE];
+  // The current and next tile's reference rows: G~; (1 - 2e-6) G~ / 2, +inf
+  // for rows past the set; for kOutSym the shared threshold (-1 in a tile that
+  // is not mirrored).
+  __shared__ double sGr[2][4 * kTile];
+  __shared__ float sHalf[2][4 * kTile];
+  __shared__ float sThr[2][4 * kTile];
+  __shared__ double sGf[4 * kTile];
+  __shared__ float sKey[MODE == kOutSym ? 4 : 1][16][64];  // mirrored scores of a wave's 32 x 32
+
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63;
+  const int ri = wave & 1;   // reference pair of the tile: slots 2 ri, 2 ri + 1
+  const int fi = wave >> 1;  // fit tiles 2 fi, 2 fi + 1 of the block
+  const int ng = P.n_groups;
+  const int n_ref = (int)P.n_ref;
+  const int fit_blocks = (int)((P.n_fit + 4 * kTile - 1) / (4 * kTile));
+  const int n_items = fit_blocks * P.phases;
+  const int nwg = gridDim.x;
+  const int logical = (int)(blockIdx.x & 7) * (nwg >> 3) + (int)(blockIdx.x >> 3);
+
+  // Wave w copies stage slots 2 w and 2 w + 1: its reference pair (waves 0
+  // and 1), or fit tiles 2 w - 4 and 2 w - 3.
+  uint4* const d0 = sbuf0 + 2 * wave * SLOT;
+  uint4* const d1 = sbuf1 + 2 * wave * SLOT;
+  uint4* const d2 = sbuf2 + 2 * wave * SLOT;
+
+  const int rounds = (n_items + nwg - 1) / nwg;
+  for (int round = 0; round < rounds; ++round) {
+    // kOutSym: an item's tiles decrease with its block, so odd rounds deal
+    // them out in reverse
+    const int turn = MODE == kOutSym && (round & 1) ? nwg - 1 - logical : logical;
+    const int item = turn + round * nwg;
+    if (item >= n_items) continue;
+    const int fb = item / P.phases;
+    const int ph = item - fb * P.phases;
+    // Tile t of the item is the two reference pairs 2 u, 2 u + 1 of the list
+    // (or of all), u = ph + t phases; past an odd list's end the last pair
+    // is read again and counts as past the set.
+    const int lb = P.tblock * (fb * 4 / kFilterFitTiles);
+    const int* const tlist = P.tlist ? P.tlist + (int64_t)lb * P.ref_pairs : nullptr;
+    const int n_pairs = P.tlist ? P.tcount[lb] : P.ref_pairs;
+    const int n_tiles = ((n_pairs + 1) / 2 - ph + P.phases - 1) / P.phases;
+    auto pair_of = [&](int t) -> int {
+      const int u = min(2 * (ph + t * P.phases) + ri, n_pairs - 1);
+      return tlist ? __builtin_amdgcn_readfirstlane(tlist[u]) : u;
+    };
+    auto real_pair = [&](int t) -> bool { return 2 * (ph + t * P.phases) + ri < n_pairs; };
+    int t0 = 0;
+    if constexpr (MODE == kOutSym)  // the first tile at or after the fit block
+      if (fb > ph) t0 = (fb - ph + P.phases - 1) / P.phases;
+    if (t0 >= n_tiles) continue;  // its list headers were cleared
+
+    const int64_t fit0 = (int64_t)(4 * fb + 2 * fi) * kTile + (lane & 31);  // j = 0; + 32: j = 1
+    const int list_id = (ph * 2 + ri) * 2 + (lane >> 5);
+    uint2* list[2];
+    float hg[2], thr[2], ovf[2];
+    int cnt[2];
+    bool fvalid[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t q = fit0 + j * kTile;
+      fvalid[j] = q < P.n_fit;
+      list[j] = P.ent + (q * P.nl + list_id) * P.cap;
+      hg[j] = fvalid[j] ? (float)(0.5 * (1.0 - 2e-6) * P.fGt[q]) : INFINITY;
+      thr[j] = ovf[j] = INFINITY;
+      cnt[j] = 0;
+    }
+
+    // stage c of K-group g of the current tile (p_cur), or for g = k_groups
+    // of the next one's first group; past the item's last tile its own again
+    int p_cur = pair_of(t0);
+    int p_next = t0 + 1 < n_tiles ? pair_of(t0 + 1) : p_cur;
+    auto copy = [&](int g, int c, uint4* dst) {
+      const bool over = g >= P.k_groups;
+      const int64_t tile = wave < 2 ? (int64_t)2 * (over ? p_next : p_cur)
+                                    : (int64_t)4 * fb + 2 * (wave - 2);
+      const uint4* const base = wave < 2 ? P.rop : P.fop;
+      const uint4* const src = base + (tile * ng + (over ? 0 : g)) * GROUP + c * SLOT + lane;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          __builtin_amdgcn_global_load_lds((const void*)(src + (int64_t)i * ng * GROUP + h * 64),
+                                           (lds_void_t*)(dst + i * SLOT + h * 64), 16, 0, 0);
+    };
+    // The rows of tile t's pair ri = wave (waves 0 and 1), read and published.
+    double g_row = 0.0;
+    float half_row = INFINITY, thr_row = -1.0f;
+    auto read_rows = [&](int t, int p) {
+      if (wave < 2) {
+        const int64_t r = (int64_t)p * 2 * kTile + lane;
+        const bool in = real_pair(t) && r < P.n_ref;
+        g_row = P.rGt[r];
+        half_row = in ? (float)(0.5 * (1.0 - 2e-6) * g_row) : INFINITY;
+        if constexpr (MODE == kOutSym)
+          thr_row = in && ph + t * P.phases > fb ? __uint_as_float(P.thr[r]) : -1.0f;
+      }
+    };
+    auto put_rows = [&](int t) {
+      if (wave < 2) {
+        sGr[t & 1][tid] = g_row;
+        sHalf[t & 1][tid] = half_row;
+        if constexpr (MODE == kOutSym) sThr[t & 1][tid] = thr_row;
+      }
+    };
+
+    __syncthreads();  // the previous item's readers are done
+    read_rows(t0, p_cur);
+    put_rows(t0);
+    if (tid < 4 * kTile) sGf[tid] = P.fGt[(int64_t)4 * fb * kTile + tid];
+    copy(0, 0, d0);
+    copy(0, 1, d1);
+    stage_barrier<LPS>();  // stage 0 landed
+
+    for (int t = t0; t < n_tiles; ++t) {
+      // read here, used at the end of the tile
+      if (t + 1 < n_tiles) read_rows(t + 1, p_next);
+      unsigned shared[2] = {kInfBits, kInfBits};
+      if (P.thr)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          if (fvalid[j]) shared[j] = __builtin_nontemporal_load(&P.thr[fit0 + j * kTile]);
+
+      f32x16 ax[4], ay[4], az[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) ax[q] = ay[q] = az[q] = (f32x16){0};
+      // Stage 3 g + c is computed from buffer c while the next one lands; the
+      // copy of the one after goes into the buffer that every wave finished
+      // reading before the last barrier.
+      for (int g = 0; g < P.k_groups; ++g) {
+        trace_plane<PREC>(ax, sbuf0 + 2 * ri * SLOT, sbuf0 + (4 + 2 * fi) * SLOT, lane);
+        copy(g, 2, d2);
+        stage_barrier<LPS>();
+        trace_plane<PREC>(ay, sbuf1 + 2 * ri * SLOT, sbuf1 + (4 + 2 * fi) * SLOT, lane);
+        copy(g + 1, 0, d0);
+        stage_barrier<LPS>();
+        trace_plane<PREC>(az, sbuf2 + 2 * ri * SLOT, sbuf2 + (4 + 2 * fi) * SLOT, lane);
+        copy(g + 1, 1, d1);
+        stage_barrier<LPS>();
+      }
+      // read by the next tile's epilogue, after at least one more barrier
+      if (t + 1 < n_tiles) put_rows(t + 1);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) thr[j] = fminf(thr[j], __uint_as_float(shared[j]));
+
+      // kOutSym: a tile past the fit block is contracted only this way round
+      const bool mirror = MODE == kOutSym && ph + t * P.phases > fb;
+      // (less the rows of the tile's pairs before this wave's)
+      const int ref_base = (real_pair(t) ? 2 * p_cur * kTile : n_ref) - 2 * ri * kTile;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          unsigned mask = 0;
+          // opaque: the compiler would keep the other fit tile's rows of the
+          // same values in registers, and spill them
+          int row0 = 2 * ri * kTile + i * kTile + 4 * (lane >> 5);
+          asm volatile("" : "+v"(row0));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int row = row0 + 8 * (r >> 2) + (r & 3);
+            const float mx = ax[2 * i + j][r], my = ay[2 * i + j][r], mz = az[2 * i + j][r];
+            // s = G_r + G_f - 2 t > every threshold, t = m_x + m_y + m_z:
+            // |m_x| + |m_y| + |m_z| <= 0.51 (G_r + G_f), so with a threshold up
+            // to 4 (G_r + G_f) the FP32 roundings of both sides come to less
+            // than 4e-7 (G_r + G_f), and the factor of the halves leaves
+            // 1e-6; with a larger one t is far above the limit.  An infinite
+            // threshold or a NaN on either side passes.
+            float rej = thr[j];
+            if constexpr (MODE == kOutSym) rej = fmaxf(rej, sThr[t & 1][row]);
+            const float limit = sHalf[t & 1][row] + fmaf(-0.5f, rej, hg[j]);
+            const bool pass = MODE == kOutDebug || !((mx + my) + mz < limit);
+            if (!__ballot(pass)) continue;
+            const int ref_idx = ref_base + row;
+            const bool valid = pass && fvalid[j] && ref_idx < n_ref;
+            const double s = sGr[t & 1][row] + sGf[(2 * fi + j) * kTile + (lane & 31)] -
+                             2.0 * ((double)mx + (double)my + (double)mz);
+            if constexpr (MODE == kOutDebug) {
+              if (valid) P.dbg[(fit0 + j * kTile) * P.n_ref + ref_idx] = s;
+              continue;
+            }
+            const float key = (float)fmax(s, 0.0);
+            if (valid && s <= (double)thr[j]) {
+              // never dropped: the compaction leaves room for a tile's 32
+              if (cnt[j] < P.cap) {
+                list[j][cnt[j]] = make_uint2(__float_as_uint(key), (unsigned)ref_idx);
+                ++cnt[j];
+              } else {
+                ovf[j] = fminf(ovf[j], key);
+              }
+            }
+            if constexpr (MODE == kOutSym) {
+              // (an approximate score can be below -1)
+              const bool mir = valid && mirror && s <= (double)sThr[t & 1][row];
+              const uint64_t b = __ballot(mir);
+              if (b) {
+                mask |= mirror_mask(b, r, lane);
+                sKey[wave][r][lane] = key;
+              }
+            }
+          }
+          if constexpr (MODE == kOutSym) {
+            // as mirror_append, the keys from LDS (registers are short here)
+            uint64_t rows = __ballot(mask != 0);
+            if (!rows) continue;
+            const int64_t tile0 = ref_base + 2 * ri * kTile + i * kTile;
+            int base = 0;
+            if (mask)
+              base = atomicAdd(
+                  &P.mcnt[tile0 + 8 * ((lane & 15) >> 2) + 4 * (lane >> 5) + (lane & 3)],
+                  __builtin_popcount(mask));
+            for (unsigned m16 = (unsigned)(rows | rows >> 32) & 0xffffu; m16; m16 &= m16 - 1) {
+              const int r = __builtin_ctz(m16);
+              const unsigned m = __shfl(mask, (lane & 32) + r);
+              const int pos0 = __shfl(base, (lane & 32) + r);
+              if (m >> (lane & 31) & 1) {
+                const int pos = pos0 + __builtin_popcount(m & ((1u << (lane & 31)) - 1u));
+                const int64_t row = tile0 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                const unsigned kb = __float_as_uint(sKey[wave][r][lane]);
+                if (pos < P.mcap)
+                  P.ment[row * P.mcap + pos] = make_uint2(kb, (unsigned)(fit0 + j * kTile));
+                else
+                  atomicMin(reinterpret_cast<unsigned*>(&P.movf[row]), kb);
+              }
+            }
+          }
+        }
+      }
+      if constexpr (MODE != kOutDebug) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const int64_t q = fit0 + j * kTile;
+          const float before = thr[j];
+          // (copies: the call takes their addresses)
+          int n = cnt[j];
+          float th = before, ov = ovf[j];
+          const bool act = fvalid[j];
+          if (__ballot(act && (n > P.cap - 32 || (n >= 2 * P.k1 && th == INFINITY)))) {
+            const float e2 = act && P.eps2 ? P.eps2[q] : 0.f;
+            compact_lists<PER>(P.ent, list[j] - P.ent, n, th, ov, e2, P.k1, P.cap, act, 32);
+            cnt[j] = n;
+            ovf[j] = ov;
+          }
+          thr[j] = fminf(th, __shfl_xor(th, 32));
+          if (act && P.thr && thr[j] < before) atomicMin(&P.thr[q], __float_as_uint(thr[j]));
+        }
+      }
+      p_cur = p_next;
+      if (t + 2 < n_tiles) p_next = pair_of(t + 2);
+    }
+    if constexpr (MODE != kOutDebug) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (fvalid[j]) {
+          const int64_t hdr = (fit0 + j * kTile) * P.nl + list_id;
+          P.cnt[hdr] = cnt[j];
+          P.ovf[hdr] = ovf[j];
+        }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the copies past the last tile have landed
 }
 
 // The bin of a 256-bin histogram that holds the rank-th (0-based) of its
@@ -2538,6 +2877,7 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
   P.ref_pairs = ref.n_tiles / kRefTilesPerWG;
   P.fit_tiles = fit.n_tiles;
   P.n_groups = ref.n_groups;
+  P.k_groups = (ref.natoms + group_atoms(ref.prec) - 1) / group_atoms(ref.prec);
   P.phases = ref_phases;
   P.k1 = k1;
   P.eps2 = eps2;
@@ -2575,65 +2915,72 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
 #define MDSCTK_CONTRACT(PR, PER, FT, MODE, TR)                                            \
   hipLaunchKernelGGL((contract_kernel<PR, PER, FT, MODE, TR>), grid,                        \
                      dim3(64 * kRefTilesPerWG * FT), 0, st, P)
-#define MDSCTK_CONTRACT_TR(PR, PER, FT, MODE)     \
+#define MDSCTK_FULL(PR, PER, FT, MODE) MDSCTK_CONTRACT(PR, PER, FT, MODE, false)
+#define MDSCTK_EITHER(PR, PER, FT, MODE)          \
   do {                                            \
     if (nofit)                                    \
       MDSCTK_CONTRACT(PR, PER, FT, MODE, true);   \
     else                                          \
       MDSCTK_CONTRACT(PR, PER, FT, MODE, false);  \
   } while (0)
-#define MDSCTK_CONTRACT_CAP(PR, FT)                 \
-  do {                                              \
-    if (dbg_scores)                                 \
-      MDSCTK_CONTRACT_TR(PR, 4, FT, kOutDebug);     \
-    else if (near)                                  \
-      MDSCTK_CONTRACT(PR, 4, FT, kOutNear, false);  \
-    else if (mirror && L.cap == 256)                \
-      MDSCTK_CONTRACT_TR(PR, 4, FT, kOutSym);       \
-    else if (mirror && L.cap == 512)                \
-      MDSCTK_CONTRACT_TR(PR, 8, FT, kOutSym);       \
-    else if (mirror && L.cap == 1024)               \
-      MDSCTK_CONTRACT_TR(PR, 16, FT, kOutSym);      \
-    else if (mirror)                                \
-      return hipErrorInvalidValue;                  \
-    else if (L.cap == 256)                          \
-      MDSCTK_CONTRACT_TR(PR, 4, FT, kOutLists);     \
-    else if (L.cap == 512)                          \
-      MDSCTK_CONTRACT_TR(PR, 8, FT, kOutLists);     \
-    else if (L.cap == 1024)                         \
-      MDSCTK_CONTRACT_TR(PR, 16, FT, kOutLists);    \
-    else                                            \
-      return hipErrorInvalidValue;                  \
-  } while (0)
-#define MDSCTK_CONTRACT_SMALL(PR)                   \
+#define MDSCTK_TRACE(PR, PER, FT, MODE) \
+  hipLaunchKernelGGL((trace_kernel<PR, PER, MODE>), grid, dim3(256), 0, st, P)
+#define MDSCTK_LISTS(LAUNCH, PR, FT, MODE)          \
   do {                                              \
     if (L.cap == 256)                               \
-      MDSCTK_CONTRACT_TR(PR, 4, 1, kOutLists);      \
+      LAUNCH(PR, 4, FT, MODE);                      \
     else if (L.cap == 512)                          \
-      MDSCTK_CONTRACT_TR(PR, 8, 1, kOutLists);      \
+      LAUNCH(PR, 8, FT, MODE);                      \
     else if (L.cap == 1024)                         \
-      MDSCTK_CONTRACT_TR(PR, 16, 1, kOutLists);     \
+      LAUNCH(PR, 16, FT, MODE);                     \
     else                                            \
       return hipErrorInvalidValue;                  \
   } while (0)
-  if (ft == 1) {
-    if (dbg_scores || near || mirror || (tiles && !tiles->shared)) return hipErrorInvalidValue;
-    switch (ref.prec) {
-      case kBF16: MDSCTK_CONTRACT_SMALL(kBF16); break;
-      case kFP16: MDSCTK_CONTRACT_SMALL(kFP16); break;
-      default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+#define MDSCTK_MODES(LAUNCH, PR, FT)                \
+  do {                                              \
+    if (dbg_scores)                                 \
+      LAUNCH(PR, 4, FT, kOutDebug);                 \
+    else if (mirror)                                \
+      MDSCTK_LISTS(LAUNCH, PR, FT, kOutSym);        \
+    else                                            \
+      MDSCTK_LISTS(LAUNCH, PR, FT, kOutLists);      \
+  } while (0)
+#define MDSCTK_SPLIT(PR)                                  \
+  do {                                                    \
+    if (ft == 1)                                          \
+      MDSCTK_LISTS(MDSCTK_EITHER, PR, 1, kOutLists);      \
+    else if (near)                                        \
+      MDSCTK_FULL(PR, 4, 4, kOutNear);                    \
+    else if (nofit)                                       \
+      MDSCTK_MODES(MDSCTK_TRACE, PR, 4);                  \
+    else                                                  \
+      MDSCTK_MODES(MDSCTK_FULL, PR, 4);                   \
+  } while (0)
+  if (ft == 1 && (ref.prec == kFP32 || dbg_scores || near || mirror || (tiles && !tiles->shared)))
+    return hipErrorInvalidValue;
+  if (nofit && ft != 1 && ref.prec != kFP32) {
+    // trace_kernel: reference pairs in twos, all phases, two workgroups a CU
+    if (ph_run || ref.n_tiles % 4 || fit.n_tiles % 4 || (tiles && mirror))
+      return hipErrorInvalidValue;
+    grid = dim3(2 * grid_wgs);
   }
   switch (ref.prec) {
-    case kFP32: MDSCTK_CONTRACT_CAP(kFP32, 2); break;
-    case kBF16: MDSCTK_CONTRACT_CAP(kBF16, 4); break;
-    case kFP16: MDSCTK_CONTRACT_CAP(kFP16, 4); break;
+    case kFP32:
+      if (near)
+        MDSCTK_FULL(kFP32, 4, 2, kOutNear);
+      else
+        MDSCTK_MODES(MDSCTK_EITHER, kFP32, 2);
+      break;
+    case kBF16: MDSCTK_SPLIT(kBF16); break;
+    case kFP16: MDSCTK_SPLIT(kFP16); break;
     default: return hipErrorInvalidValue;
   }
-#undef MDSCTK_CONTRACT_CAP
-#undef MDSCTK_CONTRACT_SMALL
-#undef MDSCTK_CONTRACT_TR
+#undef MDSCTK_SPLIT
+#undef MDSCTK_MODES
+#undef MDSCTK_LISTS
+#undef MDSCTK_TRACE
+#undef MDSCTK_EITHER
+#undef MDSCTK_FULL
 #undef MDSCTK_CONTRACT
   return hipGetLastError();
 }
