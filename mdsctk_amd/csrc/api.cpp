@@ -626,6 +626,80 @@ int cross_stride(const mdsctk_knn_ctx* c, int k1) {
   return std::max(1, std::max(ref_pairs / want, ref_pairs * 2 * kTile / kFilterMaxCells + 1));
 }
 
+int groups_of(int64_t n) { return (int)((n + 2 * kTile - 1) / (2 * kTile)); }
+
+// The middles of n frames; dith: with a query-side operand as well.
+void carve_middles(const mdsctk_knn_ctx* c, int64_t n, bool dith, Carve& cv, MiddleSet* m) {
+  const int groups = groups_of(n);
+  DevFrames f;
+  f.n = groups;
+  f.natoms = c->ref.natoms;
+  f.n_tiles = f.cap_tiles = std::max(kTileAlign, padded_tiles(groups));
+  f.n_groups = c->ref.n_groups;
+  f.prec = c->ref.prec;
+  f.owns_xyz = false;
+  const size_t rows = (size_t)f.n_tiles * kTile;
+  const size_t opb = operand_bytes(f.prec, f.n_tiles, f.n_groups);
+  f.cen = (double*)cv.take(rows * 3 * sizeof(double));
+  f.G = (double*)cv.take(rows * sizeof(double));
+  f.Gt = (double*)cv.take(rows * sizeof(double));
+  f.op = (uint4*)cv.take(opb);
+  f.rot = (double*)cv.take(rows * 9 * sizeof(double));
+  if (dith) {
+    f.Gt_q = (double*)cv.take(rows * sizeof(double));
+    f.op_q = (uint4*)cv.take(opb);
+  }
+  m->f = f;
+  m->mid = (int*)cv.take(groups * sizeof(int));
+  m->ball = (float2*)cv.take(groups * sizeof(float2));
+}
+
+size_t middles_bytes(const mdsctk_knn_ctx* c, int64_t n, bool dith) {
+  Carve cv;
+  cv.base = (char*)256;  // sizes only
+  cv.size = SIZE_MAX / 2;
+  MiddleSet m;
+  carve_middles(c, n, dith, cv, &m);
+  return cv.used;
+}
+
+// The middles' operands (of `side`, and the query side where they have one)
+// and balls; src: the frames as given, order their order, thr and eps2 the
+// ordered rows' thresholds and windows (null on a side without).
+int enqueue_middles(mdsctk_knn_ctx* c, const DevFrames& src, const int* order, int side,
+                    const unsigned* thr, const float* eps2, const MiddleSet& m, hipStream_t st) {
+  HIP_TRY(c, launch_middle(order, src.n, m.mid, st));
+  const DevFrames q = query_view(m.f);
+  HIP_TRY(c, launch_prep(m.f, c->w, side, m.f.op_q ? &q : nullptr, -1, st, src.xyz, m.mid, m.f.rot));
+  HIP_TRY(c, launch_balls(src, c->w, order, m.mid, thr, eps2, m.ball, st));
+  return 0;
+}
+
+// The ball test of `rows` fit frames (or one middle) of a block each against
+// the reference middles, into flags [blocks][pairs of the reference set].
+int enqueue_ball_test(mdsctk_knn_ctx* c, const MiddleSet& ref, const DevFrames& fit,
+                      const float2* ball, int rows, int64_t tiles, unsigned char* flags,
+                      hipStream_t st) {
+  const int ft = contract_fit_tiles(c->prec);
+  const int grid = contract_grid(c, ft);
+  Lists none;
+  none.nl = 4;
+  none.cap = 256;
+  const int pairs = ref.f.n_tiles / kRefTilesPerWG;
+  const int phases = std::max(1, std::min(pairs, 2 * grid * ft / fit.n_tiles));
+  BallTest b;
+  b.fit = ball;
+  b.ref = ref.ball;
+  b.kappa2 = 2.0 * kappa_for(c->prec, c->ref.natoms);
+  b.rows = rows;
+  b.pairs = c->ref.n_tiles / kRefTilesPerWG;
+  b.flags = flags;
+  HIP_TRY(c, launch_clear_flags(flags, tiles, st));
+  HIP_TRY(c, launch_contract(ref.f, fit, none, nullptr, 1, phases, false, nullptr, grid, st, nullptr,
+                             0, nullptr, nullptr, 0, &b));
+  return 0;
+}
+
 // Whether a query bounds its thresholds by a sample pass first: without a
 // threshold every pair of a row enters its lists until they fill, and each
 // list then bounds its own part of the row alone.
@@ -839,7 +913,7 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   HIP_TRY(c, launch_permute_thresholds(x.thr0, x.order, p.eps2, n, p.L.thr, s.st));
   HIP_TRY(c, launch_init_lists(p.L, n, s.st, false));
   HIP_TRY(c, launch_filter(o.set, x.set, c->ref.n, n, c->ref.n_tiles, x.fit.n_tiles, o.sh, o.mc,
-                           p.L.thr, p.eps2, false, x.filter_grid, x.tiles, s.st));
+                           p.L.thr, p.eps2, false, x.filter_grid, x.tiles, nullptr, s.st));
   HIP_TRY(c, launch_contract(R, x.fit, p.L, p.eps2, q.k1, p.phases, false, nullptr, p.grid, s.st,
                              nullptr, 0, &x.tiles));
   if (timing) HIP_TRY(c, hipEventRecord(s.ev[3], s.st));
@@ -1084,12 +1158,14 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   const int fit_blocks = c->ref.n_tiles / kFilterFitTiles;
   const size_t tiles_n = (size_t)fit_blocks * ref_pairs;
   const size_t sort_temp = sort_order_scratch(n);
+  const bool by_rows = n <= kBallRowsMax;
   const size_t filter_set =
       Carve::round(filter_operand_bytes(fsh, c->ref.n_tiles)) + 2 * Carve::round(rows * sizeof(float4)) +
       Carve::round(rows * 12 * sizeof(double)) + Carve::round(rows * 36 * sizeof(ushort)) +
       Carve::round(fsh.natoms * 3 * sizeof(double)) + Carve::round(fsh.slots() * sizeof(int)) +
       Carve::round(12 * kFilterSamples * sizeof(double)) + Carve::round(sizeof(FilterMean)) +
-      Carve::round(tiles_n);
+      2 * Carve::round(tiles_n) + middles_bytes(c, n, dith) +
+      (by_rows ? Carve::round((size_t)n * sizeof(float2)) : 0);
   const size_t filter_bytes =
       (fitted ? filter_set : 0) + Carve::round(tiles_n * sizeof(int)) +
       Carve::round(fit_blocks * sizeof(int)) + Carve::round(2 * sizeof(int)) +
@@ -1277,9 +1353,25 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   HIP_TRY(c, launch_init_lists(LM, n, s.st, false));
   HIP_TRY(c, launch_mirror_init(M, n, s.st));
   HIP_TRY(c, hipEventRecord(s.ev[6], s.st));
-  if (filter)
+  if (filter) {
+    MiddleSet m;
+    carve_middles(c, n, dith, fc, &m);
+    auto* near_tiles = (unsigned char*)fc.take(tiles_n);
+    auto* rball = by_rows ? (float2*)fc.take((size_t)n * sizeof(float2)) : nullptr;
+    if (!m.ball || !near_tiles || (by_rows && !rball))
+      return fail(c, MDSCTK_ERR_ARG, "symmetric self query: middles carve");
+    rc = enqueue_middles(c, c->ref, order, dith ? +1 : 0, LM.thr, meps2, m, s.st);
+    if (!rc && by_rows) {
+      HIP_TRY(c, launch_row_balls(LM.thr, meps2, n, rball, s.st));
+      rc = enqueue_ball_test(c, m, mfit, rball, kFilterFitTiles * kTile, tiles_n, near_tiles, s.st);
+    } else if (!rc) {
+      rc = enqueue_ball_test(c, m, query_view(m.f), m.ball, kFilterFitTiles / kRefTilesPerWG, tiles_n,
+                             near_tiles, s.st);
+    }
+    if (rc) return rc;
     HIP_TRY(c, launch_filter(fset, fset, n, n, c->ref.n_tiles, c->ref.n_tiles, fsh, fmean, LM.thr,
-                             meps2, true, std::max(8, c->n_cu & ~7), tiles, s.st));
+                             meps2, true, std::max(8, c->n_cu & ~7), tiles, near_tiles, s.st));
+  }
   HIP_TRY(c, launch_contract(mref, mfit, LM, meps2, q.k1, phases, q.nofit, nullptr, grid, s.st,
                              &M, 0, filter ? &tiles : nullptr));
   HIP_TRY(c, hipEventRecord(s.ev[3], s.st));

@@ -68,6 +68,14 @@ struct QueryShape {
 // cells around landmarks, their contraction operand and their filter operand
 // (filter_kernels.hip).  Made once, when queries have brought enough frames
 // to pay for it; only read afterwards.
+// The middle frames of every 64 of an ordered set, as frames of their own,
+// and the balls around them (BallTest).
+struct MiddleSet {
+  DevFrames f;
+  int* mid = nullptr;
+  float2* ball = nullptr;
+};
+
 struct OrderedRef {
   bool built = false, failed = false;
   int64_t seen = 0;  // query frames since the set became resident

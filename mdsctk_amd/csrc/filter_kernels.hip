@@ -597,6 +597,9 @@ struct FilterParams {
   int ref_pairs, fit_blocks, phases;
   const unsigned* thr;
   const float* eps2;
+  // the reference pairs to test, per fit block (rows of ref_pairs entries)
+  const int* list;
+  const int* count;
   unsigned char* flags;
   const int* ctrl;
   int part;
@@ -680,18 +683,18 @@ __global__ __launch_bounds__(512, 2) void filter_kernel(FilterParams P) {
     const int bi = item / P.phases;
     const int ph = item - bi * P.phases;
     const int fb = part_block(bi, P.part);
-    const int n_tiles = (P.ref_pairs - ph + P.phases - 1) / P.phases;
-    int t0 = 0;
-    if constexpr (SYM) {
-      const int p_min = fb * FT / kRefTilesPerWG;
-      if (p_min > ph) t0 = (p_min - ph + P.phases - 1) / P.phases;
-    }
-    if (t0 >= n_tiles) continue;
+    const int n_tiles = (P.count[fb] - ph + P.phases - 1) / P.phases;
+    if (n_tiles <= 0) continue;
+    const int* const list = P.list + (int64_t)fb * P.ref_pairs + ph;
     unsigned char* const flags = P.flags + (int64_t)fb * P.ref_pairs;
     if (skip) {
-      for (int t = t0 + tid; t < n_tiles; t += 512) flags[ph + t * P.phases] = 1;
+      for (int t = tid; t < n_tiles; t += 512) flags[list[t * P.phases]] = 1;
       continue;
     }
+    auto pair_of = [&](int t) -> int {
+      return __builtin_amdgcn_readfirstlane(list[min(t, n_tiles - 1) * P.phases]);
+    };
+    int p = pair_of(0), p_next = pair_of(1);
     const int64_t fit_idx = (int64_t)(FT * fb + fi) * kTile + (lane & 31);
     const float4 ff = P.ffull[fit_idx], fp = P.fpre[fit_idx];
     const float tf = threshold(fit_idx, P.n_fit);
@@ -703,12 +706,12 @@ __global__ __launch_bounds__(512, 2) void filter_kernel(FilterParams P) {
     int misses = 0, hold = 0;
 
     const uint4* const fit_base = P.fop + (int64_t)(FT * fb + slot - kRefTilesPerWG) * tile_vec;
-    auto dma = [&](int t, int s, uint4* dst) {
+    // stage s of reference pair q
+    auto dma = [&](int q, int s, uint4* dst) {
       if (!copier) return;
-      if (t >= n_tiles) t = n_tiles - 1;
       const bool ref = wave < kRefTilesPerWG;
       const uint4* const base =
-          ref ? P.rop + (int64_t)(kRefTilesPerWG * (ph + t * P.phases) + wave) * tile_vec : fit_base;
+          ref ? P.rop + (int64_t)(kRefTilesPerWG * q + wave) * tile_vec : fit_base;
 #pragma unroll
       for (int u = 0; u < GPS; ++u) {
         int g = s * GPS + u;
@@ -727,26 +730,25 @@ __global__ __launch_bounds__(512, 2) void filter_kernel(FilterParams P) {
 
     __syncthreads();  // previous item's readers are done
     if (tid < 2 * kTile) {
-      const int64_t f0 = (int64_t)(ph + t0 * P.phases) * 2 * kTile + tid;
-      sRow[t0 & 1][0][tid] = P.rpre[f0];
-      sRow[t0 & 1][1][tid] = P.rfull[f0];
-      sT[t0 & 1][tid] = SYM ? threshold(f0, P.n_ref) : -FLT_MAX;
+      const int64_t f0 = (int64_t)p * 2 * kTile + tid;
+      sRow[0][0][tid] = P.rpre[f0];
+      sRow[0][1][tid] = P.rfull[f0];
+      sT[0][tid] = SYM ? threshold(f0, P.n_ref) : -FLT_MAX;
     }
-    dma(t0, 0, d0);
-    dma(t0, 1, d1);
-    dma(t0, 2, d2);
+    dma(p, 0, d0);
+    dma(p, 1, d1);
+    dma(p, 2, d2);
     fence_barrier<BPG>();
     uint4 bA[3], bB[3], a;
 #pragma unroll
     for (int d = 0; d < 3; ++d) bA[d] = b0[d * 64 + lane];
     a = a0[lane];
 
-    for (int t = t0; t < n_tiles; ++t) {
-      const int p = ph + t * P.phases;
+    for (int t = 0; t < n_tiles; ++t) {
       float4 next_pre = make_float4(0, 0, 0, 0), next_full = make_float4(0, 0, 0, 0);
       float next_t = -FLT_MAX;
       if (tid < 2 * kTile && t + 1 < n_tiles) {
-        const int64_t f1 = (int64_t)(p + P.phases) * 2 * kTile + tid;
+        const int64_t f1 = (int64_t)p_next * 2 * kTile + tid;
         next_pre = P.rpre[f1];
         next_full = P.rfull[f1];
         if constexpr (SYM) next_t = threshold(f1, P.n_ref);
@@ -762,18 +764,18 @@ __global__ __launch_bounds__(512, 2) void filter_kernel(FilterParams P) {
       auto run = [&](int s0, int s1) {
         for (int s = s0; s < s1; s += 4) {
           const bool more = s + 4 < s1;
-          const int tn = more ? t : t + 1, sn = more ? s + 4 : 0;
+          const int pn = more ? p : p_next, sn = more ? s + 4 : 0;
           stage_step<GPS>(acc, a0, b0, a1, b1, bA, bB, a, lane);
-          dma(t, s + 3, d3);
+          dma(p, s + 3, d3);
           stage_end<BPG>();
           stage_step<GPS>(acc, a1, b1, a2, b2, GPS == 1 ? bB : bA, GPS == 1 ? bA : bB, a, lane);
-          dma(tn, sn, d0);
+          dma(pn, sn, d0);
           stage_end<BPG>();
           stage_step<GPS>(acc, a2, b2, a3, b3, bA, bB, a, lane);
-          dma(tn, sn + 1, d1);
+          dma(pn, sn + 1, d1);
           stage_end<BPG>();
           stage_step<GPS>(acc, a3, b3, a0, b0, GPS == 1 ? bB : bA, GPS == 1 ? bA : bB, a, lane);
-          dma(tn, sn + 2, d2);
+          dma(pn, sn + 2, d2);
           stage_end<BPG>();
         }
       };
@@ -820,9 +822,9 @@ __global__ __launch_bounds__(512, 2) void filter_kernel(FilterParams P) {
           // the buffers hold the next tile's first stages: fill them again
           // with this tile's second segment
           fence_barrier<0>();
-          dma(t, ns0, d0);
-          dma(t, ns0 + 1, d1);
-          dma(t, ns0 + 2, d2);
+          dma(p, ns0, d0);
+          dma(p, ns0 + 1, d1);
+          dma(p, ns0 + 2, d2);
 #pragma unroll
           for (int q = 0; q < 9; ++q) {
             const float cq = P.mc->C[1][q];
@@ -845,12 +847,23 @@ __global__ __launch_bounds__(512, 2) void filter_kernel(FilterParams P) {
         sRow[(t + 1) & 1][1][tid] = next_full;
         sT[(t + 1) & 1][tid] = next_t;
       }
+      p = p_next;
+      p_next = pair_of(t + 2);
     }
   }
 }
 
+// The middle frame of each 64 (the frames of a reference pair): its index
+// among the frames as given.
+__global__ void middle_kernel(const int* __restrict__ order, int64_t n, int groups,
+                              int* __restrict__ mid) {
+  const int g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (g < groups) mid[g] = order[min((int64_t)g * 2 * kTile + kTile, n - 1)];
+}
+
 // One workgroup per fit block of a part: its flagged reference pairs in
-// ascending order; ctrl[0/1] += flagged / tested pairs (part 0).
+// ascending order, in place of the tested ones; ctrl[0/1] += flagged / tested
+// pairs (part 0).  flags null: all of them.
 __global__ __launch_bounds__(256) void filter_list_kernel(const unsigned char* __restrict__ flags,
                                                           int ref_pairs, int fit_blocks, int part,
                                                           int sym_step, int* __restrict__ list,
@@ -858,14 +871,15 @@ __global__ __launch_bounds__(256) void filter_list_kernel(const unsigned char* _
                                                           int* __restrict__ ctrl) {
   const int fb = part_block(blockIdx.x, part);
   if (fb >= fit_blocks) return;
-  const unsigned char* const f = flags + (int64_t)fb * ref_pairs;
+  const unsigned char* const f = flags ? flags + (int64_t)fb * ref_pairs : nullptr;
   int* const out = list + (int64_t)fb * ref_pairs;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   __shared__ int part_n[4];
+  const int tested = count[fb];
   int base = 0;
   for (int p0 = fb * sym_step; p0 < ref_pairs; p0 += 256) {
     const int p = p0 + tid;
-    const bool on = p < ref_pairs && f[p];
+    const bool on = p < ref_pairs && (!f || f[p]);
     const uint64_t b = __ballot(on);
     if (lane == 0) part_n[wave] = __popcll(b);
     __syncthreads();
@@ -879,7 +893,7 @@ __global__ __launch_bounds__(256) void filter_list_kernel(const unsigned char* _
     count[fb] = base;
     if (part == 0) {
       atomicAdd(&ctrl[0], base);
-      atomicAdd(&ctrl[1], ref_pairs - fb * sym_step);
+      atomicAdd(&ctrl[1], tested);
     }
   }
 }
@@ -1049,7 +1063,7 @@ hipError_t launch_filter_prep(const DevFrames& f, const DevWeights& w, const Fil
 hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_ref, int64_t n_fit,
                          int ref_tiles, int fit_tiles, const FilterShape& sh, const FilterMean* mc,
                          const unsigned* thr, const float* eps2, bool sym, int grid,
-                         const TileList& tl, hipStream_t st) {
+                         const TileList& tl, const unsigned char* test, hipStream_t st) {
   constexpr int FT = 4;
   FilterParams P;
   P.rop = ref.op;
@@ -1066,6 +1080,8 @@ hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_r
   P.fit_blocks = fit_tiles / FT;
   P.thr = thr;
   P.eps2 = eps2;
+  P.list = tl.list;
+  P.count = tl.count;
   P.flags = tl.flags;
   P.ctrl = tl.ctrl;
   if (ref_tiles % kRefTilesPerWG || fit_tiles % FT || grid < 8 || (grid & 7))
@@ -1073,6 +1089,9 @@ hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_r
   const int64_t vec = ((int64_t)P.fit_blocks * P.ref_pairs + 15) / 16;
   hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((vec + 255) / 256)), dim3(256), 0, st,
                      reinterpret_cast<uint4*>(tl.flags), vec, tl.ctrl);
+  hipLaunchKernelGGL(filter_list_kernel, dim3((unsigned)P.fit_blocks), dim3(256), 0, st, test,
+                     P.ref_pairs, P.fit_blocks, 2, sym ? FT / kRefTilesPerWG : 0, tl.list, tl.count,
+                     tl.ctrl);
   // The sample costs two launches: from 64 blocks on.  Phases so that every
   // workgroup gets about four items, of eight tiles or more.
   for (int part = P.fit_blocks >= 64 ? 0 : 2; part < 3; part += part == 1 ? 2 : 1) {
@@ -1095,6 +1114,20 @@ hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_r
                        P.ref_pairs, P.fit_blocks, part, sym ? FT / kRefTilesPerWG : 0, tl.list,
                        tl.count, tl.ctrl);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_clear_flags(unsigned char* flags, int64_t n, hipStream_t st) {
+  const int64_t vec = (n + 15) / 16;
+  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((vec + 255) / 256)), dim3(256), 0, st,
+                     reinterpret_cast<uint4*>(flags), vec, (int*)nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_middle(const int* order, int64_t n, int* mid, hipStream_t st) {
+  const int groups = (int)((n + 2 * kTile - 1) / (2 * kTile));
+  hipLaunchKernelGGL(middle_kernel, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, st, order,
+                     n, groups, mid);
   return hipGetLastError();
 }
 

@@ -161,6 +161,13 @@ constexpr int64_t kCrossMinFit = 256;
 // Cells the rows are sorted into (13 bits of the sort key, above 19 bits of
 // the distance).
 constexpr int kFilterMaxCells = 8000;
+// The ball test takes a self query's rows one by one up to this many frames
+// (a contraction of 1/64 of its pairs), the middles of 64 beyond, where 64
+// frames lie closer together and the rows would cost what they save.  30000 x
+// 150, states: filter 1.60 ms without the test, 1.55 + .07 ms of test by
+// middles, .59 + .27 by rows (one basin: .3 ms of 13 in vain); 200000 x 1000
+// by middles: 91 -> 31 + 1.1 ms, where rows would take some 25.
+constexpr int64_t kBallRowsMax = 65536;
 constexpr int kFilterDistBits = 19;
 
 // How a frame's atoms are laid out: one or two segments, each a whole number
@@ -204,7 +211,30 @@ struct TileList {
   bool shared = false;  // one list for every block
 };
 
+// The test that comes before the filter (kOutBall): balls of the fit frames
+// (or of their middles) and of the middles of every 64 reference frames: a
+// radius and the square root of the largest threshold; twice the form's error
+// bound; flags[fit / rows][pairs] is set where a candidate is possible.
+struct BallTest {
+  const float2* fit = nullptr;
+  const float2* ref = nullptr;
+  double kappa2 = 0;
+  int rows = 1;
+  int pairs = 0;
+  unsigned char* flags = nullptr;
+};
+
 // Launchers (all asynchronous on `st`).
+// mid[g] = the frame in the middle of the g-th 64 of the order.
+hipError_t launch_middle(const int* order, int64_t n, int* mid, hipStream_t st);
+// ball[g] = (radius of the g-th 64 frames of the order around mid[g]: an upper
+// bound of sqrt(score); square root of the largest thr + eps2 / 2 of their
+// rows, 0 without thr).
+hipError_t launch_balls(const DevFrames& f, const DevWeights& w, const int* order, const int* mid,
+                        const unsigned* thr, const float* eps2, float2* ball, hipStream_t st);
+hipError_t launch_row_balls(const unsigned* thr, const float* eps2, int64_t n, float2* ball,
+                            hipStream_t st);
+hipError_t launch_clear_flags(unsigned char* flags, int64_t n, hipStream_t st);
 // The mean structure of the set (sqrt(w) scaled, [natoms][3]), its FilterMean
 // and the slot map (shape.slots() ints); scratch: 12 kFilterSamples doubles.
 hipError_t launch_filter_mean(const DevFrames& f, const DevWeights& w, const FilterShape& sh,
@@ -215,11 +245,12 @@ hipError_t launch_filter_prep(const DevFrames& f, const DevWeights& w, const Fil
                               const double* mean, const FilterMean* mc, const int* slots,
                               const int* perm, const FilterSet& out, hipStream_t st);
 // The tiles with a pair that may lie within thr[fit] + eps2[fit] / 2 (sym: or
-// the reference frame's), into tl.
+// the reference frame's), into tl.  test (if given): only the tiles flagged
+// there, [fit blocks][pairs].
 hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_ref, int64_t n_fit,
                          int ref_tiles, int fit_tiles, const FilterShape& sh, const FilterMean* mc,
                          const unsigned* thr, const float* eps2, bool sym, int grid,
-                         const TileList& tl, hipStream_t st);
+                         const TileList& tl, const unsigned char* test, hipStream_t st);
 // Each fit block of ft tiles against the `width` reference pairs around it.
 hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, const TileList& tl,
                             hipStream_t st);
@@ -272,12 +303,14 @@ hipError_t launch_eps(const DevFrames& fit, const DevFrames& ref, double kappa, 
 // kFilterFitTiles fit tiles, dealt out over the phases.  near: no lists, only
 // each fit frame's smallest (key << 32 | reference) there (atomic minimum).
 // ft 1: the one-fit-tile workgroup of short queries (contract_fit_tiles).
+// ball: no lists, only the flags of that test.
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st,
                            const Mirror* mirror = nullptr, int ph_run = 0,
                            const TileList* tiles = nullptr,
-                           unsigned long long* near = nullptr, int ft = 0);
+                           unsigned long long* near = nullptr, int ft = 0,
+                           const BallTest* ball = nullptr);
 // The window of a symmetric self query (fit: the reference set's query
 // view): eps2[r] = 2 kappa max(G~q[r] + max G~ref, G~ref[r] + max G~q);
 // *gmax_q receives max G~q.

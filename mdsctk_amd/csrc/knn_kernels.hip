@@ -604,6 +604,7 @@ struct ContractParams {
   const int* tcount;
   int tblock;
   unsigned long long* near;  // kOutNear: [n_fit] key bits << 32 | reference
+  BallTest ball;             // kOutBall
 };
 
 // What the contraction's epilogue produces.
@@ -618,6 +619,17 @@ constexpr int kOutDebug = 1;  // every score in FP64 (dbg, n_fit x n_ref)
 // written.
 constexpr int kOutSym = 2;
 constexpr int kOutNear = 3;  // each fit frame's nearest reference (key, index) only
+// The tiles that can hold a candidate, from one reference frame per 64: with
+// sqrt(s) a metric, R the radius of the 64 around their middle frame c, and a
+// fit frame (or the middle of a ball of them) q,
+//   sqrt(s(a, b)) >= sqrt(s(q, c)) - R_q - R_c
+// for every a, b of theirs, so the tile is flagged unless that is above the
+// larger of the sides' thresholds.  The form's error bound is taken off the
+// score twice over; a NaN or an infinity on the way flags the tile.
+// One score stands for 4096 pairs (for 64, a row at a time): 200000 frames of
+// 50 states x 1000 atoms spend .56 ms here and .5 ms on the balls, and the tile
+// filter takes 31 ms instead of 91.  One basin without states keeps all tiles.
+constexpr int kOutBall = 4;
 
 // One K-group of MFMA work for a wave: acc[c*3+d] += A_c * B_d^T over the
 // group's atoms, reading the wave's fragments from LDS.  For the split forms
@@ -1079,6 +1091,9 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     const float e2 = (fvalid && P.eps2) ? P.eps2[fit_idx] : 0.f;
     int cnt = 0;
     unsigned near_idx = 0;  // kOutNear: the reference whose key is thr
+    float2 fit_ball = make_float2(0.f, 0.f);
+    if constexpr (MODE == kOutBall)
+      if (fvalid) fit_ball = P.ball.fit[fit_idx];
     float thr = INFINITY, ovf = INFINITY;
 
     // Stage s of this item is K-group g = s % ngs of tile t = t0 + s / ngs.  Wave
@@ -1232,6 +1247,17 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
 #pragma unroll
         for (int q = 0; q < 9; ++q) m[q] = acc[q][r];
         const double gr = gr_tile[ri * kTile + rl];
+        if constexpr (MODE == kOutBall) {
+          if (valid) {
+            const float2 rb = P.ball.ref[ref_idx];
+            const double lim = (double)fit_ball.x + (double)rb.x + (double)fmaxf(fit_ball.y, rb.y);
+            const double rej = lim * lim * (1.0 + 1e-9) + P.ball.kappa2 * (gr + gf);
+            if (!(gr + gf - 2.0 * (double)lambda_upper(m) - 1e-9 * (gr + gf) > rej) &&
+                !(qcp_score_approx(m, gr, gf, rej, false) > rej))
+              P.ball.flags[fit_idx / P.ball.rows * P.ball.pairs + ref_idx] = 1;
+          }
+          continue;
+        }
         if constexpr (MODE == kOutDebug) {
           if (valid)
             P.dbg[fit_idx * P.n_ref + ref_idx] = qcp_score_approx(m, gr, gf, INFINITY, P.nofit);
@@ -1302,7 +1328,7 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
     if constexpr (MODE == kOutNear) {
       if (fvalid && thr < INFINITY)
         atomicMin(&P.near[fit_idx], ((unsigned long long)__float_as_uint(thr) << 32) | near_idx);
-    } else if (fvalid && MODE != kOutDebug) {
+    } else if (fvalid && MODE != kOutDebug && MODE != kOutBall) {
       P.cnt[hdr] = cnt;
       P.ovf[hdr] = ovf;
     }
@@ -1737,6 +1763,46 @@ __device__ __forceinline__ void group_cross(const float* __restrict__ a,
 __device__ __forceinline__ double cross_score(const double* S, double ga, double gb, bool nofit) {
   const double lam = nofit ? (S[0] + S[4] + S[8]) : qcp_lambda_exact(S, ga, gb);
   return fmax(ga + gb - 2.0 * lam, 0.0);
+}
+
+// One workgroup per 64 frames of an order: ball[g] = an upper bound of
+// sqrt(score) of each of them and the middle one, and the square root of the
+// largest threshold (with its window's half) of their rows.  16 lanes a frame;
+// bound by reading the frames once.
+__global__ __launch_bounds__(256) void ball_kernel(
+    const float* __restrict__ xyz, const double* __restrict__ cen, const double* __restrict__ G,
+    const float* __restrict__ w, int natoms, int64_t n, const int* __restrict__ order,
+    const int* __restrict__ mid, const unsigned* __restrict__ thr,
+    const float* __restrict__ eps2, float2* __restrict__ ball) {
+  const int tid = threadIdx.x, grp = tid >> 4;
+  const int64_t f0 = (int64_t)blockIdx.x * 2 * kTile;
+  const int64_t m = mid[blockIdx.x];
+  double far = 0.0;
+  bool known = true;
+  for (int j = grp; j < 2 * kTile && f0 + j < n; j += 16) {
+    const int64_t a = order[f0 + j];
+    double S[9];
+    group_cross<false>(xyz + a * natoms * 3, xyz + m * natoms * 3, cen + 3 * m, w, natoms, S);
+    const double g2 = G[a] + G[m];
+    const double s = cross_score(S, G[a], G[m], false) + 1e-9 * g2;
+    known = known && g2 < INFINITY && s >= 0.0;  // false for a NaN
+    far = fmax(far, s);
+  }
+  float big = 0.f;
+  if (thr && tid < 2 * kTile && f0 + tid < n)
+    big = __uint_as_float(thr[f0 + tid]) + 0.5f * eps2[f0 + tid];
+  __shared__ double sfar[16];
+  __shared__ float sbig[2 * kTile];
+  if ((tid & 15) == 0) sfar[grp] = known ? far : INFINITY;
+  if (tid < 2 * kTile) sbig[tid] = big;
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < 16; ++i) far = fmax(far, sfar[i]);
+    far = fmax(far, sfar[0]);
+    for (int i = 1; i < 2 * kTile; ++i) big = fmaxf(big, sbig[i]);
+    // (both rounded up)
+    ball[blockIdx.x] = make_float2((float)(sqrt(far) * (1.0 + 1e-6)), sqrtf(big) * (1.0f + 1e-6f));
+  }
 }
 
 // Exact FP64 score of one pair of data vectors (a: reference, b: query),
@@ -2866,7 +2932,8 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
 hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lists& L,
                            const float* eps2, int k1, int ref_phases, bool nofit,
                            double* dbg_scores, int grid_wgs, hipStream_t st, const Mirror* mirror,
-                           int ph_run, const TileList* tiles, unsigned long long* near, int ft) {
+                           int ph_run, const TileList* tiles, unsigned long long* near, int ft,
+                           const BallTest* ball) {
   ContractParams P;
   P.rop = ref.op;
   P.fop = fit.op;
@@ -2898,6 +2965,13 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
   P.tcount = tiles ? tiles->count : nullptr;
   P.tblock = tiles && tiles->shared ? 0 : 1;
   P.near = near;
+  P.ball = BallTest();
+  if (ball) {
+    P.ball = *ball;
+    if (near || nofit || mirror || tiles || dbg_scores || ball->rows < 1 || !ball->fit ||
+        !ball->ref || !ball->flags || ball->pairs < ref.n)
+      return hipErrorInvalidValue;
+  }
   if (near && (nofit || mirror || tiles || dbg_scores)) return hipErrorInvalidValue;
   if (tiles && (!tiles->list || !tiles->count || ph_run || fit.n_tiles % kFilterFitTiles ||
                 (mirror && tiles->shared)))
@@ -2951,12 +3025,14 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
       MDSCTK_LISTS(MDSCTK_EITHER, PR, 1, kOutLists);      \
     else if (near)                                        \
       MDSCTK_FULL(PR, 4, 4, kOutNear);                    \
+    else if (ball)                                        \
+      MDSCTK_FULL(PR, 4, 4, kOutBall);                    \
     else if (nofit)                                       \
       MDSCTK_MODES(MDSCTK_TRACE, PR, 4);                  \
     else                                                  \
       MDSCTK_MODES(MDSCTK_FULL, PR, 4);                   \
   } while (0)
-  if (ft == 1 && (ref.prec == kFP32 || dbg_scores || near || mirror || (tiles && !tiles->shared)))
+  if (ft == 1 && (ref.prec == kFP32 || dbg_scores || near || ball || mirror || (tiles && !tiles->shared)))
     return hipErrorInvalidValue;
   if (nofit && ft != 1 && ref.prec != kFP32) {
     // trace_kernel: reference pairs in twos, all phases, two workgroups a CU
@@ -2968,6 +3044,8 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
     case kFP32:
       if (near)
         MDSCTK_FULL(kFP32, 4, 2, kOutNear);
+      else if (ball)
+        MDSCTK_FULL(kFP32, 4, 2, kOutBall);
       else
         MDSCTK_MODES(MDSCTK_EITHER, kFP32, 2);
       break;
@@ -3084,6 +3162,30 @@ hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* e
   }
   hipLaunchKernelGGL(landmark_cap_kernel, dim3((unsigned)n), dim3(256), 0, st, L.ent, L.cnt, L.nl,
                      L.cap, k1, eps2, phases, thr, label, cell, keys, rows, leaders, leader_rank);
+  return hipGetLastError();
+}
+
+// ball[q] = (0, the square root of row q's threshold with its window's half).
+__global__ void row_ball_kernel(const unsigned* __restrict__ thr, const float* __restrict__ eps2,
+                                int64_t n, float2* __restrict__ ball) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n)
+    ball[q] = make_float2(0.f, sqrtf(__uint_as_float(thr[q]) + 0.5f * eps2[q]) * (1.0f + 1e-6f));
+}
+
+hipError_t launch_row_balls(const unsigned* thr, const float* eps2, int64_t n, float2* ball,
+                            hipStream_t st) {
+  hipLaunchKernelGGL(row_ball_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, thr, eps2,
+                     n, ball);
+  return hipGetLastError();
+}
+
+hipError_t launch_balls(const DevFrames& f, const DevWeights& w, const int* order, const int* mid,
+                        const unsigned* thr, const float* eps2, float2* ball, hipStream_t st) {
+  if (f.n <= 0) return hipSuccess;
+  if (w.metric != kMetricRMSD || (thr && !eps2)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(ball_kernel, dim3((unsigned)((f.n + 2 * kTile - 1) / (2 * kTile))), dim3(256), 0,
+                     st, f.xyz, f.cen, f.G, w.w, f.natoms, f.n, order, mid, thr, eps2, ball);
   return hipGetLastError();
 }
 
