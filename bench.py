@@ -20,6 +20,7 @@ import argparse
 import ctypes
 import json
 import os
+import re
 import sys
 import time
 
@@ -397,8 +398,9 @@ COPY_PROBE_BYTES = 1 << 30
 
 
 def _pmc_child(counter, child_args, tag, workdir):
-    """One `rocprofv3 --pmc <counter>` pass over a child bench.py run; returns
-    {dispatch: (kernel name, summed counter value)} or None."""
+    """One `rocprofv3 --pmc <counter>` pass over a child bench.py run (several
+    counters, space-separated, are added up); returns {dispatch: (kernel name,
+    summed counter value)} or None."""
     import csv
     import shutil
     import subprocess
@@ -406,7 +408,7 @@ def _pmc_child(counter, child_args, tag, workdir):
     if not os.path.exists(prof):
         return None
     out = os.path.join(workdir, tag)
-    cmd = ["timeout", "-s", "KILL", "240", prof, "--pmc", counter, "--output-format", "csv",
+    cmd = ["timeout", "-s", "KILL", "240", prof, "--pmc", *counter.split(), "--output-format", "csv",
            "-d", out, "-o", "run", "--", sys.executable, os.path.abspath(__file__)] + child_args
     env = dict(os.environ, TMPDIR="/tmp")
     p = subprocess.run(cmd, cwd="/tmp", env=env, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
@@ -415,7 +417,7 @@ def _pmc_child(counter, child_args, tag, workdir):
         return None
     res = {}
     for r in csv.DictReader(open(path)):
-        if r["Counter_Name"] != counter:
+        if r["Counter_Name"] not in counter.split():
             continue
         d = int(r["Dispatch_Id"])
         name, v = res.get(d, (r["Kernel_Name"], 0.0))
@@ -423,10 +425,25 @@ def _pmc_child(counter, child_args, tag, workdir):
     return res
 
 
+MFMA_COUNTERS = " ".join("SQ_INSTS_VALU_MFMA_MOPS_" + t for t in ("BF16", "F16", "F32"))
+MFMA_OP_FLOPS = 512  # of one count
+
+
+def _in_contraction(name, symmetric):
+    """Is this kernel part of the span that ms_contract times: the main
+    contraction and, for the symmetric query, the ball test and the tile filter
+    that choose its tiles?  (contract_kernel's fourth argument is its mode.)"""
+    m = re.search(r"contract_kernel<\w+, \w+, \w+, (\d+),", name)
+    if m:
+        return m.group(1) in (("2", "4") if symmetric else ("0",))
+    return symmetric and "filter_kernel<" in name
+
+
 def measure_traffic(args):
-    """HBM bytes per launch of the headline contraction: FETCH_SIZE and
-    WRITE_SIZE (KiB per dispatch, one rocprofv3 --pmc pass each), each scaled
-    by what the same counter reads for a plain 1 GiB device copy."""
+    """HBM bytes and matrix operations per query of the headline contraction:
+    FETCH_SIZE and WRITE_SIZE (KiB per dispatch, one rocprofv3 --pmc pass
+    each), each scaled by what the same counter reads for a plain 1 GiB device
+    copy, and the matrix cores' operation counters."""
     import tempfile
     work = tempfile.mkdtemp(prefix="mdsctk_pmc_", dir="/tmp")
     probe = ["--copy-probe", str(COPY_PROBE_BYTES)]
@@ -435,7 +452,8 @@ def measure_traffic(args):
              "--self-symmetric", str(args.self_symmetric)]
     r = {}
     for tag, counter, a in (("copy_fetch", "FETCH_SIZE", probe), ("copy_write", "WRITE_SIZE", probe),
-                            ("fetch", "FETCH_SIZE", child), ("write", "WRITE_SIZE", child)):
+                            ("fetch", "FETCH_SIZE", child), ("write", "WRITE_SIZE", child),
+                            ("mfma", MFMA_COUNTERS, child)):
         log(f"traffic pass {tag} ...")
         r[tag] = _pmc_child(counter, a, tag, work)
         if r[tag] is None:
@@ -443,24 +461,30 @@ def measure_traffic(args):
             return None, None
     copy_f = [v for n, v in r["copy_fetch"].values() if "copyBuffer" in n]
     copy_w = [v for n, v in r["copy_write"].values() if "copyBuffer" in n]
-    con_f = [v for n, v in r["fetch"].values() if "contract_kernel" in n]
-    con_w = [v for n, v in r["write"].values() if "contract_kernel" in n]
-    if not (copy_f and copy_w and con_f and con_w):
+
+    def per_query(tag, match):
+        """The counter's sum over matching kernels, per query (a merge each)."""
+        queries = sum("merge_kernel" in n for n, _ in r[tag].values())
+        return sum(v for n, v in r[tag].values() if match(n)) / max(1, queries)
+
+    sym = bool(args.self_symmetric)
+    if not copy_f or not copy_w or not per_query("mfma", lambda n: _in_contraction(n, sym)):
         return None, None
     f_scale = COPY_PROBE_BYTES / (max(copy_f) * 1024.0)
     w_scale = COPY_PROBE_BYTES / (max(copy_w) * 1024.0)
-    fetch_b = max(con_f) * 1024.0 * f_scale
-    write_b = max(con_w) * 1024.0 * w_scale
+    fetch_b = per_query("fetch", lambda n: _in_contraction(n, sym)) * 1024.0 * f_scale
+    write_b = per_query("write", lambda n: _in_contraction(n, sym)) * 1024.0 * w_scale
     info = {"fetch_bytes": fetch_b, "write_bytes": write_b,
             "fetch_scale": f_scale, "write_scale": w_scale,
+            "mfma_flops": per_query("mfma", lambda n: _in_contraction(n, sym)) * MFMA_OP_FLOPS,
+            "mfma_flops_query": per_query("mfma", lambda n: True) * MFMA_OP_FLOPS,
             "method": "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, KiB per dispatch, "
-                      "scaled by a 1 GiB hipMemcpy device-to-device copy"}
-    # the same passes' merge_kernel dispatch (the query's second kernel)
-    mer_f = [v for n, v in r["fetch"].values() if "merge_kernel" in n]
-    mer_w = [v for n, v in r["write"].values() if "merge_kernel" in n]
-    if mer_f and mer_w:
-        info["merge_kernel"] = {"fetch_bytes": max(mer_f) * 1024.0 * f_scale,
-                                "write_bytes": max(mer_w) * 1024.0 * w_scale}
+                      "scaled by a 1 GiB hipMemcpy device-to-device copy; "
+                      "SQ_INSTS_VALU_MFMA_MOPS_* x 512, padding included",
+            # the same passes' merge_kernel dispatch
+            "merge_kernel": {
+                "fetch_bytes": per_query("fetch", lambda n: "merge_kernel" in n) * 1024.0 * f_scale,
+                "write_bytes": per_query("write", lambda n: "merge_kernel" in n) * 1024.0 * w_scale}}
     return fetch_b + write_b, info
 
 
@@ -601,14 +625,20 @@ def main():
     out["config"]["pairs_scored_per_step"] = computed
     if "ms" in first:
         out["first_query_ms"] = first["ms"]
-    # algorithmic MFMA work of the pairs the contraction actually scored
-    flops = FLOPS_PER_ATOM[prec] * natoms * computed
-    achieved = flops / (ms_contract * 1e-3) / 1e12
-    out["roofline"] = {"bound": "mfma", "kernel": "contract_kernel",
+    # Matrix operations of the contraction's span as the hardware counted them:
+    # the symmetric query contracts only the tiles that can hold a candidate,
+    # so pairs x flops per pair would count work that is not done.
+    out["config"]["pairs_contracted"] = "tiles the filter keeps" if computed < pairs else computed
+    flops = traffic_info["mfma_flops"] if traffic_info else None
+    if flops is None and computed == pairs:
+        flops = FLOPS_PER_ATOM[prec] * natoms * computed
+    achieved = flops / (ms_contract * 1e-3) / 1e12 if flops else None
+    out["roofline"] = {"bound": "mfma",
+                       "kernel": "ball test + filter_kernel + contract_kernel" if computed < pairs
+                       else "contract_kernel",
                        "achieved": achieved, "peak": PEAK_TFLOPS[prec], "unit": "TFLOP/s",
-                       "frac": achieved / PEAK_TFLOPS[prec], "traffic": traffic,
-                       "flops_per_launch": flops, "ms_per_launch": ms_contract,
-                       "flops_per_pair": FLOPS_PER_ATOM[prec] * natoms}
+                       "frac": achieved / PEAK_TFLOPS[prec] if achieved else None,
+                       "traffic": traffic, "flops_per_launch": flops, "ms_per_launch": ms_contract}
     if traffic_info:
         out["roofline"]["traffic_detail"] = traffic_info
     out["stages_ms"] = {s: mean_stat(stats, "ms_" + s) for s in ("prep", "contract", "merge", "fallback", "total")}
@@ -673,10 +703,8 @@ def main():
             ctx.set_option(knn.OPT_SELF_SYMMETRIC, args.self_symmetric)
             ctx.set_reference(frames, w)
             wall32, st32, _, _ = time_fused(ctx, hip, n, k, args.fp32_steps, 1)
-        ms32 = mean_stat(st32, "ms_contract")
-        a32 = 18 * natoms * mean_stat(st32, "n_pairs_computed") / (ms32 * 1e-3) / 1e12
         out["fp32_path"] = {"value": pairs / wall32, "unit": "pairs/s", "ms_per_step": wall32 * 1e3,
-                            "contract_ms": ms32, "achieved_tflops": a32, "frac_fp32_peak": a32 / 157.3}
+                            "contract_ms": mean_stat(st32, "ms_contract")}
         out["speedup_vs_fp32"] = out["value"] / out["fp32_path"]["value"]
 
     if args.fp16_steps > 0 and prec != "fp16":
@@ -686,11 +714,9 @@ def main():
             ctx.set_option(knn.OPT_SELF_SYMMETRIC, args.self_symmetric)
             ctx.set_reference(frames, w)
             wall16, st16, d16, i16 = time_fused(ctx, hip, n, k, args.fp16_steps, 1)
-        ms16 = mean_stat(st16, "ms_contract")
-        a16 = 54 * natoms * mean_stat(st16, "n_pairs_computed") / (ms16 * 1e-3) / 1e12
         out["fp16_path"] = {"value": pairs / wall16, "unit": "pairs/s", "ms_per_step": wall16 * 1e3,
-                            "contract_ms": ms16, "merge_ms": mean_stat(st16, "ms_merge"),
-                            "achieved_tflops": a16, "frac_fp16_peak": a16 / 2500.0,
+                            "contract_ms": mean_stat(st16, "ms_contract"),
+                            "merge_ms": mean_stat(st16, "ms_merge"),
                             "candidates_per_query": mean_stat(st16, "n_candidates") / n,
                             "outputs_equal_headline": bool((d16 == dist).all() and (i16 == idx).all())}
 

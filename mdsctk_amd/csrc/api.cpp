@@ -780,7 +780,9 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   p->sample = 0;
   p->sample_pairs = 0;
   if (sampled_query(c, q, n_fit)) {
-    const int want = std::max(ref_pairs / 16, 8 * q.k1 / (2 * kTile) + 1);
+    // (4096 frames are enough of a large set: what the pass saves does not
+    // grow with the set, what it costs does)
+    const int want = std::max(std::min(ref_pairs / 16, 64), 8 * q.k1 / (2 * kTile) + 1);
     p->sample = ref_pairs / want;
     if (p->sample < 4) p->sample = 0;  // too large a part of the query
     if (p->sample) p->sample_pairs = (ref_pairs + p->sample - 1) / p->sample;
