@@ -1846,6 +1846,15 @@ int mdsctk_knn_set_option(mdsctk_knn_ctx* c, int option, double value) {
   switch (option) {
     case MDSCTK_OPT_HBM_BUDGET:
       if (value < 0) return fail(c, MDSCTK_ERR_ARG, "budget must be >= 0");
+      if (value > 0 && !c->server) {
+        // no ordered copy under a budget (ensure_ordered): give back what an
+        // earlier one holds, so that the budget's queries have that room
+        std::lock_guard<std::mutex> g(c->plain_mu);
+        free_ordered(c);
+        dfree(c, c->main.ws_cross);
+        c->main.ws_cross = nullptr;
+        c->main.ws_cross_bytes = 0;
+      }
       {
         std::lock_guard<std::mutex> lk(c->mem_mu);  // the serving thread allocates too
         c->budget = (size_t)value;

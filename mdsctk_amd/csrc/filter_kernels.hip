@@ -29,12 +29,13 @@
 // bounds the rest by Cauchy-Schwarz: lambda(M) <= lambda(M') + |x''_a||x''_b|.
 //
 // Measured, self query of 200000 x 1000 atoms, k = 64 (50 metastable
-// states): the contraction over every tile took 917 ms; the filter takes
-// 100 ms (0.9 PFLOP/s of BF16, what a large matrix product reaches on this
-// card is 1.1) and leaves 2.3 % of the tiles, which take 30 ms.  Without the
-// first segment the filter alone took over 220 ms.  Cross query of 4096
+// states): the contraction over every tile took 917 ms; the filter took
+// 91 ms over all tiles (1 PFLOP/s of BF16, what a large matrix product reaches
+// on this card is 1.1), takes 31 ms over those that the ball test (kOutBall)
+// leaves, and leaves 2.3 % of the tiles, which take 31 ms.  Without the first
+// segment the filter alone took over 220 ms.  Cross query of 4096
 // against 100000 x 500 atoms, k = 50 (one basin): contraction 10.0 ms before;
-// the filter takes 4.2 ms (1.1 PFLOP/s) and leaves tiles for 2.1 ms.  50000
+// the filter takes 4.0 ms (1.1 PFLOP/s) and leaves tiles for 2.1 ms.  50000
 // against 50000 x 304 atoms in plain FP32, k = 100: 124 ms before, now 5 for
 // the landmarks, 15 for the filter and 26 for the tiles left.
 #include <hip/hip_runtime.h>

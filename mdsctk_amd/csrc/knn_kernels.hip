@@ -14,10 +14,11 @@
 //                    an approximate score s~ = G_r + G_f - 2 lambda_max, and
 //                    per-lane candidate lists (threshold + append, ballot
 //                    select compaction); no distance matrix is written.
-//                    For a self query it may instead score the upper block
-//                    triangle only and write the n x n FP32 score matrix,
-//                    from which sym_select_kernel lists each row's
-//                    candidates.
+//                    For a self query it scores the upper block triangle
+//                    only, and each pair may join both frames' lists; with a
+//                    tile list (filter_kernels.hip) it walks those tiles.
+//   trace_kernel     the same where only the block's trace counts (--nofit and
+//                    data vectors, split forms).
 //   merge_kernel     per query: radix-select the (k+1)-th smallest s~ over
 //                    its lists, take every candidate within the certified
 //                    window, re-score them exactly in FP64 from the raw
