@@ -1336,6 +1336,12 @@ __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(C
   }
 }
 
+// The epilogue's half of G~ in FP32, lowered by its slack; G~ near the end of
+// FP32's range (and NaN) gives -inf, which rejects nothing.
+__device__ __forceinline__ float trace_half(double g) {
+  return g <= 1e36 ? (float)(0.5 * (1.0 - 2e-6) * g) : -INFINITY;
+}
+
 // One plane of a K-group for a wave's 2 x 2 tiles: acc[2 i + j] += A_i * B_j^T,
 // the three split products in mma_group's order (the same sums, bit for bit).
 template <int PREC>
@@ -1452,7 +1458,7 @@ __global__ __launch_bounds__(256, 2) void trace_kernel(ContractParams P) {
       const int64_t q = fit0 + j * kTile;
       fvalid[j] = q < P.n_fit;
       list[j] = P.ent + (q * P.nl + list_id) * P.cap;
-      hg[j] = fvalid[j] ? (float)(0.5 * (1.0 - 2e-6) * P.fGt[q]) : INFINITY;
+      hg[j] = fvalid[j] ? trace_half(P.fGt[q]) : INFINITY;
       thr[j] = ovf[j] = INFINITY;
       cnt[j] = 0;
     }
@@ -1482,7 +1488,7 @@ __global__ __launch_bounds__(256, 2) void trace_kernel(ContractParams P) {
         const int64_t r = (int64_t)p * 2 * kTile + lane;
         const bool in = real_pair(t) && r < P.n_ref;
         g_row = P.rGt[r];
-        half_row = in ? (float)(0.5 * (1.0 - 2e-6) * g_row) : INFINITY;
+        half_row = in ? trace_half(g_row) : INFINITY;
         if constexpr (MODE == kOutSym)
           thr_row = in && ph + t * P.phases > fb ? __uint_as_float(P.thr[r]) : -1.0f;
       }

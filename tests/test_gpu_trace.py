@@ -60,3 +60,20 @@ def test_frames_as_given_against_themselves(prec):
             out.append(ctx.query(None, 40, knn.KNN_NOFIT))
     np.testing.assert_array_equal(out[0][1], out[1][1])
     np.testing.assert_array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("power", [-60, 60])
+def test_vectors_near_the_ends_of_the_range(power):
+    """Scaling by a power of two scales every value, sum and distance exactly:
+    the same rows at G terms around 1e-36 and 1e37."""
+    x = synth.data_vectors(4300, 45, 3, "dihedral")
+    out = []
+    for f in (1.0, 2.0 ** power):
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_data_reference(x * f, "euclidean")
+            out.append(ctx.data_query(None, 20))
+            out[-1] += ctx.data_query(x[:500] * f, 20)
+    for j in (1, 3):
+        np.testing.assert_array_equal(out[0][j], out[1][j])
+    for j in (0, 2):
+        np.testing.assert_array_equal(out[0][j] * 2.0 ** power, out[1][j])
