@@ -433,9 +433,12 @@ __global__ __launch_bounds__(256) void filter_stats_kernel(
     const double a0 = mc->norm0 + dn0, a = mc->norm + dn;
     const double e0 = step * (sh.groups0() + 2) * 0.5 * a0 * a0;
     const double e1 = step * (sh.groups() + 4) * 0.5 * a * a;
-    // a frame whose squares leave FP32's range (or that is not finite) is
-    // never past a threshold: every comparison with NaN keeps its tiles
-    const double nan = gt >= 1e-20 && gt <= 1e29 ? 0.0 : (double)NAN;
+    // A frame whose squares leave FP32's range (or that is not finite) is
+    // never past a threshold: every comparison with NaN keeps its tiles.  The
+    // test's square roots take squares below 1.2e-38 as zero, so that its sum
+    // of column norms may be short by 3.3e-19: from 1e-12 on that is less than
+    // the 1e-6 gt taken off below.
+    const double nan = gt >= 1e-12 && gt <= 1e29 ? 0.0 : (double)NAN;
     full[f] = make_float4((float)(0.5 * gt - res[0] - res[1] - e1 - 1e-6 * gt + nan),
                           (float)(dn * up), (float)(sqrt(l2[0] + l2[1]) * up), 0.f);
     pre[f] = make_float4((float)(0.5 * gt - res[0] - e0 - 1e-6 * gt + nan), (float)(dn0 * up),

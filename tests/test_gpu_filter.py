@@ -117,3 +117,22 @@ def test_ordered_cross_query(gen, natoms, n_ref, n_fit, k, prec):
     rows = np.arange(0, n_fit, n_fit // 5)
     d_o, i_o = oracle.knn_exact(ref, fit[rows], w, k)
     check_knn(ref, fit[rows], w, d0[rows], i0[rows], d_o, i_o)
+
+
+@pytest.mark.parametrize("power", [-18, -23, -24, -27, -31, -33, -34])
+def test_filtered_self_query_of_tiny_frames(power):
+    """G terms from 2e-9 down to 4e-19, on both sides of 1e-12, below which a
+    frame's tiles are all kept: there the filter's FP32 squares reach the
+    subnormal numbers.  No row may need a second pass either."""
+    frames = synth.trajectory(4300, 64, 5)
+    frames = (frames - frames.mean(axis=1, keepdims=True)) * np.float32(2.0 ** power)
+    rows = []
+    for sym in (1, 0):
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_option(knn.OPT_SELF_SYMMETRIC, sym)
+            ctx.set_reference(frames)
+            rows.append(ctx.query(None, 8))
+            st = ctx.stats()
+            assert st["n_relisted_rows"] == 0 and st["n_fallback_rows"] == 0
+    np.testing.assert_array_equal(rows[0][1], rows[1][1])
+    np.testing.assert_array_equal(rows[0][0], rows[1][0])
