@@ -353,7 +353,9 @@ int set_reference_impl(mdsctk_knn_ctx* c, const float* xyz, bool on_device, int6
   // after trajectory of one system): nine allocations and their frees, each
   // of which waits for the device, took a third of a 1000 x 60-frame run.
   // Not under an HBM budget, which is checked as the buffers are allocated.
-  const bool same = c->has_ref && !c->budget && c->w.metric == kMetricRMSD && c->ref.vdim == 0 &&
+  // Nor for frames in device memory, which another stream may still be
+  // writing: freeing the last set's buffers waits for the device.
+  const bool same = c->has_ref && !c->budget && !on_device && c->w.metric == kMetricRMSD && c->ref.vdim == 0 &&
                     c->ref.n == n_ref && c->ref.natoms == natoms;
   if (!same) free_frames(c, c->ref);
   free_plain(c);
