@@ -98,7 +98,16 @@ int fail(mdsctk_knn_ctx* c, int code, const char* fmt, ...) {
   return code;
 }
 
+// A failure that the caller makes good: no text of it is left.
+void forget_error(mdsctk_knn_ctx* c) {
+  if (tl_err_sink)
+    tl_err_sink->clear();
+  else
+    tl_ctx_err.erase(c);
+}
+
 int hip_fail(mdsctk_knn_ctx* c, hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here, not by the next launch
   return fail(c, e == hipErrorOutOfMemory ? MDSCTK_ERR_NOMEM : MDSCTK_ERR_HIP, "%s: %s", what,
               hipGetErrorString(e));
 }
@@ -124,6 +133,9 @@ int dalloc(mdsctk_knn_ctx* c, void** p, size_t bytes, const char* what) {
   hipError_t e = hipMalloc(p, bytes);
   std::lock_guard<std::mutex> g(c->mem_mu);
   if (e != hipSuccess) {
+    // The runtime keeps the error until it is read: the launches of a caller
+    // that goes on without this buffer would report it as theirs.
+    (void)hipGetLastError();
     *p = nullptr;
     c->held -= bytes;
     return fail(c, MDSCTK_ERR_NOMEM, "%s: hipMalloc(%zu) failed: %s", what, bytes,
@@ -858,7 +870,7 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   if (xb) {
     int rc = ensure(c, &s.ws_cross, &s.ws_cross_bytes, xb, "ordered query frames");
     if (rc == MDSCTK_ERR_NOMEM) {
-      tl_ctx_err.erase(c);  // every tile instead
+      forget_error(c);  // every tile instead
       return 0;
     }
     if (rc) return rc;
@@ -980,7 +992,7 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
   if (dalloc(c, &o.mem, bytes, "ordered reference set") || dalloc(c, &tmp, scratch, "ordering")) {
     dfree(c, o.mem);
     o.mem = nullptr;
-    tl_ctx_err.erase(c);
+    forget_error(c);
     return 0;
   }
   Carve cv, ct;
@@ -1211,7 +1223,7 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   if (!rc) rc = ensure(c, &s.ws_small, &s.ws_small_bytes, small, "list headers");
   if (rc == MDSCTK_ERR_NOMEM) {  // the list path instead, without the mirrored lists
     release_mirror_lists(c);
-    tl_ctx_err.erase(c);
+    forget_error(c);
     return 1;
   }
   if (rc) return rc;
@@ -1546,7 +1558,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
     if (rc == 0) {
       plain_missing = false;
     } else if (rc == MDSCTK_ERR_NOMEM) {
-      tl_ctx_err.erase(c);  // no room for them: the exact rows instead
+      forget_error(c);  // no room for them: the exact rows instead
     } else {
       return rc;
     }
@@ -1627,7 +1639,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
     if (!xyz) ws.fit = saved;
     if (fused_rc == MDSCTK_ERR_NOMEM && !cv) {
       // even one phase's lists do not fit: the exact rows, in batches that do
-      tl_ctx_err.erase(c);
+      forget_error(c);
       fused_rc = 1;
     }
     if (fused_rc < 0) return fused_rc;

@@ -210,6 +210,8 @@ namespace mdsctk {
 // thread, that thread's error sink) and returns `code`.
 int fail(mdsctk_knn_ctx* c, int code, const char* fmt, ...);
 int hip_fail(mdsctk_knn_ctx* c, hipError_t e, const char* what);
+// Drops the calling thread's error text of a failure that was made good.
+void forget_error(mdsctk_knn_ctx* c);
 // Directs fail() on the calling thread to `sink` (nullptr = the context).
 void set_error_sink(std::string* sink);
 // The calling thread's error text for context c (mdsctk_knn_last_error).

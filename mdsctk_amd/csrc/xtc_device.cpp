@@ -108,6 +108,7 @@ int mdsctk_xtc_read_device(const char* path, int32_t natoms, int device, float**
   } h;
   h.fd = fd;
   auto hip_err = [&](hipError_t e, const char* what) {
+    (void)hipGetLastError();  // reported here, not by the next launch
     return io_fail(e == hipErrorOutOfMemory ? MDSCTK_ERR_NOMEM : MDSCTK_ERR_HIP,
                    "xtc_read_device: %s failed%lld", what, (long long)e);
   };

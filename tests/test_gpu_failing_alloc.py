@@ -1,0 +1,82 @@
+"""Queries whose optional buffers cannot be allocated: the ordered copy of the
+resident set, the scratch it is made with, the ordered query frames.  The
+runtime refuses one chosen allocation, and the query takes the route that does
+without, with the same rows, not exact rows nor an error.  In a process of
+its own, where failing_alloc.c stands in front of the runtime's calls."""
+import ctypes
+import json
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+pytestmark = pytest.mark.gpu
+
+
+def _child(shim_path):
+    shim = ctypes.CDLL(shim_path, mode=ctypes.RTLD_GLOBAL)
+    shim.fail_alloc.argtypes = [ctypes.c_int, ctypes.c_long]
+    shim.alloc_calls.restype = ctypes.c_long
+    sys.path.insert(0, os.path.dirname(HERE))
+    from mdsctk_amd import knn, synth
+
+    def say(name, **kw):
+        print(json.dumps(dict(name=name, **kw)), flush=True)
+
+    n_ref, natoms, k, m = 8200, 520, 12, 4100
+    x = synth.metastable_trajectory(n_ref + m, natoms, 3, n_centres=12)
+    ref, fit, w = x[:n_ref], x[n_ref:], synth.masses(natoms, "random", 2)
+    want = None
+    # the second query of 4100 frames makes the ordered copy (8200 seen)
+    for call in (-1, 0, 1, 2):
+        print(f"call {call}, synchronous", flush=True)
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_reference(ref, w)
+            d0, i0 = ctx.query(fit, k)
+            want = want or (d0, i0)
+            for turn in (0, 1):
+                shim.fail_alloc(0, call if turn == 0 else -1)
+                d, i = ctx.query(fit, k)
+                say("sync", call=call, turn=turn, allocs=shim.alloc_calls(0),
+                    same=bool((d == want[0]).all() and (i == want[1]).all()),
+                    fallback=ctx.stats()["n_fallback_rows"], text=ctx.last_error())
+        print(f"call {call}, served", flush=True)
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_reference(ref, w)
+            ctx.query(fit, k)
+            ctx.wait(ctx.submit(fit[:2048], k))
+            ctx.wait(ctx.submit(fit[:1900], k))
+            for turn in (0, 1):
+                shim.fail_alloc(0, call if turn == 0 else -1)
+                r = ctx.wait(ctx.submit(fit[:2048], k))
+                say("served", call=call, turn=turn, allocs=shim.alloc_calls(0),
+                    same=bool((r.dist == want[0][:2048]).all() and (r.idx == want[1][:2048]).all()),
+                    fallback=r.info["n_fallback_rows"], text="")
+    print("DONE", flush=True)
+
+
+@pytest.fixture(scope="module")
+def shim(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("shim") / "failing_alloc.so")
+    subprocess.run(["cc", "-shared", "-fPIC", "-O1", "-o", lib,
+                    os.path.join(HERE, "failing_alloc.c"), "-ldl"], check=True)
+    return lib
+
+
+def test_optional_buffers_that_cannot_be_allocated(shim):
+    p = subprocess.run([sys.executable, "-u", os.path.abspath(__file__), shim], capture_output=True,
+                       text=True, timeout=100)
+    print(p.stdout[-6000:], p.stderr[-3000:])
+    assert p.returncode == 0 and "DONE" in p.stdout
+    rows = [json.loads(l) for l in p.stdout.splitlines() if l.startswith("{")]
+    assert len(rows) == 16
+    for r in rows:
+        assert r["same"] and r["fallback"] == 0 and r["text"] == "", r
+    assert any(r["allocs"] >= 3 for r in rows if r["call"] == -1 and r["name"] == "sync")
+
+
+if __name__ == "__main__":
+    _child(sys.argv[1])
