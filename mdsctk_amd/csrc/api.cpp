@@ -1713,9 +1713,15 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
   // Short outputs come back in one copy (they lie side by side) to a pinned
   // buffer of the slot's, long ones straight to the caller's memory.
   const size_t out_bytes = out_elems * (sizeof(double) + sizeof(int));
-  const bool pinned = !out_on_device && out_bytes <= kPinnedOut;
-  if (pinned && !s.h_out)
-    HIP_TRY(c, hipHostMalloc(&s.h_out, kPinnedOut, hipHostMallocDefault));
+  // (Measured, 360 KB: pinning .04 to .1 ms once, the copy .02 ms against .17
+  // to memory that is not pinned.)
+  bool pinned = !out_on_device && out_bytes <= kPinnedOut;
+  if (pinned && !s.h_out &&
+      hipHostMalloc(&s.h_out, kPinnedOut, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    s.h_out = nullptr;
+    pinned = false;
+  }
   if (pinned) {
     HIP_TRY(c, hipMemcpyAsync(s.h_out, d_dist, out_bytes, hipMemcpyDeviceToHost, s.st));
   } else if (!out_on_device) {

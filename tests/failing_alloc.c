@@ -6,7 +6,7 @@
 #include <dlfcn.h>
 #include <stddef.h>
 
-static long calls[2], chosen[2] = {-1, -1};
+static long calls[3], chosen[3] = {-1, -1, -1};
 
 static size_t ask(int kind, size_t bytes) {
   const long call = __atomic_fetch_add(&calls[kind], 1, __ATOMIC_SEQ_CST);
@@ -17,8 +17,8 @@ static void* real(const char* name) {
   return dlsym(dlopen("libamdhip64.so.7", RTLD_NOLOAD | RTLD_LAZY), name);
 }
 
-/* Start counting kind 0 (device memory) or 1 (pinned memory) from zero; call
- * number `call` is to fail (-1: none). */
+/* Start counting kind 0 (device memory), 1 (pinned memory) or 2 (the free
+ * memory's size) from zero; call number `call` is to fail (-1: none). */
 void fail_alloc(int kind, long call) {
   __atomic_store_n(&chosen[kind], call, __ATOMIC_SEQ_CST);
   __atomic_store_n(&calls[kind], 0, __ATOMIC_SEQ_CST);
@@ -32,4 +32,9 @@ int hipMalloc(void** p, size_t bytes) {
 
 int hipHostMalloc(void** p, size_t bytes, unsigned flags) {
   return ((int (*)(void**, size_t, unsigned))real("hipHostMalloc"))(p, ask(1, bytes), flags);
+}
+
+int hipMemGetInfo(size_t* free_bytes, size_t* total) {
+  if (ask(2, 0)) return 1;
+  return ((int (*)(size_t*, size_t*))real("hipMemGetInfo"))(free_bytes, total);
 }

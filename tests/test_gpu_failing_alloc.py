@@ -16,16 +16,20 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 pytestmark = pytest.mark.gpu
 
 
-def _child(shim_path):
-    shim = ctypes.CDLL(shim_path, mode=ctypes.RTLD_GLOBAL)
+def _shim(path):
+    shim = ctypes.CDLL(path, mode=ctypes.RTLD_GLOBAL)
     shim.fail_alloc.argtypes = [ctypes.c_int, ctypes.c_long]
     shim.alloc_calls.restype = ctypes.c_long
     sys.path.insert(0, os.path.dirname(HERE))
+    return shim
+
+
+def say(name, **kw):
+    print(json.dumps(dict(name=name, **kw)), flush=True)
+
+
+def child_optional(shim):
     from mdsctk_amd import knn, synth
-
-    def say(name, **kw):
-        print(json.dumps(dict(name=name, **kw)), flush=True)
-
     n_ref, natoms, k, m = 8200, 520, 12, 4100
     x = synth.metastable_trajectory(n_ref + m, natoms, 3, n_centres=12)
     ref, fit, w = x[:n_ref], x[n_ref:], synth.masses(natoms, "random", 2)
@@ -58,6 +62,31 @@ def _child(shim_path):
     print("DONE", flush=True)
 
 
+def child_pinned(shim):
+    from mdsctk_amd import knn, synth
+    x = synth.trajectory(500, 40, 1)
+    want = None
+    for call in (-1, 0):
+        print(f"call {call}", flush=True)
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_reference(x)
+            for turn in (0, 1):
+                shim.fail_alloc(1, call if turn == 0 else -1)
+                d, i = ctx.query(None, 8)
+                want = want or (d, i)
+                say("pinned", call=call, turn=turn,
+                    same=bool((d == want[0]).all() and (i == want[1]).all()))
+    print("DONE", flush=True)
+
+
+def _run(shim, name):
+    p = subprocess.run([sys.executable, "-u", os.path.abspath(__file__), shim, name],
+                       capture_output=True, text=True, timeout=100)
+    print(p.stdout[-6000:], p.stderr[-3000:])
+    assert p.returncode == 0 and "DONE" in p.stdout
+    return [json.loads(l) for l in p.stdout.splitlines() if l.startswith("{")]
+
+
 @pytest.fixture(scope="module")
 def shim(tmp_path_factory):
     lib = str(tmp_path_factory.mktemp("shim") / "failing_alloc.so")
@@ -67,16 +96,17 @@ def shim(tmp_path_factory):
 
 
 def test_optional_buffers_that_cannot_be_allocated(shim):
-    p = subprocess.run([sys.executable, "-u", os.path.abspath(__file__), shim], capture_output=True,
-                       text=True, timeout=100)
-    print(p.stdout[-6000:], p.stderr[-3000:])
-    assert p.returncode == 0 and "DONE" in p.stdout
-    rows = [json.loads(l) for l in p.stdout.splitlines() if l.startswith("{")]
+    rows = _run(shim, "optional")
     assert len(rows) == 16
     for r in rows:
         assert r["same"] and r["fallback"] == 0 and r["text"] == "", r
     assert any(r["allocs"] >= 3 for r in rows if r["call"] == -1 and r["name"] == "sync")
 
 
+def test_pinned_output_buffer_that_cannot_be_allocated(shim):
+    rows = _run(shim, "pinned")
+    assert len(rows) == 4 and all(r["same"] for r in rows), rows
+
+
 if __name__ == "__main__":
-    _child(sys.argv[1])
+    globals()["child_" + sys.argv[2]](_shim(sys.argv[1]))
