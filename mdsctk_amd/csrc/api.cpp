@@ -961,6 +961,7 @@ size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
 // the other workspaces keep their room.
 int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
   const int64_t n = c->ref.n;
+  if (n_fit < kCrossMinFit) return 0;  // such queries never walk the copy
   if (!c->ref_axes || n < kCrossMinRef || n * c->ref.natoms < kCrossMinWork || c->budget) return 0;
   std::lock_guard<std::mutex> g(c->plain_mu);
   OrderedRef& o = c->ordered;

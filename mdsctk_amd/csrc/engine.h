@@ -78,7 +78,7 @@ struct MiddleSet {
 
 struct OrderedRef {
   bool built = false, failed = false;
-  int64_t seen = 0;  // query frames since the set became resident
+  int64_t seen = 0;  // frames, since the set became resident, of queries that could use it
   void* mem = nullptr;
   DevFrames f;  // xyz null: the coordinates are the resident set's
   int* order = nullptr;
@@ -242,8 +242,8 @@ int slot_frames(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
 int prep_slot(mdsctk_knn_ctx* c, Slot& s, bool nofit);
 // The resident set's --nofit operands, built on first use (synchronous).
 int ensure_plain(mdsctk_knn_ctx* c, hipStream_t st);
-// Counts a fitted query's frames and, once they pay for it, orders the
-// resident set for cross queries (synchronous, on slot s); no error if it
+// Counts a fitted query's frames (of kCrossMinFit or more: shorter ones never
+// take the ordered form) and, once they pay for it, orders the resident set for cross queries (synchronous, on slot s); no error if it
 // cannot.
 int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
 // Bytes of slot workspace the ordered form of a cross query of n_fit frames

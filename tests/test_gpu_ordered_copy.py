@@ -1,0 +1,34 @@
+"""When a context makes the ordered copy of its resident set, what it holds for
+it, and when it gives it back.  Rows are the same with and without."""
+import numpy as np
+import pytest
+
+from mdsctk_amd import knn, synth
+
+pytestmark = pytest.mark.gpu
+
+N_REF, NATOMS, K = 8200, 520, 12
+COPY = 12 * N_REF * NATOMS  # bytes of the copy's operand alone
+
+
+@pytest.fixture(scope="module")
+def frames():
+    x = synth.metastable_trajectory(N_REF + 2100, NATOMS, 3, n_centres=12)
+    return x[:N_REF], x[N_REF:]
+
+
+def _held(ctx):
+    return ctx.stats()["device_bytes"]
+
+
+def test_short_queries_do_not_make_the_copy(frames):
+    """Queries below 256 frames never walk the copy, however many there are."""
+    ref, fit = frames
+    with knn.KnnContext(0, "bf16") as ctx:
+        ctx.set_reference(ref)
+        want = ctx.query(fit[:255], K)
+        before = _held(ctx)
+        for _ in range(40):
+            d, i = ctx.query(fit[:255], K)
+        np.testing.assert_array_equal(i, want[1])
+        assert _held(ctx) == before
