@@ -986,16 +986,21 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
                          3 * Carve::round((size_t)n * sizeof(int)) + Carve::round(sort_temp) +
                          Carve::round(12 * kFilterSamples * sizeof(double));
   size_t free_b = 0, total_b = 0;
-  HIP_TRY(c, hipMemGetInfo(&free_b, &total_b));
   void* tmp = nullptr;
-  o.failed = true;  // until everything below has worked
-  if (bytes + scratch > free_b / 4) return 0;
-  if (dalloc(c, &o.mem, bytes, "ordered reference set") || dalloc(c, &tmp, scratch, "ordering")) {
+  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+    (void)hipGetLastError();
+    free_b = 0;
+  }
+  if (bytes + scratch > free_b / 4 || dalloc(c, &o.mem, bytes, "ordered reference set") ||
+      dalloc(c, &tmp, scratch, "ordering")) {
+    // asked again after as many frames: there may be room by then
     dfree(c, o.mem);
     o.mem = nullptr;
+    o.seen = 0;
     forget_error(c);
     return 0;
   }
+  o.failed = true;  // until everything below has worked
   Carve cv, ct;
   cv.base = (char*)o.mem;
   cv.size = bytes;
@@ -1050,7 +1055,8 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
   if (rc) {
     dfree(c, o.mem);
     o.mem = nullptr;
-    return rc;
+    forget_error(c);  // the query goes on without (and meets a broken device itself)
+    return 0;
   }
   o.f = f;
   o.failed = false;

@@ -77,7 +77,8 @@ struct MiddleSet {
 };
 
 struct OrderedRef {
-  bool built = false, failed = false;
+  bool built = false;
+  bool failed = false;  // its kernels failed: not tried again
   int64_t seen = 0;  // frames, since the set became resident, of queries that could use it
   void* mem = nullptr;
   DevFrames f;  // xyz null: the coordinates are the resident set's

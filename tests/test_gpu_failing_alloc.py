@@ -62,6 +62,28 @@ def child_optional(shim):
     print("DONE", flush=True)
 
 
+def child_retry(shim):
+    """The copy is refused once, for its memory or because the free memory's
+    size cannot be had, and made after as many frames more."""
+    from mdsctk_amd import knn, synth
+    n_ref, natoms, k, m = 8200, 520, 12, 4100
+    x = synth.metastable_trajectory(n_ref + m, natoms, 3, n_centres=12)
+    want = None
+    for kind in (0, 2):
+        print(f"kind {kind}", flush=True)
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_reference(x[:n_ref])
+            for turn in range(5):
+                shim.fail_alloc(kind, 0 if turn == 1 else -1)
+                shim.fail_alloc(2 - kind, -1)
+                d, i = ctx.query(x[n_ref:], k)
+                want = want or (d, i)
+                say("retry", kind=kind, turn=turn, held=ctx.stats()["device_bytes"],
+                    same=bool((d == want[0]).all() and (i == want[1]).all()),
+                    fallback=ctx.stats()["n_fallback_rows"], copy=12 * n_ref * natoms)
+    print("DONE", flush=True)
+
+
 def child_pinned(shim):
     from mdsctk_amd import knn, synth
     x = synth.trajectory(500, 40, 1)
@@ -101,6 +123,16 @@ def test_optional_buffers_that_cannot_be_allocated(shim):
     for r in rows:
         assert r["same"] and r["fallback"] == 0 and r["text"] == "", r
     assert any(r["allocs"] >= 3 for r in rows if r["call"] == -1 and r["name"] == "sync")
+
+
+def test_the_ordered_copy_is_asked_for_again(shim):
+    rows = _run(shim, "retry")
+    assert len(rows) == 10
+    for r in rows:
+        assert r["same"] and r["fallback"] == 0, r
+        base = next(b["held"] for b in rows if b["kind"] == r["kind"] and b["turn"] == 0)
+        made = r["held"] > base + r["copy"]
+        assert made == (r["turn"] >= 3), r
 
 
 def test_pinned_output_buffer_that_cannot_be_allocated(shim):
