@@ -866,7 +866,8 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
                                          : kappa_data(c->prec, c->ref.natoms)) *
              c->eps_scale;
   p->x.on = false;
-  const size_t xb = (cv || fit.xyz == c->ref.xyz) ? 0 : cross_bytes(c, q, n_fit);
+  size_t xb = (cv || fit.xyz == c->ref.xyz || n_fit > s.cross_most) ? 0 : cross_bytes(c, q, n_fit);
+  if (xb && s.cross_room > n_fit) xb = cross_bytes(c, q, s.cross_room);
   if (xb) {
     int rc = ensure(c, &s.ws_cross, &s.ws_cross_bytes, xb, "ordered query frames");
     if (rc == MDSCTK_ERR_NOMEM) {

@@ -48,6 +48,8 @@ struct Slot {
   size_t ws_sort_bytes = 0;
   void* ws_cross = nullptr;  // a cross query's ordered copy and tile lists (CrossPlan)
   size_t ws_cross_bytes = 0;
+  int64_t cross_room = 0;          // frames it is sized for at least
+  int64_t cross_most = INT64_MAX;  // longest query that takes the ordered form
   // ev[0] start, ev[1] query prepared, ev[2] before the contraction, ev[3]
   // after it, ev[4] after the merge, ev[5] end; ev[6] after a symmetric self
   // query's landmark pass (so ev[2]..ev[6] is that pass).

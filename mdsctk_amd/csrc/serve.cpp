@@ -165,9 +165,6 @@ class HipServeDevice {
       if (!q.nofit && (rc = ensure_ordered(c_, s, b.n))) return rc;
       FusedPlan plan;
       if ((rc = plan_fused(c_, s, q, &plan))) return rc;
-      // beyond the rank sort the ordering takes a library sort, which is not
-      // for a captured graph
-      if (b.n > kRankSortMax) plan.x.on = false;
       if (c_->serve_share_cus && slots_.size() > 1) {
         plan.grid = std::max(8, (plan.grid / (int)slots_.size()) & ~7);
         plan.x.filter_grid = std::max(8, (plan.x.filter_grid / (int)slots_.size()) & ~7);
@@ -295,6 +292,11 @@ class HipServeDevice {
                      "serve outputs")))
       return rc;
     if ((rc = ensure_host(sl, elems, (size_t)limit))) return rc;
+    // The ordered form's workspace comes with the slot's first batch that
+    // takes it, at its largest.  Beyond the rank sort the ordering takes a
+    // library sort, which is not for a captured graph.
+    s.cross_most = kRankSortMax;
+    s.cross_room = std::min<int64_t>(limit, kRankSortMax);
     sl.sized_limit = limit;
     sl.sized_k_out = q.k_out;
     sl.sized_k1 = q.k1;

@@ -32,3 +32,22 @@ def test_short_queries_do_not_make_the_copy(frames):
             d, i = ctx.query(fit[:255], K)
         np.testing.assert_array_equal(i, want[1])
         assert _held(ctx) == before
+
+
+def test_served_batches_of_growing_size_allocate_nothing(frames):
+    """A slot's first batch against the ordered copy sizes its workspace for
+    the largest one."""
+    ref, fit = frames
+    with knn.KnnContext(0, "bf16") as ctx:
+        ctx.set_option(knn.OPT_SERVE_SLOTS, 1)
+        ctx.set_reference(ref)
+        want = ctx.query(fit, K)
+        for _ in range(4):
+            ctx.query(fit, K)
+        ctx.wait(ctx.submit(fit[:300], K))
+        before = _held(ctx)
+        for m in (300, 640, 1100, 2048, 1999):
+            r = ctx.wait(ctx.submit(fit[:m], K))
+            np.testing.assert_array_equal(r.idx, want[1][:m])
+            np.testing.assert_array_equal(r.dist, want[0][:m])
+            assert _held(ctx) == before
