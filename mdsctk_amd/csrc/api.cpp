@@ -127,7 +127,7 @@ int dalloc(mdsctk_knn_ctx* c, void** p, size_t bytes, const char* what) {
     if (c->budget && c->held + bytes > c->budget)
       return fail(c, MDSCTK_ERR_NOMEM,
                   "%s: %zu bytes would exceed the HBM budget (%zu held of %zu)", what, bytes,
-                  c->held, c->budget);
+                  c->held, c->budget.load());
     c->held += bytes;  // reserved before the allocation so that threads cannot overshoot
   }
   hipError_t e = hipMalloc(p, bytes);
@@ -1065,6 +1065,12 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
   return 0;
 }
 
+void drop_ordered(mdsctk_knn_ctx* c) {
+  if (!c->budget) return;
+  std::lock_guard<std::mutex> g(c->plain_mu);
+  if (c->ordered.mem) free_ordered(c);
+}
+
 int enqueue_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPlan& p,
                   double* d_dist, int* d_idx, bool timing) {
   const DevFrames& fit = s.fit;
@@ -1550,6 +1556,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
     return q.k_out;
   }
   HIP_TRY(c, hipSetDevice(c->device));
+  if (c->budget && !cv && server_idle(c)) drop_ordered(c);
   // A query that is not a self query does not need the self query's
   // mirrored lists; their memory goes back to the lists it does need.
   if (xyz && !cv) release_mirror_lists(c);
@@ -1874,18 +1881,18 @@ int mdsctk_knn_set_option(mdsctk_knn_ctx* c, int option, double value) {
   switch (option) {
     case MDSCTK_OPT_HBM_BUDGET:
       if (value < 0) return fail(c, MDSCTK_ERR_ARG, "budget must be >= 0");
-      if (value > 0 && !c->server) {
-        // no ordered copy under a budget (ensure_ordered): give back what an
-        // earlier one holds, so that the budget's queries have that room
-        std::lock_guard<std::mutex> g(c->plain_mu);
-        free_ordered(c);
-        dfree(c, c->main.ws_cross);
-        c->main.ws_cross = nullptr;
-        c->main.ws_cross_bytes = 0;
-      }
       {
         std::lock_guard<std::mutex> lk(c->mem_mu);  // the serving thread allocates too
         c->budget = (size_t)value;
+      }
+      if (value > 0) {
+        // no ordered copy under a budget (ensure_ordered): give back what an
+        // earlier one holds, so that the budget's queries have that room.
+        // While served requests are in flight the next query does.
+        dfree(c, c->main.ws_cross);
+        c->main.ws_cross = nullptr;
+        c->main.ws_cross_bytes = 0;
+        if (server_idle(c)) drop_ordered(c);
       }
       return 0;
     case MDSCTK_OPT_EPS_SCALE:

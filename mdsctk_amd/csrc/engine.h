@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <chrono>
 #include <cstdint>
 #include <mutex>
@@ -171,7 +172,7 @@ struct mdsctk_knn_ctx {
   int n_cu = 256;
   // Device memory accounting; the serving thread allocates too.
   mutable std::mutex mem_mu;
-  size_t budget = 0;  // 0 = unlimited
+  std::atomic<size_t> budget{0};  // 0 = unlimited; set under mem_mu
   size_t held = 0;
   std::unordered_map<void*, size_t> allocs;
   double eps_scale = 1.0;
@@ -249,6 +250,10 @@ int ensure_plain(mdsctk_knn_ctx* c, hipStream_t st);
 // take the ordered form) and, once they pay for it, orders the resident set for cross queries (synchronous, on slot s); no error if it
 // cannot.
 int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
+// Under an HBM budget, which the ordered copy is not made under: gives back
+// one made before.  No query that was planned before the budget was set may
+// still be running.
+void drop_ordered(mdsctk_knn_ctx* c);
 // Bytes of slot workspace the ordered form of a cross query of n_fit frames
 // takes (0: it takes every tile).
 size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);

@@ -135,6 +135,22 @@ class HipServeDevice {
     const QueryShape& q = b.q;
     const int natoms = c_->ref.natoms;
     int rc;
+    if (c_->budget) {
+      // set while serving ran: no batch takes the ordered copy any more, and
+      // once those in flight have ended nothing reads it
+      dfree(c_, s.ws_cross);
+      s.ws_cross = nullptr;
+      s.ws_cross_bytes = 0;
+      bool held;
+      {
+        std::lock_guard<std::mutex> g(c_->plain_mu);
+        held = c_->ordered.mem != nullptr;
+      }
+      if (held) {
+        for (auto& other : slots_) (void)hipStreamSynchronize(other.s.st);
+        drop_ordered(c_);
+      }
+    }
     if (sl.sized_limit < b.limit || sl.sized_k_out != q.k_out || sl.sized_k1 != q.k1)
       if ((rc = presize(sl, q, b.limit))) return rc;
     if ((rc = slot_frames(c_, s, b.n))) return rc;

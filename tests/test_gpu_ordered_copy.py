@@ -51,3 +51,39 @@ def test_served_batches_of_growing_size_allocate_nothing(frames):
             np.testing.assert_array_equal(r.idx, want[1][:m])
             np.testing.assert_array_equal(r.dist, want[0][:m])
             assert _held(ctx) == before
+
+
+@pytest.mark.parametrize("busy", [False, True])
+def test_budget_set_while_serving_gives_the_copy_back(frames, busy):
+    """At once when no request is in flight, else with the next batch."""
+    ref, fit = frames
+    with knn.KnnContext(0, "bf16") as ctx:
+        ctx.set_reference(ref)
+        want = ctx.query(fit, K)
+        plain = _held(ctx)
+        for _ in range(4):
+            ctx.query(fit, K)
+        made = _held(ctx)
+        assert made > plain + COPY
+        reqs = [ctx.submit(fit, K) for _ in range(12)]
+        if not busy:
+            for r in reqs:
+                ctx.wait(r)
+        before = _held(ctx)
+        ctx.set_option(knn.OPT_HBM_BUDGET, 64 << 30)
+        if not busy:
+            assert _held(ctx) < before - COPY
+        for r in reqs + [ctx.submit(fit, K)]:
+            ctx.wait(r)
+            np.testing.assert_array_equal(r.idx, want[1])
+            np.testing.assert_array_equal(r.dist, want[0])
+        d, i = ctx.query(fit, K)
+        np.testing.assert_array_equal(i, want[1])
+        held = _held(ctx)
+        # without the budget the copy comes back, and is what was missing
+        ctx.set_option(knn.OPT_HBM_BUDGET, 0)
+        for _ in range(5):
+            d, i = ctx.query(fit, K)
+        np.testing.assert_array_equal(i, want[1])
+        np.testing.assert_array_equal(d, want[0])
+        assert _held(ctx) > held + COPY
