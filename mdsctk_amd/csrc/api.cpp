@@ -1137,7 +1137,6 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     for (phases = 4; phases * blocks < 2 * grid; phases *= 2) {
     }
   phases = std::max(1, std::min(ref_pairs, phases));
-  const int nl = phases * 4;
   // Landmark pass: every lstride-th reference tile pair.  The (k+1)-th
   // smallest key of L landmarks ranks about (k+1) n / L among a row's n
   // keys, and a row may receive up to that many mirrored scores before its
@@ -1154,9 +1153,6 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
                                      (int)((int64_t)ref_pairs * 2 * kTile / lm_target))));
   const int lm_pairs = (ref_pairs + lstride - 1) / lstride;
   const int nlab = lm_pairs * 2 * kTile;
-  // its pairs as one list, split over enough phases to fill the grid
-  const int lm_phases = std::max(1, std::min({phases, lm_pairs, 2 * grid / blocks}));
-  const size_t ent_bytes = (size_t)n * nl * cap * sizeof(uint2);
   // Canonical form (kFilterMinFrames frames or more): the main pass runs over
   // a copy of the set in landmark order, for fitted scores with every frame in
   // its principal axes.  (Below that, ordering and copying cost more than the
@@ -1203,9 +1199,15 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
       2 * Carve::round((size_t)nlab * sizeof(int));
   bool band = canon;  // order by cells, the band pass, and if fitted the filter
   size_t sym_bytes = Carve::round(mir_bytes) + perm_bytes + (band ? filter_bytes : 0);
-  const size_t small = (size_t)n * nl * (sizeof(int) + sizeof(float)) +
-                       (size_t)n * 7 * sizeof(int) + (size_t)nlab * sizeof(int) +
-                       (size_t)(lm_pairs + 1) * sizeof(int) + 1024;
+  int nl = 0;
+  size_t ent_bytes = 0, small = 0;
+  auto size_lists = [&]() {
+    nl = phases * 4;
+    ent_bytes = (size_t)n * nl * cap * sizeof(uint2);
+    small = (size_t)n * nl * (sizeof(int) + sizeof(float)) + (size_t)n * 7 * sizeof(int) +
+            (size_t)nlab * sizeof(int) + (size_t)(lm_pairs + 1) * sizeof(int) + 1024;
+  };
+  size_lists();
   // Room: the free device memory plus what the buffers already hold, less a
   // reserve for everything else; and the context's budget.
   // (Buffers that are large enough already need no look at the device.)
@@ -1222,6 +1224,11 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     std::lock_guard<std::mutex> g(c->mem_mu);
     return !(c->budget && c->held - std::min(c->held, have) + need > c->budget);
   };
+  // Fewer phases, down to four, before anything else goes.
+  while (c->forced_phases <= 0 && phases > 4 && !fits()) {
+    phases /= 2;
+    size_lists();
+  }
   if (band && !fits()) {  // every tile is contracted instead
     band = false;
     sym_bytes = Carve::round(mir_bytes) + perm_bytes;
@@ -1241,6 +1248,8 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
     return 1;
   }
   if (rc) return rc;
+  // the landmark pairs as one list, split over enough phases to fill the grid
+  const int lm_phases = std::max(1, std::min({phases, lm_pairs, 2 * grid / blocks}));
   Lists L;
   L.nl = nl;
   L.cap = cap;
