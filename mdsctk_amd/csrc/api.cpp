@@ -1722,7 +1722,15 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
       // the exact path
       if (info.symmetric) {
         S.n_relisted_rows = (int64_t)rows.size();
-        if ((rc = relist_rows(c, s, q, rows, d_dist, d_idx))) return rc;
+        // Under a budget the rows need the room that the mirrored lists hold
+        // (read by the merge, which has ended); without room for theirs they
+        // take the exact rows, in batches that fit.
+        if (c->budget) release_mirror_lists(c);
+        rc = relist_rows(c, s, q, rows, d_dist, d_idx);
+        if (rc == MDSCTK_ERR_NOMEM)
+          forget_error(c);
+        else if (rc)
+          return rc;
       }
       if (!rows.empty()) {
         rc = exact_rows_select(c, ws, *fitp, rows.data(), (int)rows.size(), q, d_dist, d_idx, cv);

@@ -38,3 +38,27 @@ def test_symmetric_form_with_fewer_lists(frames):
         assert (st["n_pairs_landmark"] > 0, st["ref_splits"]) == (True, splits), part
         np.testing.assert_array_equal(rows[1], want[1])
         np.testing.assert_array_equal(rows[0], want[0])
+
+
+def test_rows_in_a_second_pass_fit_any_budget(frames):
+    """Short mirrored lists overflow, and their rows go through the candidate
+    lists once more: whatever the budget, also one that the first pass fills
+    to the last bytes, the query returns its rows."""
+    want, st, base = _query(frames, mirror_cap=8)
+    assert st["n_relisted_rows"] > 1000
+    size = st["device_bytes"] - base
+    # the largest use of each number of phases, and just above and below
+    for splits in (16, 8, 4):
+        lo, hi = 0.02, 1.4
+        for _ in range(22):
+            mid = (lo + hi) / 2
+            _, st, _ = _query(frames, int(base + mid * size), 8)
+            if st["n_pairs_landmark"] and st["ref_splits"] >= splits:
+                hi = mid
+            else:
+                lo = mid
+        edge = int(base + hi * size)
+        for budget in (edge - 70000, edge, edge + 1000, edge + 300000, edge + 4000000):
+            rows, st, _ = _query(frames, budget, 8)
+            np.testing.assert_array_equal(rows[1], want[1])
+            np.testing.assert_array_equal(rows[0], want[0])
