@@ -996,13 +996,6 @@ __global__ __launch_bounds__(256) void rank_sort_kernel(const unsigned* __restri
   if (wave == 0 && q < n) order[part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]] = q;
 }
 
-__global__ void stride_list_kernel(int ref_pairs, int stride, int* __restrict__ list,
-                                   int* __restrict__ count) {
-  const int m = (ref_pairs + stride - 1) / stride;
-  for (int i = threadIdx.x; i < m; i += blockDim.x) list[i] = i * stride;
-  if (threadIdx.x == 0) count[0] = m;
-}
-
 __global__ void rank_keys_kernel(const int* __restrict__ rank, int ncells, int64_t n,
                                  unsigned* __restrict__ keys) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1140,13 +1133,6 @@ hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, con
   hipLaunchKernelGGL(band_list_kernel, dim3((unsigned)(fit_tiles / ft)), dim3(64), 0, st,
                      ref_tiles / kRefTilesPerWG, fit_tiles / ft, ft / kRefTilesPerWG, width,
                      tl.list, tl.count);
-  return hipGetLastError();
-}
-
-hipError_t launch_stride_list(int ref_tiles, int stride, const TileList& tl, hipStream_t st) {
-  if (stride < 1 || !tl.shared) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(stride_list_kernel, dim3(1), dim3(256), 0, st, ref_tiles / kRefTilesPerWG,
-                     stride, tl.list, tl.count);
   return hipGetLastError();
 }
 

@@ -2329,6 +2329,16 @@ __global__ void order_scatter_kernel(const int* __restrict__ label, int64_t n,
   if (q < n) order[atomicAdd(&offsets[label[q]], 1)] = (int)q;
 }
 
+// Every stride-th reference pair.  (Here, not beside the filter's lists: every
+// query with a landmark or sample pass takes it, and a process's first launch
+// from another source's code object loads that object, 4 ms for the filter's.)
+__global__ void stride_list_kernel(int ref_pairs, int stride, int* __restrict__ list,
+                                   int* __restrict__ count) {
+  const int m = (ref_pairs + stride - 1) / stride;
+  for (int i = threadIdx.x; i < m; i += blockDim.x) list[i] = i * stride;
+  if (threadIdx.x == 0) count[0] = m;
+}
+
 __global__ void iota_kernel(int* __restrict__ p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = i;
@@ -2945,6 +2955,13 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
   const int64_t n = fit.n > 0 ? fit.n : 1;
   hipLaunchKernelGGL(eps_sym_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, fit.Gt,
                      ref.Gt, fit.n, ref.gmax, gmax_q, kappa, eps2, sum);
+  return hipGetLastError();
+}
+
+hipError_t launch_stride_list(int ref_tiles, int stride, const TileList& tl, hipStream_t st) {
+  if (stride < 1 || !tl.shared) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(stride_list_kernel, dim3(1), dim3(256), 0, st, ref_tiles / kRefTilesPerWG,
+                     stride, tl.list, tl.count);
   return hipGetLastError();
 }
 
