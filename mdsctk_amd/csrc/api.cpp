@@ -1374,18 +1374,20 @@ int launch_fused_sym(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, double* d_
   if (band) {
     // A band pass over the neighbours in that order tightens the thresholds
     // that the filter and the epilogue test against: each block against the
-    // reference pairs around it, into the first 4 lists.
+    // reference pairs around it, split over phases until the items fill the
+    // grid (two pairs each at least).
     tiles.list = (int*)fc.take(tiles_n * sizeof(int));
     tiles.count = (int*)fc.take(fit_blocks * sizeof(int));
     tiles.ctrl = (int*)fc.take(2 * sizeof(int));
     if (!tiles.list || !tiles.count || !tiles.ctrl)
       return fail(c, MDSCTK_ERR_ARG, "symmetric self query: band workspace carve");
+    const int width = std::min(ref_pairs, std::max(12, q.k1 / 8 + 2));
+    const int band_phases = std::max(1, std::min({phases, width / 2, 2 * grid / blocks}));
     Lists LB = LM;
-    LB.nl = 4;
+    LB.nl = 4 * band_phases;
     HIP_TRY(c, launch_init_lists(LB, n, s.st, false));
-    HIP_TRY(c, launch_band_list(c->ref.n_tiles, c->ref.n_tiles, kFilterFitTiles,
-                                std::min(ref_pairs, std::max(12, q.k1 / 8 + 2)), tiles, s.st));
-    HIP_TRY(c, launch_contract(mref, mfit, LB, meps2, q.k1, 1, q.nofit, nullptr, grid, s.st,
+    HIP_TRY(c, launch_band_list(c->ref.n_tiles, c->ref.n_tiles, kFilterFitTiles, width, tiles, s.st));
+    HIP_TRY(c, launch_contract(mref, mfit, LB, meps2, q.k1, band_phases, q.nofit, nullptr, grid, s.st,
                                nullptr, 0, &tiles));
     HIP_TRY(c, launch_landmark_cap(LB, n, q.k1, meps2, 1, LM.thr, nullptr, s.st));
   }
