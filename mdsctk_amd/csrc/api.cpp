@@ -606,11 +606,15 @@ int contract_grid(const mdsctk_knn_ctx* c, int ft) {
   return std::max(8, (c->n_cu * (ft <= 2 ? 2 : 1)) & ~7);
 }
 
-int fused_phases(const mdsctk_knn_ctx* c, int64_t n_fit) {
+int fused_phases(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
   const int ft = contract_fit_tiles(c->prec == kExact ? kFP32 : c->prec, n_fit);
   const int fit_blocks = ft == 1 ? 1 : std::max(1, std::max(kTileAlign, padded_tiles(n_fit)) / ft);
   const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
-  const int grid = contract_grid(c, ft);
+  // trace_kernel runs two workgroups a CU: 4000 x 20000 x 2000 --nofit, k 10,
+  // 5.3 ms with items for one on four XCDs, 3.9 on all eight, 3.3 with items
+  // for two (contract_kernel's trace form took 3.7)
+  const bool trace = q.nofit && ft == 4;
+  const int grid = contract_grid(c, ft) * (trace ? 2 : 1);
   int phases = c->forced_phases;
   if (phases <= 0) {
     // enough (fit block, phase) items to fill the grid, at least 8 phases
@@ -621,12 +625,13 @@ int fused_phases(const mdsctk_knn_ctx* c, int64_t n_fit) {
     while (p2 < phases) p2 <<= 1;
     phases = p2;
   }
-  return std::max(1, std::min(phases, ref_pairs));
+  // (its tiles are two reference pairs)
+  return std::max(1, std::min(phases, trace ? (ref_pairs + 1) / 2 : ref_pairs));
 }
 
-size_t fused_list_entries(const mdsctk_knn_ctx* c, int64_t n_fit, int k1) {
-  const int phases = fused_phases(c, n_fit);
-  return (size_t)n_fit * phases * 4 * list_capacity_for(k1);
+size_t fused_list_entries(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
+  const int phases = fused_phases(c, q, n_fit);
+  return (size_t)n_fit * phases * 4 * list_capacity_for(q.k1);
 }
 
 namespace {
@@ -786,7 +791,7 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
   const int cap = list_capacity_for(q.k1);
   p->ft = contract_fit_tiles(c->prec == kExact ? kFP32 : c->prec, n_fit);
   p->grid = contract_grid(c, p->ft);
-  p->phases = fused_phases(c, n_fit);
+  p->phases = fused_phases(c, q, n_fit);
   auto ent_bytes_for = [&](int phases) { return (size_t)n_fit * phases * 4 * cap * sizeof(uint2); };
   // A sample pass: 1/16 of the reference pairs, or enough
   // for 8 (k+1) frames.

@@ -261,8 +261,8 @@ size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);
 // batch of n_fit frames; candidate-list entries a batch of n_fit frames
 // needs (each entry 8 bytes; the headers take 8 bytes per list).
 int contract_grid(const mdsctk_knn_ctx* c, int ft);
-int fused_phases(const mdsctk_knn_ctx* c, int64_t n_fit);
-size_t fused_list_entries(const mdsctk_knn_ctx* c, int64_t n_fit, int k1);
+int fused_phases(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);
+size_t fused_list_entries(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);
 // The fused pipeline (lists, contraction, merge) for the slot's query
 // frames: plan_fused sizes the slot's workspace (it may allocate);
 // enqueue_fused only enqueues kernels on the slot's stream (with timing,

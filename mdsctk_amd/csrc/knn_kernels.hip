@@ -1535,14 +1535,14 @@ __global__ __launch_bounds__(256, 2) void trace_kernel(ContractParams P) {
       // copy of the one after goes into the buffer that every wave finished
       // reading before the last barrier.
       for (int g = 0; g < P.k_groups; ++g) {
-        trace_plane<PREC>(ax, sbuf0 + 2 * ri * SLOT, sbuf0 + (4 + 2 * fi) * SLOT, lane);
         copy(g, 2, d2);
+        trace_plane<PREC>(ax, sbuf0 + 2 * ri * SLOT, sbuf0 + (4 + 2 * fi) * SLOT, lane);
         stage_barrier<LPS>();
-        trace_plane<PREC>(ay, sbuf1 + 2 * ri * SLOT, sbuf1 + (4 + 2 * fi) * SLOT, lane);
         copy(g + 1, 0, d0);
+        trace_plane<PREC>(ay, sbuf1 + 2 * ri * SLOT, sbuf1 + (4 + 2 * fi) * SLOT, lane);
         stage_barrier<LPS>();
-        trace_plane<PREC>(az, sbuf2 + 2 * ri * SLOT, sbuf2 + (4 + 2 * fi) * SLOT, lane);
         copy(g + 1, 1, d1);
+        trace_plane<PREC>(az, sbuf2 + 2 * ri * SLOT, sbuf2 + (4 + 2 * fi) * SLOT, lane);
         stage_barrier<LPS>();
       }
       // read by the next tile's epilogue, after at least one more barrier
@@ -3082,10 +3082,13 @@ hipError_t launch_contract(const DevFrames& ref, const DevFrames& fit, const Lis
   if (ft == 1 && (ref.prec == kFP32 || dbg_scores || near || ball || mirror || (tiles && !tiles->shared)))
     return hipErrorInvalidValue;
   if (nofit && ft != 1 && ref.prec != kFP32) {
-    // trace_kernel: reference pairs in twos, all phases, two workgroups a CU
+    // trace_kernel: reference pairs in twos, all phases, two workgroups a CU;
+    // no more than there are items, since consecutive items go to one XCD
+    // (512 workgroups left four of the eight XCDs idle with 256 items)
     if (ph_run || ref.n_tiles % 4 || fit.n_tiles % 4 || (tiles && mirror))
       return hipErrorInvalidValue;
-    grid = dim3(2 * grid_wgs);
+    const int64_t items = (fit.n + 4 * kTile - 1) / (4 * kTile) * ref_phases;
+    grid = dim3((unsigned)std::min<int64_t>(2 * grid_wgs, (items + 7) & ~int64_t(7)));
   }
   switch (ref.prec) {
     case kFP32:

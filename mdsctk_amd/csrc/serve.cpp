@@ -266,7 +266,7 @@ class HipServeDevice {
     const size_t cap = (size_t)list_capacity_for(q.k1);
     for (int64_t n = std::min<int64_t>(limit, kTile);;
          n = std::min<int64_t>(limit, n < 128 ? 128 : n + 128)) {
-      const size_t e = fused_list_entries(c_, n, q.k1);
+      const size_t e = fused_list_entries(c_, q, n);
       *entries = std::max(*entries, e);
       *headers = std::max(*headers, e / cap);
       if (n == limit) break;
