@@ -725,18 +725,25 @@ int enqueue_ball_test(mdsctk_knn_ctx* c, const MiddleSet& ref, const DevFrames& 
 // Short queries: kSampleMinRef.  Longer ones: the pass (1/16 of the
 // contraction and a cap kernel, 50 us at least) against the epilogue's work
 // on the pairs that it rejects.  Measured, bf16, whole query without -> with:
-//   8000 x 8000 x 100, k 32, fitted 2.38 -> 1.92 ms, --nofit 1.55 -> 1.17
-//   2000 x 8000 x 100, k 32, fitted .78 -> .59,      --nofit .79 -> .46
-//   1500 x 20000 x 100, k 4, fitted 1.17 -> .79,     --nofit .68 -> .67
-//   2000 x 8000 x 600, k 4,  fitted 1.33 -> 1.37,    --nofit 1.23 -> 1.33
-//   1500 x 20000 x 2000, k 32,                       --nofit 3.54 -> 3.31
-//   8000 x 2000 x 100, k 32, fitted 1.18 -> 1.23,    --nofit 1.05 -> 1.11
-//   400 x 4000 x 100, k 32,  fitted .21 -> .25,      --nofit .20 -> .23
-// Without a QCP to save, a short list (k below 11) gains nothing.
+//   8000 x 8000 x 100, k 32, fitted 2.38 -> 1.92 ms
+//   2000 x 8000 x 100, k 32, fitted .78 -> .59
+//   1500 x 20000 x 100, k 4, fitted 1.17 -> .79
+//   2000 x 8000 x 600, k 4,  fitted 1.33 -> 1.37
+//   8000 x 2000 x 100, k 32, fitted 1.18 -> 1.23
+//   400 x 4000 x 100, k 32,  fitted .21 -> .25
+// trace_kernel, which without thresholds compacts every list of the chip after
+// its first tiles, gains at every length of frame and list:
+//   300 x 40000 x 304, k 2   .93 -> .37 ms
+//   2000 x 8000 x 304, k 2   .60 -> .34
+//   2000 x 5500 x 700, k 4   .73 -> .48
+//   2000 x 20000 x 1000, k 4 1.23 -> 1.03
+//   2000 x 3500 x 2000, k 4  .68 -> .79 (the one kind that loses)
+//   2000 x 20000 x 2000, k 30 2.37 -> 2.10
+// --nofit in FP32 goes as the fitted form: 2000 x 20000 x 700, k 2 1.83 -> 2.01.
 bool sampled_query(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
   if (n_fit < kCrossMinFit && c->ref.n >= kSampleMinRef) return true;
-  return c->ref.n >= 3000 && n_fit * c->ref.n >= 6000000 && c->ref.natoms <= 64 * q.k1 &&
-         (!q.nofit || q.k1 >= 12);
+  return c->ref.n >= 3000 && n_fit * c->ref.n >= 6000000 &&
+         ((q.nofit && c->prec != kFP32) || c->ref.natoms <= 64 * q.k1);
 }
 
 // The ordered form's workspace, carved from `cv` (or only its size).
