@@ -900,8 +900,9 @@ int plan_fused(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, FusedPlan* p, Ca
 namespace {
 
 // A cross query against the ordered set: a landmark pass (every lstride-th
-// reference pair) bounds each row's threshold and names its nearest landmark,
-// the queries are put in that order, the filter lists the tiles that can hold
+// reference pair as given) bounds each row's threshold and names its nearest
+// landmark, the queries are put in the order of these landmarks' places, the
+// filter lists the tiles that can hold
 // a candidate, and the contraction walks those.  The merge re-scores from the
 // frames as given, so outputs equal the unordered form's.
 int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPlan& p,
@@ -925,10 +926,10 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   HIP_TRY(c, launch_stride_list(c->ref.n_tiles, x.lstride, lm, s.st));
   HIP_TRY(c, launch_init_lists(LL, n, s.st));
   HIP_TRY(c, launch_eps(fit, R, p.kappa, x.eps0, s.sum, s.st));
-  HIP_TRY(c, launch_contract(R, fit, LL, x.eps0, q.k1, lm_phases, false, nullptr, p.grid, s.st,
+  HIP_TRY(c, launch_contract(c->ref, fit, LL, x.eps0, q.k1, lm_phases, false, nullptr, p.grid, s.st,
                              nullptr, 0, &lm));
   HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, x.eps0, x.lstride, x.thr0, x.label, s.st, 1, x.keys,
-                                 x.rows));
+                                 x.rows, nullptr, 0, o.place));
   if (x.sort_temp)
     HIP_TRY(c, launch_sort_order(nullptr, nullptr, 0, x.keys, x.keys_out, x.rows, x.order, n,
                                  x.sort_temp, x.sort_bytes, s.st));
@@ -940,6 +941,18 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   HIP_TRY(c, launch_filter_prep(src, c->w, o.sh, o.mean, o.mc, o.slots, x.order, x.set, s.st));
   HIP_TRY(c, launch_eps(x.fit, R, p.kappa, p.eps2, nullptr, s.st));
   HIP_TRY(c, launch_permute_thresholds(x.thr0, x.order, p.eps2, n, p.L.thr, s.st));
+  // a pass over the reference pairs around each block's places tightens them
+  const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
+  const int width = std::min(ref_pairs, std::max(3, q.k1 / 32 + 1));
+  const int most = std::max(8 * width, ref_pairs / 32);
+  Lists LB = p.L;
+  LB.nl = 4 * std::max(1, std::min({p.phases, most, 2 * p.grid / blocks}));
+  HIP_TRY(c, launch_init_lists(LB, n, s.st, false));
+  HIP_TRY(c, launch_place_band_list(x.keys, x.order, n, c->ref.n_tiles, x.fit.n_tiles, width,
+                                    most, x.tiles, s.st));
+  HIP_TRY(c, launch_contract(R, x.fit, LB, p.eps2, q.k1, LB.nl / 4, false, nullptr, p.grid, s.st,
+                             nullptr, 0, &x.tiles));
+  HIP_TRY(c, launch_landmark_cap(LB, n, q.k1, p.eps2, 1, p.L.thr, nullptr, s.st));
   HIP_TRY(c, launch_init_lists(p.L, n, s.st, false));
   HIP_TRY(c, launch_filter(o.set, x.set, c->ref.n, n, c->ref.n_tiles, x.fit.n_tiles, o.sh, o.mc,
                            p.L.thr, p.eps2, false, x.filter_grid, x.tiles, nullptr, s.st));
@@ -991,7 +1004,8 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
   const size_t bytes =
       Carve::round(rows * 3 * sizeof(double)) + 2 * Carve::round(rows * sizeof(double)) +
       Carve::round(opb) + Carve::round(rows * 9 * sizeof(double)) +
-      Carve::round((size_t)n * sizeof(int)) + Carve::round(filter_operand_bytes(o.sh, c->ref.n_tiles)) +
+      2 * Carve::round((size_t)n * sizeof(int)) +
+      Carve::round(filter_operand_bytes(o.sh, c->ref.n_tiles)) +
       2 * Carve::round(rows * sizeof(float4)) + Carve::round(rows * 12 * sizeof(double)) +
       Carve::round(rows * 36 * sizeof(ushort)) + Carve::round(o.sh.natoms * 3 * sizeof(double)) +
       Carve::round(o.sh.slots() * sizeof(int)) + Carve::round(sizeof(FilterMean));
@@ -1030,6 +1044,7 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
   f.op = (uint4*)cv.take(opb);
   f.rot = (double*)cv.take(rows * 9 * sizeof(double));
   o.order = (int*)cv.take((size_t)n * sizeof(int));
+  o.place = (int*)cv.take((size_t)n * sizeof(int));
   o.set.op = (uint4*)cv.take(filter_operand_bytes(o.sh, c->ref.n_tiles));
   o.set.full = (float4*)cv.take(rows * sizeof(float4));
   o.set.pre = (float4*)cv.take(rows * sizeof(float4));
@@ -1056,6 +1071,7 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
     HIP_TRY(c, launch_near_keys(near, n, lstride, keys, ids, s.st));
     HIP_TRY(c, launch_sort_order(nullptr, nullptr, 0, keys, keys_out, ids, o.order, n, temp,
                                  sort_temp, s.st));
+    HIP_TRY(c, launch_places(o.order, n, o.place, s.st));
     HIP_TRY(c, launch_prep(f, c->w, dithered(c) ? +1 : 0, nullptr, 0, s.st, c->ref.xyz, o.order,
                            f.rot));
     HIP_TRY(c, launch_filter_mean(c->ref, c->w, o.sh, align, o.mean, o.mc, o.slots, s.st));

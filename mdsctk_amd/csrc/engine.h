@@ -86,6 +86,7 @@ struct OrderedRef {
   void* mem = nullptr;
   DevFrames f;  // xyz null: the coordinates are the resident set's
   int* order = nullptr;
+  int* place = nullptr;  // place[order[i]] = i
   FilterShape sh;
   FilterSet set;
   double* mean = nullptr;

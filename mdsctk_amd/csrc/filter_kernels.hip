@@ -914,6 +914,41 @@ __global__ void band_list_kernel(int ref_pairs, int fit_blocks, int block_pairs,
   if (threadIdx.x == 0) count[fb] = m;
 }
 
+// The same for a cross query: the rows of a block are in the order of their
+// keys, places in the ordered set, and may stand around several of them: the
+// `width` reference pairs around each row's place.  One row without a
+// candidate nearby keeps every tile of its block, so all rows count unless
+// that makes more than `most` pairs; then every second, fourth ... row.
+__global__ __launch_bounds__(128) void place_band_list_kernel(const unsigned* __restrict__ keys,
+                                                              const int* __restrict__ order,
+                                                              int64_t n, int ref_pairs, int width,
+                                                              int most, int* __restrict__ list,
+                                                              int* __restrict__ count) {
+  constexpr int kRows = kFilterFitTiles * kTile;
+  __shared__ int at[kRows];
+  const int fb = blockIdx.x;
+  const int64_t row = min((int64_t)fb * kRows + threadIdx.x, n - 1);
+  at[threadIdx.x] = (int)(keys[order[row]] / (2u * kTile));
+  __syncthreads();
+  if (threadIdx.x) return;
+  int* const out = list + (int64_t)fb * ref_pairs;
+  auto walk = [&](int step, bool write) {
+    int m = 0, end = 0;
+    for (int r = step / 2; r < kRows; r += step) {
+      const int lo = max(max(0, min(at[r] - width / 2, ref_pairs - width)), end);
+      const int hi = min(max(0, min(at[r] - width / 2, ref_pairs - width)) + width, ref_pairs);
+      if (write)
+        for (int p = lo; p < hi; ++p) out[m + p - lo] = p;
+      m += max(0, hi - lo);
+      end = max(end, hi);
+    }
+    return m;
+  };
+  int step = 1;
+  while (step < kRows / 4 && walk(step, false) > most) step *= 2;
+  count[fb] = walk(step, true);
+}
+
 __global__ void clear_kernel(uint4* p, int64_t n, int* ctrl) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = make_uint4(0, 0, 0, 0);
@@ -962,6 +997,11 @@ __global__ void near_keys_kernel(const unsigned long long* __restrict__ near, in
   keys[q] = (cell << kFilterDistBits) |
             ((unsigned)(b >> 32) >> (31 - kFilterDistBits) & ((1u << kFilterDistBits) - 1u));
   rows[q] = (int)q;
+}
+
+__global__ void places_kernel(const int* __restrict__ order, int64_t n, int* __restrict__ place) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) place[order[i]] = (int)i;
 }
 
 // order[place of row q among the keys] = q: 64 rows a workgroup against all
@@ -1133,6 +1173,21 @@ hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, con
   hipLaunchKernelGGL(band_list_kernel, dim3((unsigned)(fit_tiles / ft)), dim3(64), 0, st,
                      ref_tiles / kRefTilesPerWG, fit_tiles / ft, ft / kRefTilesPerWG, width,
                      tl.list, tl.count);
+  return hipGetLastError();
+}
+
+hipError_t launch_place_band_list(const unsigned* keys, const int* order, int64_t n, int ref_tiles,
+                                  int fit_tiles, int width, int most, const TileList& tl,
+                                  hipStream_t st) {
+  if (n < 1 || width < 1 || fit_tiles % kFilterFitTiles) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(place_band_list_kernel, dim3((unsigned)(fit_tiles / kFilterFitTiles)), dim3(128),
+                     0, st, keys, order, n, ref_tiles / kRefTilesPerWG, width, most, tl.list, tl.count);
+  return hipGetLastError();
+}
+
+hipError_t launch_places(const int* order, int64_t n, int* place, hipStream_t st) {
+  hipLaunchKernelGGL(places_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, order, n,
+                     place);
   return hipGetLastError();
 }
 

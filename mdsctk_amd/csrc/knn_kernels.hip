@@ -2185,7 +2185,8 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
                                                            unsigned* __restrict__ keys,
                                                            int* __restrict__ rows,
                                                            int* __restrict__ leaders,
-                                                           int leader_rank) {
+                                                           int leader_rank,
+                                                           const int* __restrict__ place) {
   const int64_t q = blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   __shared__ unsigned hist[256];
@@ -2246,8 +2247,11 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
       // cell number, then the distance's leading 19 bits (its exponent and
       // 11 of the fraction): enough to lay like distances side by side
       const unsigned long long b = s_cell != ~0ull ? s_cell : s_best;
-      const unsigned lab = b != ~0ull ? dense((unsigned)(b & 0xffffffffu)) / (unsigned)cell : 0u;
-      keys[q] = (lab << 19) | ((unsigned)(b >> 32) >> 12 & 0x7ffffu);
+      const unsigned r = (unsigned)(b & 0xffffffffu);
+      const unsigned lab = b != ~0ull ? dense(r) / (unsigned)cell : 0u;
+      keys[q] = place ? (b != ~0ull ? (unsigned)place[r] : 0u)
+                      : (lab << kFilterDistBits) |
+                            ((unsigned)(b >> 32) >> (31 - kFilterDistBits) & ((1u << kFilterDistBits) - 1u));
       rows[q] = (int)q;
     }
   }
@@ -3201,7 +3205,8 @@ hipError_t launch_permute_thresholds(const unsigned* src, const int* perm, const
 
 hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* eps2,
                                int phases, unsigned* thr, int* label, hipStream_t st, int cell,
-                               unsigned* keys, int* rows, int* leaders, int leader_rank) {
+                               unsigned* keys, int* rows, int* leaders, int leader_rank,
+                               const int* place) {
   if (n <= 0) return hipSuccess;
   if (k1 < 1 || phases < 1 || !thr || cell < 1 || (keys && (!label || !rows)))
     return hipErrorInvalidValue;
@@ -3211,7 +3216,7 @@ hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* e
                        ncells);
   }
   hipLaunchKernelGGL(landmark_cap_kernel, dim3((unsigned)n), dim3(256), 0, st, L.ent, L.cnt, L.nl,
-                     L.cap, k1, eps2, phases, thr, label, cell, keys, rows, leaders, leader_rank);
+                     L.cap, k1, eps2, phases, thr, label, cell, keys, rows, leaders, leader_rank, place);
   return hipGetLastError();
 }
 

@@ -87,3 +87,36 @@ def test_budget_set_while_serving_gives_the_copy_back(frames, busy):
         np.testing.assert_array_equal(i, want[1])
         np.testing.assert_array_equal(d, want[0])
         assert _held(ctx) > held + COPY
+
+
+@pytest.mark.parametrize("prec", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("gen,n_ref,natoms,n_fit,k", [
+    ("states", 16385, 260, 2500, 1), ("states", 16385, 260, 2300, 70), ("basin", 15000, 290, 2100, 12),
+    ("loose", 10007, 420, 4097, 5), ("copies", 12000, 350, 3000, 30), ("states", 9000, 470, 17000, 9)])
+def test_ordered_rows_equal_the_unordered_ones(gen, n_ref, natoms, n_fit, k, prec):
+    """Blocks around one place and around many, unrelated frames (more places
+    than a block's pass takes), a resident set of 40 frames' copies (equal
+    keys), more query frames than the rank sort takes."""
+    rng = np.random.default_rng(n_ref)
+    n = n_ref + n_fit
+    if gen == "states":
+        x = synth.metastable_trajectory(n, natoms, 3, n_centres=50)
+    elif gen == "basin":
+        x = synth.trajectory(n, natoms, 4)
+    elif gen == "loose":
+        x = np.stack([synth.random_walk(natoms, rng) for _ in range(n)]).astype(np.float32)
+    else:
+        x = synth.metastable_trajectory(40, natoms, 3, n_centres=40)[rng.integers(0, 40, n)]
+    ref, fit = x[:n_ref], x[n_ref:]
+    w = synth.masses(natoms, "random", 2)
+    with knn.KnnContext(0, prec) as ctx:
+        ctx.set_option(knn.OPT_HBM_BUDGET, 200e9)  # no copy under a budget
+        ctx.set_reference(ref, w)
+        d0, i0 = ctx.query(fit, k)
+        ctx.set_option(knn.OPT_HBM_BUDGET, 0)
+        plain = _held(ctx)
+        for _ in range(8192 // n_fit + 2):
+            d, i = ctx.query(fit, k)
+        assert _held(ctx) > plain + n_ref * natoms * (6 if prec == "fp32" else 12)
+    np.testing.assert_array_equal(i, i0)
+    np.testing.assert_array_equal(d, d0)
