@@ -967,8 +967,28 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
 
 }  // namespace
 
+namespace {
+
+// Whether a query is long enough for the ordered form: its launches and the
+// passes over the query frames against the pairs that it saves.  Measured,
+// whole query unordered -> ordered, k 10, one basin | 50 states:
+//   600 x 50000 x 304    bf16  .96 -> 1.13 ms | 1.04 -> 1.39
+//   1200 x 32000 x 304        1.22 -> 1.13    | 1.34 -> 1.33
+//   2500 x 15000 x 304        1.27 -> 1.16    | 1.44 -> 1.29
+//   1200 x 15000 x 1000       1.86 -> 1.61    | 2.02 -> 2.00
+//   2500 x 10000 x 2000       4.37 -> 4.15    | 4.56 -> 4.69
+//   1200 x 15000 x 304   fp32 1.71 -> 1.31    | 1.80 -> 1.90
+// A set of 8192 frames takes 1.2 to 3 times as long with 256 of them.
+bool cross_pays(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
+  if (!q.fused || q.nofit || n_fit < kCrossMinFit) return false;
+  const double pairs = (1.2e7 + 2.4e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.7 : 1.0);
+  return (double)n_fit * (double)c->ref.n >= pairs;
+}
+
+}  // namespace
+
 size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
-  if (!q.fused || q.nofit || n_fit < kCrossMinFit || c->budget) return 0;
+  if (!cross_pays(c, q, n_fit) || c->budget) return 0;
   {
     std::lock_guard<std::mutex> g(c->plain_mu);
     if (!c->ordered.built) return 0;
@@ -985,9 +1005,9 @@ size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
 // done when the frames queried so far reach kCrossMinSeen.  Not under an HBM
 // budget, nor when it would take more than a quarter of the free memory:
 // the other workspaces keep their room.
-int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit) {
+int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, int64_t n_fit) {
   const int64_t n = c->ref.n;
-  if (n_fit < kCrossMinFit) return 0;  // such queries never walk the copy
+  if (!cross_pays(c, q, n_fit)) return 0;  // such queries never walk the copy
   if (!c->ref_axes || n < kCrossMinRef || n * c->ref.natoms < kCrossMinWork || c->budget) return 0;
   std::lock_guard<std::mutex> g(c->plain_mu);
   OrderedRef& o = c->ordered;
@@ -1685,7 +1705,7 @@ int query_impl(mdsctk_knn_ctx* c, const void* xyz, bool data, bool on_device, in
   int fused_rc = 1;  // 1: the fused pipeline did not run
   FusedInfo info;
   if (!q.full && q.fused && !plain_missing) {
-    if (xyz && !cv && !q.nofit && (rc = ensure_ordered(c, s, n_fit))) return rc;
+    if (xyz && !cv && !q.nofit && (rc = ensure_ordered(c, s, q, n_fit))) return rc;
     DevFrames saved = ws.fit;
     if (!xyz) ws.fit = query_view(ref_ops(c, q.nofit));
     if (!xyz && c->self_sym && !cv) fused_rc = launch_fused_sym(c, ws, q, d_dist, d_idx, &info);

@@ -247,10 +247,10 @@ int slot_frames(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
 int prep_slot(mdsctk_knn_ctx* c, Slot& s, bool nofit);
 // The resident set's --nofit operands, built on first use (synchronous).
 int ensure_plain(mdsctk_knn_ctx* c, hipStream_t st);
-// Counts a fitted query's frames (of kCrossMinFit or more: shorter ones never
-// take the ordered form) and, once they pay for it, orders the resident set for cross queries (synchronous, on slot s); no error if it
+// Counts a fitted query's frames (if it is long enough for the ordered form)
+// and, once they pay for it, orders the resident set for cross queries (synchronous, on slot s); no error if it
 // cannot.
-int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, int64_t n_fit);
+int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, int64_t n_fit);
 // Under an HBM budget, which the ordered copy is not made under: gives back
 // one made before.  No query that was planned before the budget was set may
 // still be running.

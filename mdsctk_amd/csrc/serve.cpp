@@ -178,7 +178,7 @@ class HipServeDevice {
     }
     sl.all_exact = !fused;
     if (fused) {
-      if (!q.nofit && (rc = ensure_ordered(c_, s, b.n))) return rc;
+      if (!q.nofit && (rc = ensure_ordered(c_, s, q, b.n))) return rc;
       FusedPlan plan;
       if ((rc = plan_fused(c_, s, q, &plan))) return rc;
       if (c_->serve_share_cus && slots_.size() > 1) {

@@ -7,7 +7,7 @@ from mdsctk_amd import knn, synth
 
 pytestmark = pytest.mark.gpu
 
-N_REF, NATOMS, K = 8200, 520, 12
+N_REF, NATOMS, K = 20000, 520, 12
 COPY = 12 * N_REF * NATOMS  # bytes of the copy's operand alone
 
 
@@ -22,16 +22,18 @@ def _held(ctx):
 
 
 def test_short_queries_do_not_make_the_copy(frames):
-    """Queries below 256 frames never walk the copy, however many there are."""
+    """Queries below 256 frames never walk the copy, nor do those whose pairs
+    are too few for it (800 frames here), however many there are."""
     ref, fit = frames
-    with knn.KnnContext(0, "bf16") as ctx:
-        ctx.set_reference(ref)
-        want = ctx.query(fit[:255], K)
-        before = _held(ctx)
-        for _ in range(40):
-            d, i = ctx.query(fit[:255], K)
-        np.testing.assert_array_equal(i, want[1])
-        assert _held(ctx) == before
+    for m in (255, 800):
+        with knn.KnnContext(0, "bf16") as ctx:
+            ctx.set_reference(ref)
+            want = ctx.query(fit[:m], K)
+            before = _held(ctx)
+            for _ in range(9000 // m + 1):
+                d, i = ctx.query(fit[:m], K)
+            np.testing.assert_array_equal(i, want[1])
+            assert _held(ctx) == before
 
 
 def test_served_batches_of_growing_size_allocate_nothing(frames):
@@ -44,9 +46,9 @@ def test_served_batches_of_growing_size_allocate_nothing(frames):
         want = ctx.query(fit, K)
         for _ in range(4):
             ctx.query(fit, K)
-        ctx.wait(ctx.submit(fit[:300], K))
+        ctx.wait(ctx.submit(fit[:900], K))
         before = _held(ctx)
-        for m in (300, 640, 1100, 2048, 1999):
+        for m in (900, 300, 1100, 2048, 1999):
             r = ctx.wait(ctx.submit(fit[:m], K))
             np.testing.assert_array_equal(r.idx, want[1][:m])
             np.testing.assert_array_equal(r.dist, want[0][:m])
