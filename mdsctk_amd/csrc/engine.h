@@ -130,7 +130,13 @@ struct FusedPlan {
   int* sample_list = nullptr;
   double kappa = 0;
   CrossPlan x;
-  int kind() const { return x.on ? 2 : sample ? 1 : 0; }  // sequence of kernels
+  // Which kernels run, in which sequence, for one k and one set of flags: a
+  // captured graph is updated in place only by another of its kind.
+  static constexpr int kKinds = 8;
+  int kind(int64_t n_fit) const {
+    const bool wide = n_fit <= kMergeWideRows;
+    return x.on ? 6 + wide : (sample ? 3 : 0) + (ft == 1 ? 2 : wide);
+  }
 };
 
 // What the fused pipeline did for a batch.

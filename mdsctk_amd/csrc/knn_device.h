@@ -170,6 +170,9 @@ constexpr int kFilterMaxCells = 8000;
 constexpr int64_t kBallRowsMax = 65536;
 constexpr int kFilterDistBits = 19;
 
+// Rows up to which the merge takes 1024 threads a row.
+constexpr int64_t kMergeWideRows = 256;
+
 // How a frame's atoms are laid out: one or two segments, each a whole number
 // of units of four stages of gps K-groups (16 slots each).
 struct FilterShape {

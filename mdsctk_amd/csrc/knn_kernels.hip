@@ -3171,7 +3171,7 @@ hipError_t launch_merge(const DevFrames& ref, const DevFrames& fit, const DevWei
   const bool stage = w.metric == kMetricRMSD && ref.natoms <= kMergeStageAtoms;
   const size_t dyn = stage ? (size_t)ref.natoms * 3 * sizeof(double) : 0;
   // few rows: a CU or more to each
-  const bool wide = fit.n <= 256;
+  const bool wide = fit.n <= kMergeWideRows;
   const dim3 grid((unsigned)fit.n);
 #define MDSCTK_MERGE(ST, CA)                                                                 \
   do {                                                                                       \

@@ -45,12 +45,12 @@ struct HipSlot {
   hipEvent_t done = nullptr;
   // the slot's batch kernels, updated per batch: one per
   // sequence of kernels (FusedPlan::kind)
-  hipGraphExec_t exec[3] = {};
+  hipGraphExec_t exec[FusedPlan::kKinds] = {};
   // the captured graph exec was last instantiated or updated from; kept
   // until a later capture has replaced it in exec (and that exec has been
   // launched), so nothing the executable may refer to is released while it
   // can still run
-  hipGraph_t graph[3] = {};
+  hipGraph_t graph[FusedPlan::kKinds] = {};
   // shape the workspace was last sized for
   int64_t sized_limit = 0;
   int sized_k_out = -1, sized_k1 = -1;
@@ -365,8 +365,8 @@ class HipServeDevice {
   // then never reads released memory).
   int replay_graph(HipSlot& sl, const QueryShape& q, const FusedPlan& plan) {
     Slot& s = sl.s;
-    hipGraphExec_t& exec = sl.exec[plan.kind()];
-    hipGraph_t& graph = sl.graph[plan.kind()];
+    hipGraphExec_t& exec = sl.exec[plan.kind(s.fit.n)];
+    hipGraph_t& graph = sl.graph[plan.kind(s.fit.n)];
     hipError_t e = hipStreamBeginCapture(s.st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return hip_fail(c_, e, "serve: graph capture");
     int rc = prep_slot(c_, s, q.nofit);
