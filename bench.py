@@ -622,7 +622,7 @@ def main():
     out["ms_per_step"] = wall * 1e3
     out["config"]["self_symmetric"] = bool(computed < pairs)
     out["config"]["pairs_per_step"] = pairs
-    out["config"]["pairs_scored_per_step"] = computed
+    out["config"]["pairs_covered_per_step"] = computed
     if "ms" in first:
         out["first_query_ms"] = first["ms"]
     # Matrix operations of the contraction's span as the hardware counted them:

@@ -121,8 +121,10 @@ typedef struct mdsctk_knn_stats {
   int32_t ref_splits;      /* reference phases used by the contraction */
   int32_t list_capacity;   /* per-list candidate capacity */
   double eps_rel;          /* candidate window relative to (G_q + max G_ref) */
-  int64_t n_pairs_computed; /* pairs the contraction scored: n_pairs, or about half of
-                               them for a symmetric self query */
+  int64_t n_pairs_computed; /* pairs that the query's form covers: n_pairs, or for a
+                               symmetric self query its upper block triangle (about
+                               half).  A fitted query on a large set contracts only
+                               those of their tiles that can hold a neighbour */
   double ms_landmark;       /* symmetric self query: its landmark pass (thresholds) */
   int64_t n_pairs_landmark; /* pairs the landmark pass scored */
   int64_t n_mirrored;       /* scores appended to frames' mirrored lists */
