@@ -684,7 +684,7 @@ size_t middles_bytes(const mdsctk_knn_ctx* c, int64_t n, bool dith) {
 
 // The middles' operands (of `side`, and the query side where they have one)
 // and balls; src: the frames as given, order their order, thr and eps2 the
-// ordered rows' thresholds and windows (null on a side without).
+// ordered rows' thresholds and windows.
 int enqueue_middles(mdsctk_knn_ctx* c, const DevFrames& src, const int* order, int side,
                     const unsigned* thr, const float* eps2, const MiddleSet& m, hipStream_t st) {
   HIP_TRY(c, launch_middle(order, src.n, m.mid, st));
@@ -788,6 +788,37 @@ size_t carve_cross(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit, Carve&
   x->tiles.ctrl = (int*)cv.take(2 * sizeof(int));
   x->lstride = cross_stride(c, q.k1);
   return cv.used;
+}
+
+// Whether a query is long enough for the ordered form: its launches and the
+// passes over the query frames against the pairs that it saves.  Measured,
+// whole query unordered -> ordered, k 10, one basin | 50 states:
+//   600 x 50000 x 304    bf16  .96 -> 1.13 ms | 1.04 -> 1.39
+//   1200 x 32000 x 304        1.22 -> 1.13    | 1.34 -> 1.33
+//   2500 x 15000 x 304        1.27 -> 1.16    | 1.44 -> 1.29
+//   1200 x 15000 x 1000       1.86 -> 1.61    | 2.02 -> 2.00
+//   2500 x 10000 x 2000       4.37 -> 4.15    | 4.56 -> 4.69
+//   1200 x 15000 x 304   fp32 1.71 -> 1.31    | 1.80 -> 1.90
+// A set of 8192 frames takes 1.2 to 3 times as long with 256 of them.
+bool cross_pays(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
+  if (!q.fused || q.nofit || n_fit < kCrossMinFit) return false;
+  const double pairs = (1.2e7 + 2.4e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.7 : 1.0);
+  return (double)n_fit * (double)c->ref.n >= pairs;
+}
+
+// Bytes of slot workspace the ordered form of a cross query of n_fit frames
+// takes (0: it takes every tile).
+size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
+  if (!cross_pays(c, q, n_fit) || c->budget) return 0;
+  {
+    std::lock_guard<std::mutex> g(c->plain_mu);
+    if (!c->ordered.built) return 0;
+  }
+  Carve cv;
+  cv.base = (char*)256;  // sizes only
+  cv.size = SIZE_MAX / 2;
+  CrossPlan x;
+  return carve_cross(c, q, n_fit, cv, &x);
 }
 
 }  // namespace
@@ -901,10 +932,11 @@ namespace {
 
 // A cross query against the ordered set: a landmark pass (every lstride-th
 // reference pair as given) bounds each row's threshold and names its nearest
-// landmark, the queries are put in the order of these landmarks' places, the
-// filter lists the tiles that can hold
-// a candidate, and the contraction walks those.  The merge re-scores from the
-// frames as given, so outputs equal the unordered form's.
+// landmark, the queries are put in the order of these landmarks' places, a
+// pass around each block's places tightens the thresholds, the filter lists
+// the tiles that can hold a candidate, and the contraction walks those.  The
+// merge re-scores from the frames as given, so outputs equal the unordered
+// form's.
 int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPlan& p,
                   double* d_dist, int* d_idx, bool timing) {
   const DevFrames& fit = s.fit;
@@ -966,39 +998,6 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
 }
 
 }  // namespace
-
-namespace {
-
-// Whether a query is long enough for the ordered form: its launches and the
-// passes over the query frames against the pairs that it saves.  Measured,
-// whole query unordered -> ordered, k 10, one basin | 50 states:
-//   600 x 50000 x 304    bf16  .96 -> 1.13 ms | 1.04 -> 1.39
-//   1200 x 32000 x 304        1.22 -> 1.13    | 1.34 -> 1.33
-//   2500 x 15000 x 304        1.27 -> 1.16    | 1.44 -> 1.29
-//   1200 x 15000 x 1000       1.86 -> 1.61    | 2.02 -> 2.00
-//   2500 x 10000 x 2000       4.37 -> 4.15    | 4.56 -> 4.69
-//   1200 x 15000 x 304   fp32 1.71 -> 1.31    | 1.80 -> 1.90
-// A set of 8192 frames takes 1.2 to 3 times as long with 256 of them.
-bool cross_pays(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
-  if (!q.fused || q.nofit || n_fit < kCrossMinFit) return false;
-  const double pairs = (1.2e7 + 2.4e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.7 : 1.0);
-  return (double)n_fit * (double)c->ref.n >= pairs;
-}
-
-}  // namespace
-
-size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
-  if (!cross_pays(c, q, n_fit) || c->budget) return 0;
-  {
-    std::lock_guard<std::mutex> g(c->plain_mu);
-    if (!c->ordered.built) return 0;
-  }
-  Carve cv;
-  cv.base = (char*)256;  // sizes only
-  cv.size = SIZE_MAX / 2;
-  CrossPlan x;
-  return carve_cross(c, q, n_fit, cv, &x);
-}
 
 // Ordering costs about a landmark pass of the whole set (L landmarks a
 // frame) and two operand builds, and saves most of a query's pairs: it is

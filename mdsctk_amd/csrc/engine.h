@@ -67,10 +67,6 @@ struct QueryShape {
   bool fused = false;  // contraction + merge (else exact rows)
 };
 
-// The resident set in the order its cross queries walk it: rows sorted into
-// cells around landmarks, their contraction operand and their filter operand
-// (filter_kernels.hip).  Made once, when queries have brought enough frames
-// to pay for it; only read afterwards.
 // The middle frames of every 64 of an ordered set, as frames of their own,
 // and the balls around them (BallTest).
 struct MiddleSet {
@@ -79,10 +75,14 @@ struct MiddleSet {
   float2* ball = nullptr;
 };
 
+// The resident set in the order its cross queries walk it: rows sorted into
+// cells around landmarks, their contraction operand and their filter operand
+// (filter_kernels.hip).  Made once, when queries have brought enough frames
+// to pay for it; only read afterwards.
 struct OrderedRef {
   bool built = false;
   bool failed = false;  // its kernels failed: not tried again
-  int64_t seen = 0;  // frames, since the set became resident, of queries that could use it
+  int64_t seen = 0;     // frames, since the set became resident, of queries that could use it
   void* mem = nullptr;
   DevFrames f;  // xyz null: the coordinates are the resident set's
   int* order = nullptr;
@@ -95,7 +95,8 @@ struct OrderedRef {
 };
 
 // A cross query against the ordered set: the query frames in the order of
-// their nearest landmark, and the tiles that can hold a candidate.
+// their nearest landmarks' places in it, and the tiles that can hold a
+// candidate.
 struct CrossPlan {
   bool on = false;
   int lstride = 1;  // every lstride-th reference pair is a landmark pair
@@ -145,7 +146,9 @@ struct FusedInfo {
   int cap = 0;
   double kappa = 0;
   int* d_fallback = nullptr;  // [n_fit] device flags (in the slot's workspace)
-  int64_t pairs_computed = 0;  // pairs the main contraction scored
+  // pairs the form covers: all, or the upper block triangle (of which a
+  // filtered query contracts only the tiles that can hold a neighbour)
+  int64_t pairs_computed = 0;
   // symmetric self query only
   bool symmetric = false;
   int64_t pairs_landmark = 0;  // pairs of its landmark pass (0: none)
@@ -254,16 +257,13 @@ int prep_slot(mdsctk_knn_ctx* c, Slot& s, bool nofit);
 // The resident set's --nofit operands, built on first use (synchronous).
 int ensure_plain(mdsctk_knn_ctx* c, hipStream_t st);
 // Counts a fitted query's frames (if it is long enough for the ordered form)
-// and, once they pay for it, orders the resident set for cross queries (synchronous, on slot s); no error if it
-// cannot.
+// and, once they pay for it, orders the resident set for cross queries
+// (synchronous, on slot s); no error if it cannot.
 int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, int64_t n_fit);
 // Under an HBM budget, which the ordered copy is not made under: gives back
 // one made before.  No query that was planned before the budget was set may
 // still be running.
 void drop_ordered(mdsctk_knn_ctx* c);
-// Bytes of slot workspace the ordered form of a cross query of n_fit frames
-// takes (0: it takes every tile).
-size_t cross_bytes(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit);
 // Contraction grid (workgroups of ft fit tiles) and reference phases for a
 // batch of n_fit frames; candidate-list entries a batch of n_fit frames
 // needs (each entry 8 bytes; the headers take 8 bytes per list).

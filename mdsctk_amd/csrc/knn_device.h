@@ -232,7 +232,7 @@ struct BallTest {
 hipError_t launch_middle(const int* order, int64_t n, int* mid, hipStream_t st);
 // ball[g] = (radius of the g-th 64 frames of the order around mid[g]: an upper
 // bound of sqrt(score); square root of the largest thr + eps2 / 2 of their
-// rows, 0 without thr).
+// rows).
 hipError_t launch_balls(const DevFrames& f, const DevWeights& w, const int* order, const int* mid,
                         const unsigned* thr, const float* eps2, float2* ball, hipStream_t st);
 hipError_t launch_row_balls(const unsigned* thr, const float* eps2, int64_t n, float2* ball,
@@ -265,10 +265,10 @@ hipError_t launch_place_band_list(const unsigned* keys, const int* order, int64_
                                   hipStream_t st);
 // Every stride-th reference pair, as a list shared by every block.
 hipError_t launch_stride_list(int ref_tiles, int stride, const TileList& tl, hipStream_t st);
-// The resident set's order for cross queries, from each frame's nearest
-// landmark (near: launch_contract): keys[q] = cell and distance, rows[q] = q.
 // place[order[i]] = i.
 hipError_t launch_places(const int* order, int64_t n, int* place, hipStream_t st);
+// The resident set's order for cross queries, from each frame's nearest
+// landmark (near: launch_contract): keys[q] = cell and distance, rows[q] = q.
 hipError_t launch_fill_near(unsigned long long* near, int64_t n, hipStream_t st);
 hipError_t launch_near_keys(const unsigned long long* near, int64_t n, int phases, unsigned* keys,
                             int* rows, hipStream_t st);
@@ -309,8 +309,8 @@ hipError_t launch_eps(const DevFrames& fit, const DevFrames& ref, double kappa, 
 // only: each pair joins the fit frame's lists and, contracted one way round
 // only, the reference frame's mirrored list when it lies below that
 // frame's shared threshold L.thr.  ph_run < ref_phases walks phases
-// 0..ph_run-1 only (every ref_phases-th reference tile pair: the landmark
-// pass); 0 = all.  tiles: only the listed reference pairs of each block of
+// 0..ph_run-1 only (1: every ref_phases-th reference tile pair, the landmarks
+// that the resident set is ordered around); 0 = all.  tiles: only the listed reference pairs of each block of
 // kFilterFitTiles fit tiles, dealt out over the phases.  near: no lists, only
 // each fit frame's smallest (key << 32 | reference) there (atomic minimum).
 // ft 1: the one-fit-tile workgroup of short queries (contract_fit_tiles).

@@ -588,8 +588,8 @@ struct ContractParams {
   int nofit;
   double* dbg;
   // Reference phases actually walked: items are (fit block, phase) for
-  // phases 0..ph_run-1 (ph_run < phases: every phases-th reference tile
-  // pair only, the landmark pass of a symmetric self query).
+  // phases 0..ph_run-1 (1 of them: every phases-th reference tile pair only,
+  // the landmarks that the resident set is ordered around).
   int ph_run;
   // kOutSym: one list per reference frame for the scores it receives as
   // the reference side of a pair (mcap entries each, appended through the
@@ -981,9 +981,9 @@ __device__ __forceinline__ void stage_barrier_vm() {
   asm volatile("" ::: "memory");
 }
 
-// FT = fit tiles per workgroup (2 or 4); the workgroup has 2*FT waves, one
-// per (reference tile, fit tile) pair.  MODE: kOutLists, kOutDebug or
-// kOutSym.
+// FT = fit tiles per workgroup (FP32 2; the split forms 4, or 1 for queries of
+// one tile); the workgroup has 2*FT waves, one per (reference tile, fit tile)
+// pair.  MODE: one of kOut*.
 template <int PREC, int PER, int FT, int MODE, bool TRACE>
 __global__ __launch_bounds__(64 * kRefTilesPerWG * FT, 2) void contract_kernel(ContractParams P) {
   constexpr int BPG = (PREC == kFP32) ? 3 : 6;
@@ -1807,7 +1807,7 @@ __global__ __launch_bounds__(256) void ball_kernel(
     far = fmax(far, s);
   }
   float big = 0.f;
-  if (thr && tid < 2 * kTile && f0 + tid < n)
+  if (tid < 2 * kTile && f0 + tid < n)
     big = __uint_as_float(thr[f0 + tid]) + 0.5f * eps2[f0 + tid];
   __shared__ double sfar[16];
   __shared__ float sbig[2 * kTile];
@@ -3238,7 +3238,7 @@ hipError_t launch_row_balls(const unsigned* thr, const float* eps2, int64_t n, f
 hipError_t launch_balls(const DevFrames& f, const DevWeights& w, const int* order, const int* mid,
                         const unsigned* thr, const float* eps2, float2* ball, hipStream_t st) {
   if (f.n <= 0) return hipSuccess;
-  if (w.metric != kMetricRMSD || (thr && !eps2)) return hipErrorInvalidValue;
+  if (w.metric != kMetricRMSD || !thr || !eps2) return hipErrorInvalidValue;
   hipLaunchKernelGGL(ball_kernel, dim3((unsigned)((f.n + 2 * kTile - 1) / (2 * kTile))), dim3(256), 0,
                      st, f.xyz, f.cen, f.G, w.w, f.natoms, f.n, order, mid, thr, eps2, ball);
   return hipGetLastError();
