@@ -39,7 +39,6 @@
 // against 50000 x 304 atoms in plain FP32, k = 100: 124 ms before, now 5 for
 // the landmarks, 15 for the filter and 26 for the tiles left.
 #include <hip/hip_runtime.h>
-#include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cfloat>
@@ -1036,6 +1035,118 @@ __global__ __launch_bounds__(256) void rank_sort_kernel(const unsigned* __restri
   if (wave == 0 && q < n) order[part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane]] = q;
 }
 
+// One pass of the stable sort by digits of 8 bits, in two kernels of at most
+// kSortBlocks workgroups of 4 waves.  A wave takes 64 rows a round, `rounds`
+// rounds side by side, so rows keep their order within a digit: workgroups,
+// waves, rounds, lanes.  Bound by its eight launches and each pass's chain of
+// loads: 5000 rows 26 us, 40007 35, 200000 72, 1000000 123.  (hipCUB's sort took
+// 24, 38, 60 and 164, and its 468 kernels 4 ms to load on a process's first use.)
+constexpr int kSortBlocks = 256;
+
+// counts[workgroup][digit] of the rows of each workgroup.
+__global__ __launch_bounds__(256) void sort_count_kernel(const unsigned* __restrict__ keys, int n,
+                                                         int rounds, int shift,
+                                                         int* __restrict__ counts) {
+  __shared__ int bin[256];
+  const int tid = threadIdx.x;
+  bin[tid] = 0;
+  __syncthreads();
+  const int64_t i0 = (int64_t)blockIdx.x * rounds * 256 + tid;
+  for (int r = 0; r < rounds; r += 4) {
+    unsigned k[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t i = i0 + (r + j) * 256;
+      k[j] = i < n ? keys[i] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i0 + (r + j) * 256 < n) atomicAdd(&bin[k[j] >> shift & 255u], 1);
+  }
+  __syncthreads();
+  counts[blockIdx.x * 256 + tid] = bin[tid];
+}
+
+// Rows to their places by that digit.  A digit's rows start after all rows of
+// smaller digits and those of the workgroups and waves before; within a wave's
+// round a lane's place is the number of lower lanes with its digit.
+__global__ __launch_bounds__(256) void sort_scatter_kernel(
+    const unsigned* __restrict__ keys, const int* __restrict__ rows, int n, int rounds, int shift,
+    const int* __restrict__ counts, unsigned* __restrict__ keys_out, int* __restrict__ rows_out) {
+  __shared__ int at[4][256];
+  __shared__ int wave_sum[4];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  for (int w = 0; w < 4; ++w) at[w][tid] = 0;
+  __syncthreads();
+  const int64_t i0 = ((int64_t)blockIdx.x * 4 + wave) * rounds * 64 + lane;
+  unsigned k[4];
+  auto load = [&](int r) {  // the keys of four rounds
+#pragma unroll
+    for (int j = 0; j < 4; ++j) k[j] = i0 + (r + j) * 64 < n ? keys[i0 + (r + j) * 64] : 0u;
+  };
+  for (int r = 0; r < rounds; r += 4) {
+    load(r);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i0 + (r + j) * 64 < n) atomicAdd(&at[wave][k[j] >> shift & 255u], 1);
+  }
+  // thread = digit: its rows in all workgroups, and in those before this one
+  // (sixteen loads in flight: one by one, 200000 rows took 208 us)
+  int total = 0, before = 0;
+  for (int b0 = 0; b0 < (int)gridDim.x; b0 += 16) {
+    int c[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      c[j] = b0 + j < (int)gridDim.x ? counts[(b0 + j) * 256 + tid] : 0;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      total += c[j];
+      before += b0 + j < (int)blockIdx.x ? c[j] : 0;
+    }
+  }
+  int upto = total;  // inclusive sum over the digits
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(upto, o);
+    upto += lane >= o ? v : 0;
+  }
+  if (lane == 63) wave_sum[wave] = upto;
+  __syncthreads();
+  int start = before + upto - total;
+  for (int w = 0; w < wave; ++w) start += wave_sum[w];
+  for (int w = 0; w < 4; ++w) {
+    const int c = at[w][tid];
+    at[w][tid] = start;
+    start += c;
+  }
+  __syncthreads();
+  for (int r = 0; r < rounds; r += 4) {
+    if (rounds > 4) load(r);  // else they are the ones counted
+    int row[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) row[j] = i0 + (r + j) * 64 < n ? rows[i0 + (r + j) * 64] : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bool on = i0 + (r + j) * 64 < n;
+      const unsigned digit = k[j] >> shift & 255u;
+      uint64_t same = __ballot(on);
+#pragma unroll
+      for (int bit = 0; bit < 8; ++bit) {
+        const uint64_t set = __ballot(digit >> bit & 1u);
+        same &= digit >> bit & 1u ? set : ~set;
+      }
+      const int rank = __popcll(same & ((1ull << lane) - 1ull));
+      // the first lane of a digit takes the places of all its lanes
+      int base = 0;
+      if (on && rank == 0) base = atomicAdd(&at[wave][digit], __popcll(same));
+      base = __shfl(base, on ? __builtin_ctzll(same) : lane);
+      if (on) {
+        keys_out[base + rank] = k[j];
+        rows_out[base + rank] = row[j];
+      }
+    }
+  }
+}
+
 __global__ void rank_keys_kernel(const int* __restrict__ rank, int ncells, int64_t n,
                                  unsigned* __restrict__ keys) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1211,10 +1322,7 @@ hipError_t launch_rank_sort(const unsigned* keys, int* order, int64_t n, hipStre
 }
 
 size_t sort_order_scratch(int64_t n) {
-  size_t temp = 0;
-  (void)hipcub::DeviceRadixSort::SortPairs<unsigned, int>(nullptr, temp, nullptr, nullptr, nullptr,
-                                                          nullptr, (int)n);
-  return temp;
+  return (size_t)n * (sizeof(unsigned) + sizeof(int)) + kSortBlocks * 256 * sizeof(int);
 }
 
 hipError_t launch_sort_order(const int* leaders, int* rank, int ncells, unsigned* keys,
@@ -1227,8 +1335,23 @@ hipError_t launch_sort_order(const int* leaders, int* rank, int ncells, unsigned
     hipLaunchKernelGGL(rank_keys_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, rank,
                        ncells, n, keys);
   }
-  return hipcub::DeviceRadixSort::SortPairs(temp, temp_bytes, keys, keys_out, rows, order, (int)n, 0,
-                                            32, st);
+  if (n < 1 || n > INT_MAX || temp_bytes < sort_order_scratch(n)) return hipErrorInvalidValue;
+  // four rounds, or a multiple that makes no more than kSortBlocks workgroups:
+  // each reads the counts of all
+  const int rounds = 4 * (int)((n + 1024 * kSortBlocks - 1) / (1024 * kSortBlocks));
+  const dim3 grid((unsigned)((n + 256 * rounds - 1) / (256 * rounds)));
+  unsigned* const tkeys = (unsigned*)temp;
+  int* const trows = (int*)(tkeys + n);
+  int* const counts = trows + n;
+  for (int pass = 0; pass < 4; ++pass) {
+    const unsigned* const kin = pass == 0 ? keys : pass & 1 ? tkeys : keys_out;
+    const int* const rin = pass == 0 ? rows : pass & 1 ? trows : order;
+    hipLaunchKernelGGL(sort_count_kernel, grid, dim3(256), 0, st, kin, (int)n, rounds, 8 * pass,
+                       counts);
+    hipLaunchKernelGGL(sort_scatter_kernel, grid, dim3(256), 0, st, kin, rin, (int)n, rounds,
+                       8 * pass, counts, pass & 1 ? keys_out : tkeys, pass & 1 ? order : trows);
+  }
+  return hipGetLastError();
 }
 
 }  // namespace mdsctk

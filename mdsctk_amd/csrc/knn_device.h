@@ -276,11 +276,13 @@ hipError_t launch_near_keys(const unsigned long long* near, int64_t n, int phase
 // kRankSortMax rows and allocates and clears nothing (it may be captured).
 constexpr int64_t kRankSortMax = 16384;
 hipError_t launch_rank_sort(const unsigned* keys, int* order, int64_t n, hipStream_t st);
-// order = rows sorted by key (stable), the cells of the keys first put in the
-// order of their leaders (rank: ncells ints of scratch).
+// order = rows (0, 1, ... n - 1) sorted by key (stable), the cells of the keys
+// first put in the order of their leaders if given (rank: ncells ints of
+// scratch).  keys_out: n more of scratch.
 size_t sort_order_scratch(int64_t n);
-hipError_t launch_sort_order(const int* leaders, int* rank, int ncells, unsigned* keys, unsigned* keys_out, const int* rows, int* order,
-                             int64_t n, void* temp, size_t temp_bytes, hipStream_t st);
+hipError_t launch_sort_order(const int* leaders, int* rank, int ncells, unsigned* keys,
+                             unsigned* keys_out, const int* rows, int* order, int64_t n, void* temp,
+                             size_t temp_bytes, hipStream_t st);
 
 // The prep pass: the FP64 centroids, G and G~ (one wave per frame), then,
 // if f.op is set, the operand (one workgroup per tile and 4 K-groups).

@@ -309,8 +309,9 @@ class HipServeDevice {
       return rc;
     if ((rc = ensure_host(sl, elems, (size_t)limit))) return rc;
     // The ordered form's workspace comes with the slot's first batch that
-    // takes it, at its largest.  Beyond the rank sort the ordering takes a
-    // library sort, which is not for a captured graph.
+    // takes it, at its largest.  Batches beyond the rank sort's rows (2048 is
+    // the default limit) take every tile: each slot would hold as much for
+    // them.
     s.cross_most = kRankSortMax;
     s.cross_room = std::min<int64_t>(limit, kRankSortMax);
     sl.sized_limit = limit;
