@@ -1979,7 +1979,9 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(T == 256 ? 5 
   // entries (coalesced).  Many lists (a small query batch spread over many
   // reference phases): a thread per list, streaming its entries with four
   // loads in flight -- a wave per list would wait on one list's count and
-  // entries at a time, hundreds of times per pass.
+  // entries at a time, hundreds of times per pass.  With 128 lists a row, 2000
+  // against 20000 x 304, k 20: 83 us so, 188 with waves over the lists; 252
+  // lists, 1000 against 8000 x 100: 50, 219.
   const bool list_per_thread = P.nl >= 64;
   auto visit = [&](auto&& f) {
     if (list_per_thread) {
