@@ -791,19 +791,29 @@ size_t carve_cross(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit, Carve&
 }
 
 // Whether a query is long enough for the ordered form: its launches and the
-// passes over the query frames against the pairs that it saves.  Measured,
-// whole query unordered -> ordered, k 10, one basin | 50 states:
-//   600 x 50000 x 304    bf16  .96 -> 1.13 ms | 1.04 -> 1.39
-//   1200 x 32000 x 304        1.22 -> 1.13    | 1.34 -> 1.33
-//   2500 x 15000 x 304        1.27 -> 1.16    | 1.44 -> 1.29
-//   1200 x 15000 x 1000       1.86 -> 1.61    | 2.02 -> 2.00
-//   2500 x 10000 x 2000       4.37 -> 4.15    | 4.56 -> 4.69
-//   1200 x 15000 x 304   fp32 1.71 -> 1.31    | 1.80 -> 1.90
-// A set of 8192 frames takes 1.2 to 3 times as long with 256 of them.
+// passes over the query frames against the pairs that it saves, which are
+// fewer for long lists (looser thresholds).  Measured, whole query unordered ->
+// ordered, one basin | 50 states, and pairs / line:
+//   2000 x 15000 x 304   bf16 k 4   .75 ->  .93 ms |  .81 -> 1.04     .86
+//   2000 x 30000 x 304        k 4  1.36 -> 1.24    | 1.44 -> 1.38    1.72
+//   1000 x 15000 x 1000       k 4  1.10 -> 1.43    | 1.18 -> 1.58     .60
+//   2000 x 15000 x 1000       k 4  1.80 -> 1.70    | 1.93 -> 1.92    1.19
+//   1000 x 30000 x 1000       k 40 1.78 -> 1.65    | 1.98 -> 2.81     .89
+//   2000 x 30000 x 1000       k 40 3.31 -> 2.63    | 3.57 -> 4.33    1.77
+//   2000 x 8192 x 2000        k 4  2.27 -> 2.65    | 2.38 -> 2.73     .71
+//   2000 x 15000 x 2000       k 4  3.57 -> 3.49    | 3.71 -> 3.58    1.30
+//   1000 x 15000 x 304   fp32 k 4   .99 -> 1.05    | 1.02 -> 1.24     .86
+//   2000 x 15000 x 304        k 4  1.64 -> 1.25    | 1.69 -> 1.52    1.72
+// Of 402 sizes between a quarter and six times the line, half of them of
+// either kind, 26 are slower ordered past it (1.06 to 1.32: states, most with
+// k above 40), 13 faster ordered below it (.66 to .9).
+double cross_line(const mdsctk_knn_ctx* c) {
+  return (2e7 + 4e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.5 : 1.0);
+}
+
 bool cross_pays(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
-  if (!q.fused || q.nofit || n_fit < kCrossMinFit) return false;
-  const double pairs = (1.2e7 + 2.4e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.7 : 1.0);
-  return (double)n_fit * (double)c->ref.n >= pairs;
+  return q.fused && !q.nofit && n_fit >= kCrossMinFit &&
+         (double)n_fit * (double)c->ref.n >= cross_line(c) * (1.0 + 0.01 * q.k1);
 }
 
 // Bytes of slot workspace the ordered form of a cross query of n_fit frames
@@ -1006,7 +1016,10 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
 // the other workspaces keep their room.
 int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, int64_t n_fit) {
   const int64_t n = c->ref.n;
-  if (!cross_pays(c, q, n_fit)) return 0;  // such queries never walk the copy
+  // Queries that are far from walking the copy do not count; lengths vary, so
+  // those not far below the line do.
+  if (!q.fused || q.nofit || n_fit < kCrossMinFit || (double)n_fit * (double)n < 0.6 * cross_line(c))
+    return 0;
   if (!c->ref_axes || n < kCrossMinRef || n * c->ref.natoms < kCrossMinWork || c->budget) return 0;
   std::lock_guard<std::mutex> g(c->plain_mu);
   OrderedRef& o = c->ordered;

@@ -46,7 +46,7 @@ def test_served_batches_of_growing_size_allocate_nothing(frames):
         want = ctx.query(fit, K)
         for _ in range(4):
             ctx.query(fit, K)
-        ctx.wait(ctx.submit(fit[:900], K))
+        ctx.wait(ctx.submit(fit[:1700], K))
         before = _held(ctx)
         for m in (900, 300, 1100, 2048, 1999):
             r = ctx.wait(ctx.submit(fit[:m], K))
@@ -94,11 +94,13 @@ def test_budget_set_while_serving_gives_the_copy_back(frames, busy):
 @pytest.mark.parametrize("prec", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("gen,n_ref,natoms,n_fit,k", [
     ("states", 16385, 260, 2500, 1), ("states", 16385, 260, 2300, 70), ("basin", 15000, 290, 2100, 12),
-    ("loose", 10007, 420, 4097, 5), ("copies", 12000, 350, 3000, 30), ("states", 9000, 470, 17000, 9)])
+    ("loose", 10007, 420, 4097, 5), ("copies", 12000, 350, 3000, 30), ("states", 9000, 470, 17000, 9),
+    ("states", 16385, 260, 4100, 70), ("basin", 15000, 290, 2700, 12), ("copies", 12000, 350, 3700, 30)])
 def test_ordered_rows_equal_the_unordered_ones(gen, n_ref, natoms, n_fit, k, prec):
     """Blocks around one place and around many, unrelated frames (more places
     than a block's pass takes), a resident set of 40 frames' copies (equal
-    keys), more query frames than the rank sort takes."""
+    keys), more query frames than the rank sort takes; on both sides of the
+    length from which queries are ordered."""
     rng = np.random.default_rng(n_ref)
     n = n_ref + n_fit
     if gen == "states":
