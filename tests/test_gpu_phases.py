@@ -38,3 +38,15 @@ def test_self_rows_with_a_band_pass_over_several_lists(n, k, flags):
     d_e, i_e = _rows("exact", frames, None, [(frames[::7], k, flags)])[0]
     np.testing.assert_array_equal(i[::7], i_e)
     np.testing.assert_array_equal(d[::7], d_e)
+
+
+@pytest.mark.parametrize("n_ref,natoms", [(16400, 256), (16400, 257), (32768, 300), (32767, 300)])
+def test_short_fp32_rows_equal_the_exact_form(n_ref, natoms):
+    """With a sample pass and without, by frame length, rows and references."""
+    x = synth.metastable_trajectory(n_ref + 255, natoms, 5, n_centres=9)
+    ref, fit = x[:n_ref], x[n_ref:]
+    w = synth.masses(natoms, "random", 1)
+    queries = [(fit[:m], k, 0) for m in (1, 31, 32, 255) for k in (1, 40)]
+    for (d, i), (d_e, i_e) in zip(_rows("fp32", ref, w, queries), _rows("exact", ref, w, queries)):
+        np.testing.assert_array_equal(i, i_e)
+        np.testing.assert_array_equal(d, d_e)
