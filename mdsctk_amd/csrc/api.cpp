@@ -740,14 +740,14 @@ int enqueue_ball_test(mdsctk_knn_ctx* c, const MiddleSet& ref, const DevFrames& 
 //   2000 x 3500 x 2000, k 4  .68 -> .79 (the one kind that loses)
 //   2000 x 20000 x 2000, k 30 2.37 -> 2.10
 // --nofit in FP32 goes as the fitted form: 2000 x 20000 x 700, k 2 1.83 -> 2.01.
-// Short queries in FP32, whose contraction is the larger part, gain with short
+// Short fitted queries in FP32, whose contraction is the larger part, gain with short
 // frames, or with enough rows and either references or shorter lists:
 //   1 x 40000 x 500, k 4     .59 -> .72, x 1200 1.15 -> 1.46, x 100 .29 -> .31
 //   64 x 40000 x 500, k 15   .80 -> .73, x 1200 1.41 -> 1.52, x 100 .51 -> .32
 //   64 x 17000 x 500, k 15   .40 -> .46, k 1 .52 -> .45
 bool sampled_query(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
   if (n_fit < kCrossMinFit && c->ref.n >= kSampleMinRef)
-    return c->prec != kFP32 || c->ref.natoms <= 256 ||
+    return c->prec != kFP32 || q.nofit || c->ref.natoms <= 256 ||
            (c->ref.natoms <= 640 && n_fit >= 32 &&
             (c->ref.n >= 2 * kSampleMinRef || q.k1 <= 8));
   return c->ref.n >= 3000 && n_fit * c->ref.n >= 6000000 &&
