@@ -799,29 +799,29 @@ size_t carve_cross(mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit, Carve&
 }
 
 // Whether a query is long enough for the ordered form: its launches and the
-// passes over the query frames against the pairs that it saves, which are
-// fewer for long lists (looser thresholds).  Measured, whole query unordered ->
-// ordered, one basin | 50 states, and pairs / line:
-//   2000 x 15000 x 304   bf16 k 4   .75 ->  .93 ms |  .81 -> 1.04     .86
-//   2000 x 30000 x 304        k 4  1.36 -> 1.24    | 1.44 -> 1.38    1.72
-//   1000 x 15000 x 1000       k 4  1.10 -> 1.43    | 1.18 -> 1.58     .60
-//   2000 x 15000 x 1000       k 4  1.80 -> 1.70    | 1.93 -> 1.92    1.19
-//   1000 x 30000 x 1000       k 40 1.78 -> 1.65    | 1.98 -> 2.81     .89
-//   2000 x 30000 x 1000       k 40 3.31 -> 2.63    | 3.57 -> 4.33    1.77
-//   2000 x 8192 x 2000        k 4  2.27 -> 2.65    | 2.38 -> 2.73     .71
-//   2000 x 15000 x 2000       k 4  3.57 -> 3.49    | 3.71 -> 3.58    1.30
-//   1000 x 15000 x 304   fp32 k 4   .99 -> 1.05    | 1.02 -> 1.24     .86
-//   2000 x 15000 x 304        k 4  1.64 -> 1.25    | 1.69 -> 1.52    1.72
+// passes over the query frames against the pairs that it saves.  Measured,
+// whole query unordered -> ordered, one basin | 50 states, and pairs / line:
+//   2000 x 15000 x 304  bf16 k 4  0.75 -> 0.90 ms | 0.81 -> 1.01   0.89
+//   2000 x 30000 x 304       k 4  1.36 -> 1.20    | 1.44 -> 1.35   1.78
+//   1000 x 15000 x 1000      k 4  1.10 -> 1.40    | 1.18 -> 1.55   0.75
+//   2000 x 15000 x 1000      k 4  1.80 -> 1.64    | 1.93 -> 1.84   1.50
+//   1000 x 30000 x 1000      k 40 1.78 -> 1.61    | 1.98 -> 2.70   1.50
+//   2000 x 30000 x 1000      k 40 3.31 -> 2.61    | 3.57 -> 4.16   3.00
+//   2000 x 8192 x 2000       k 4  2.27 -> 2.56    | 2.38 -> 2.69   0.96
+//   2000 x 15000 x 2000      k 4  3.57 -> 3.40    | 3.71 -> 3.49   1.76
+//   1000 x 15000 x 304  fp32 k 4  0.99 -> 1.06    | 1.02 -> 1.25   0.89
+//   2000 x 15000 x 304       k 4  1.64 -> 1.22    | 1.69 -> 1.49   1.78
 // Of 402 sizes between a quarter and six times the line, half of them of
-// either kind, 26 are slower ordered past it (1.06 to 1.32: states, most with
-// k above 40), 13 faster ordered below it (.66 to .9).
+// either kind, 31 are slower ordered past it (1.05 to 1.5: states, most with k
+// above 40), 3 faster ordered below it (.8 to .9).  Served batches, which have
+// half the CUs, lie the same way.
 double cross_line(const mdsctk_knn_ctx* c) {
-  return (2e7 + 4e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.5 : 1.0);
+  return (1.4e7 + 6e9 / c->ref.natoms) * (c->prec == kFP32 ? 0.5 : 1.0);
 }
 
 bool cross_pays(const mdsctk_knn_ctx* c, const QueryShape& q, int64_t n_fit) {
   return q.fused && !q.nofit && n_fit >= kCrossMinFit &&
-         (double)n_fit * (double)c->ref.n >= cross_line(c) * (1.0 + 0.01 * q.k1);
+         (double)n_fit * (double)c->ref.n >= cross_line(c);
 }
 
 // Bytes of slot workspace the ordered form of a cross query of n_fit frames
@@ -973,13 +973,17 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   Lists LL = p.L;
   LL.nl = 4 * lm_phases;
   LL.thr = x.thr0;
+  // What a row's key has left for the distance beside a place.  (A few frames of
+  // one basin are the nearest landmark of most rows: without the distance 50000
+  // against 50000 x 304 in FP32, k 100, took 55.9 ms instead of 52.8.)
+  const int dist_bits = std::min(kFilterDistBits, __builtin_clz((unsigned)c->ref.n));
   HIP_TRY(c, launch_stride_list(c->ref.n_tiles, x.lstride, lm, s.st));
   HIP_TRY(c, launch_init_lists(LL, n, s.st));
   HIP_TRY(c, launch_eps(fit, R, p.kappa, x.eps0, s.sum, s.st));
   HIP_TRY(c, launch_contract(c->ref, fit, LL, x.eps0, q.k1, lm_phases, false, nullptr, p.grid, s.st,
                              nullptr, 0, &lm));
   HIP_TRY(c, launch_landmark_cap(LL, n, q.k1, x.eps0, x.lstride, x.thr0, x.label, s.st, 1, x.keys,
-                                 x.rows, nullptr, 0, o.place));
+                                 x.rows, nullptr, 0, o.place, dist_bits));
   if (x.sort_temp)
     HIP_TRY(c, launch_sort_order(nullptr, nullptr, 0, x.keys, x.keys_out, x.rows, x.order, n,
                                  x.sort_temp, x.sort_bytes, s.st));
@@ -998,8 +1002,8 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   Lists LB = p.L;
   LB.nl = 4 * std::max(1, std::min({p.phases, most, 2 * p.grid / blocks}));
   HIP_TRY(c, launch_init_lists(LB, n, s.st, false));
-  HIP_TRY(c, launch_place_band_list(x.keys, x.order, n, c->ref.n_tiles, x.fit.n_tiles, width,
-                                    most, x.tiles, s.st));
+  HIP_TRY(c, launch_place_band_list(x.keys, dist_bits, x.order, n, c->ref.n_tiles, x.fit.n_tiles,
+                                    width, most, x.tiles, s.st));
   HIP_TRY(c, launch_contract(R, x.fit, LB, p.eps2, q.k1, LB.nl / 4, false, nullptr, p.grid, s.st,
                              nullptr, 0, &x.tiles));
   HIP_TRY(c, launch_landmark_cap(LB, n, q.k1, p.eps2, 1, p.L.thr, nullptr, s.st));
@@ -1026,7 +1030,7 @@ int ensure_ordered(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, int64_t n_fi
   const int64_t n = c->ref.n;
   // Queries that are far from walking the copy do not count; lengths vary, so
   // those not far below the line do.
-  if (!q.fused || q.nofit || n_fit < kCrossMinFit || (double)n_fit * (double)n < 0.6 * cross_line(c))
+  if (!q.fused || q.nofit || n_fit < kCrossMinFit || (double)n_fit * (double)n < 0.65 * cross_line(c))
     return 0;
   if (!c->ref_axes || n < kCrossMinRef || n * c->ref.natoms < kCrossMinWork || c->budget) return 0;
   std::lock_guard<std::mutex> g(c->plain_mu);

@@ -918,16 +918,14 @@ __global__ void band_list_kernel(int ref_pairs, int fit_blocks, int block_pairs,
 // `width` reference pairs around each row's place.  One row without a
 // candidate nearby keeps every tile of its block, so all rows count unless
 // that makes more than `most` pairs; then every second, fourth ... row.
-__global__ __launch_bounds__(128) void place_band_list_kernel(const unsigned* __restrict__ keys,
-                                                              const int* __restrict__ order,
-                                                              int64_t n, int ref_pairs, int width,
-                                                              int most, int* __restrict__ list,
-                                                              int* __restrict__ count) {
+__global__ __launch_bounds__(128) void place_band_list_kernel(
+    const unsigned* __restrict__ keys, int dist_bits, const int* __restrict__ order, int64_t n,
+    int ref_pairs, int width, int most, int* __restrict__ list, int* __restrict__ count) {
   constexpr int kRows = kFilterFitTiles * kTile;
   __shared__ int at[kRows];
   const int fb = blockIdx.x;
   const int64_t row = min((int64_t)fb * kRows + threadIdx.x, n - 1);
-  at[threadIdx.x] = (int)(keys[order[row]] / (2u * kTile));
+  at[threadIdx.x] = (int)((keys[order[row]] >> dist_bits) / (2u * kTile));
   __syncthreads();
   if (threadIdx.x) return;
   int* const out = list + (int64_t)fb * ref_pairs;
@@ -1287,12 +1285,13 @@ hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, con
   return hipGetLastError();
 }
 
-hipError_t launch_place_band_list(const unsigned* keys, const int* order, int64_t n, int ref_tiles,
-                                  int fit_tiles, int width, int most, const TileList& tl,
-                                  hipStream_t st) {
+hipError_t launch_place_band_list(const unsigned* keys, int dist_bits, const int* order, int64_t n,
+                                  int ref_tiles, int fit_tiles, int width, int most,
+                                  const TileList& tl, hipStream_t st) {
   if (n < 1 || width < 1 || fit_tiles % kFilterFitTiles) return hipErrorInvalidValue;
   hipLaunchKernelGGL(place_band_list_kernel, dim3((unsigned)(fit_tiles / kFilterFitTiles)), dim3(128),
-                     0, st, keys, order, n, ref_tiles / kRefTilesPerWG, width, most, tl.list, tl.count);
+                     0, st, keys, dist_bits, order, n, ref_tiles / kRefTilesPerWG, width, most,
+                     tl.list, tl.count);
   return hipGetLastError();
 }
 

@@ -258,11 +258,12 @@ hipError_t launch_filter(const FilterSet& ref, const FilterSet& fit, int64_t n_r
 hipError_t launch_band_list(int ref_tiles, int fit_tiles, int ft, int width, const TileList& tl,
                             hipStream_t st);
 // The fit blocks of a cross query in the order of their keys (places in the
-// ordered set): `width` reference pairs around each row's place, or around
-// every second, fourth ... row's where that makes more than `most` pairs.
-hipError_t launch_place_band_list(const unsigned* keys, const int* order, int64_t n, int ref_tiles,
-                                  int fit_tiles, int width, int most, const TileList& tl,
-                                  hipStream_t st);
+// ordered set, above dist_bits of the distance): `width` reference pairs around
+// each row's place, or around every second, fourth ... row's where that makes
+// more than `most` pairs.
+hipError_t launch_place_band_list(const unsigned* keys, int dist_bits, const int* order, int64_t n,
+                                  int ref_tiles, int fit_tiles, int width, int most,
+                                  const TileList& tl, hipStream_t st);
 // Every stride-th reference pair, as a list shared by every block.
 hipError_t launch_stride_list(int ref_tiles, int stride, const TileList& tl, hipStream_t st);
 // place[order[i]] = i.
@@ -335,14 +336,15 @@ hipError_t launch_eps_sym(const DevFrames& fit, const DevFrames& ref, double kap
 // keys (if given): keys[q] orders rows by their nearest landmark among every
 // cell-th one, then by the distance to it, and rows[q] = q; leaders[cell] =
 // the first cell whose landmark is among the leader_rank + 1 nearest of this
-// cell's landmark.  place: keys[q] is its nearest landmark's place there.
+// cell's landmark.  place: keys[q] is its nearest landmark's place there, above
+// dist_bits of the distance.
 // label null: the lists are of a band or sample pass, and thr[q] is only
 // lowered.
 hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* eps2,
                                int phases, unsigned* thr, int* label, hipStream_t st,
                                int cell = 1, unsigned* keys = nullptr, int* rows = nullptr,
                                int* leaders = nullptr, int leader_rank = 0,
-                               const int* place = nullptr);
+                               const int* place = nullptr, int dist_bits = kFilterDistBits);
 // order[0..n) = rows grouped by label (counting sort; counts holds nlab ints).
 hipError_t launch_row_order(const int* label, int64_t n, int nlab, int* counts, int* order,
                             hipStream_t st);

@@ -2191,7 +2191,8 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
                                                            int* __restrict__ rows,
                                                            int* __restrict__ leaders,
                                                            int leader_rank,
-                                                           const int* __restrict__ place) {
+                                                           const int* __restrict__ place,
+                                                           int dist_bits) {
   const int64_t q = blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   __shared__ unsigned hist[256];
@@ -2249,14 +2250,13 @@ __global__ __launch_bounds__(256) void landmark_cap_kernel(const uint2* __restri
   if (tid == 0 && label) {
     label[q] = s_best != ~0ull ? (int)dense((unsigned)(s_best & 0xffffffffu)) : 0;
     if (keys) {
-      // cell number, then the distance's leading 19 bits (its exponent and
-      // 11 of the fraction): enough to lay like distances side by side
+      // cell number or place, then the distance's leading bits (19: its exponent
+      // and 11 of the fraction): enough to lay like distances side by side
       const unsigned long long b = s_cell != ~0ull ? s_cell : s_best;
       const unsigned r = (unsigned)(b & 0xffffffffu);
-      const unsigned lab = b != ~0ull ? dense(r) / (unsigned)cell : 0u;
-      keys[q] = place ? (b != ~0ull ? (unsigned)place[r] : 0u)
-                      : (lab << kFilterDistBits) |
-                            ((unsigned)(b >> 32) >> (31 - kFilterDistBits) & ((1u << kFilterDistBits) - 1u));
+      const unsigned lab = b == ~0ull ? 0u : place ? (unsigned)place[r] : dense(r) / (unsigned)cell;
+      keys[q] = (lab << dist_bits) |
+                ((unsigned)(b >> 32) >> (31 - dist_bits) & ((1u << dist_bits) - 1u));
       rows[q] = (int)q;
     }
   }
@@ -3211,9 +3211,10 @@ hipError_t launch_permute_thresholds(const unsigned* src, const int* perm, const
 hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* eps2,
                                int phases, unsigned* thr, int* label, hipStream_t st, int cell,
                                unsigned* keys, int* rows, int* leaders, int leader_rank,
-                               const int* place) {
+                               const int* place, int dist_bits) {
   if (n <= 0) return hipSuccess;
-  if (k1 < 1 || phases < 1 || !thr || cell < 1 || (keys && (!label || !rows)))
+  if (k1 < 1 || phases < 1 || !thr || cell < 1 || (keys && (!label || !rows)) || dist_bits < 1 ||
+      dist_bits > 30)
     return hipErrorInvalidValue;
   if (leaders) {  // a cell whose landmark is padding leads itself
     const int ncells = (int)((2 * kTile * ((n + 2 * kTile * phases - 1) / (2 * kTile * phases)) + cell - 1) / cell);
@@ -3221,7 +3222,8 @@ hipError_t launch_landmark_cap(const Lists& L, int64_t n, int k1, const float* e
                        ncells);
   }
   hipLaunchKernelGGL(landmark_cap_kernel, dim3((unsigned)n), dim3(256), 0, st, L.ent, L.cnt, L.nl,
-                     L.cap, k1, eps2, phases, thr, label, cell, keys, rows, leaders, leader_rank, place);
+                     L.cap, k1, eps2, phases, thr, label, cell, keys, rows, leaders, leader_rank, place,
+                     dist_bits);
   return hipGetLastError();
 }
 
