@@ -998,7 +998,13 @@ int enqueue_cross(mdsctk_knn_ctx* c, Slot& s, const QueryShape& q, const FusedPl
   // a pass over the reference pairs around each block's places tightens them
   const int ref_pairs = c->ref.n_tiles / kRefTilesPerWG;
   const int width = std::min(ref_pairs, std::max(3, q.k1 / 32 + 1));
-  const int most = std::max(8 * width, ref_pairs / 32);
+  // In FP32, where the pass costs most, half as many pairs do for a block whose
+  // share of the places is narrower than that (50000 against 50000 x 304, k 100:
+  // 53.0 -> 52.0 ms; 12 sizes within 2 %).  Wider blocks lose by it (2627 x
+  // 18493 x 398, 50 states, k 81: 3.7 -> 5.2 ms).
+  const int share = ref_pairs / (x.fit.n_tiles / kFilterFitTiles);
+  const int half = c->prec == kFP32 && share < width ? 2 : 1;
+  const int most = std::max(8 * width, ref_pairs / 32) / half;
   Lists LB = p.L;
   LB.nl = 4 * std::max(1, std::min({p.phases, most, 2 * p.grid / blocks}));
   HIP_TRY(c, launch_init_lists(LB, n, s.st, false));
