@@ -36,8 +36,8 @@
 // segment the filter alone took over 220 ms.  Cross query of 4096
 // against 100000 x 500 atoms, k = 50 (one basin): contraction 10.0 ms before;
 // the filter takes 4.0 ms (1.1 PFLOP/s) and leaves tiles for 2.1 ms.  50000
-// against 50000 x 304 atoms in plain FP32, k = 100: 124 ms before, now 5 for
-// the landmarks, 15 for the filter and 26 for the tiles left.
+// against 50000 x 304 atoms in plain FP32, k = 100: 124 ms before, now 6 for
+// the landmarks and places, 14 for the filter and 25 for the tiles left.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
